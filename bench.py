@@ -72,6 +72,9 @@ def kernel_work(arch, h, w, hp=None, wp=None):
         "qkv_window_attention": ("mfma", 2 * P * 3 * C * C + 4 * P * win * win * C,
                                  f * (P * 2 * C + 3 * C * C)),
         "window_attention": ("mfma", 4 * P * win * win * C, f * P * (3 * C + C)),
+        # proj + LayerNorm + residual, fc1 + GELU, fc2 + LayerNorm + residual as
+        # one kernel (the attention output and the block input in, the block out)
+        "token_mlp": ("mfma", 2 * P * (C * C + 2 * Hd * C), f * P * 3 * C),
         "proj_ln_res": ("mfma", 2 * P * C * C, f * P * 3 * C),
         "fc1_gelu": ("mfma", 2 * P * Hd * C, f * P * (C + Hd)),
         "fc2_ln_res": ("mfma", 2 * P * C * Hd, f * P * (Hd + 2 * C)),

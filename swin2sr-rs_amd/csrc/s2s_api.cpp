@@ -62,6 +62,10 @@ struct BlockW {
     float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr;
     float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
     float *ls = nullptr, *cpbt = nullptr;
+    // the token half as k_token_mlp reads it (token_mlp_pack), for the widths
+    // it takes; wproj .. b2 above are then not uploaded
+    float *tok_w = nullptr, *tok_prm = nullptr;
+    float ln1_bound = 0.f, fc1_l1 = 0.f, fc1_bmax = 0.f;
 };
 
 struct StageW {
@@ -790,6 +794,24 @@ int s2s_ctx::block_fwd(const BlockW &b, int hp, int wp, int shift, const float *
             return -1;
     }
 
+    if (b.tok_w) {
+        TokMlpArgs t{};
+        t.o = o;
+        t.x = x_in;
+        t.out = x_out;
+        t.w = b.tok_w;
+        t.prm = b.tok_prm;
+        t.ln1_bound = b.ln1_bound;
+        t.fc1_l1 = b.fc1_l1;
+        t.fc1_bmax = b.fc1_bmax;
+        t.inv_c = 1.0f / (float)c;
+        t.M = P;
+        t.C = c;
+        t.chunks = arch.mlp_ratio;
+        return run("token_mlp", dim3(token_mlp_grid(P, c)), dim3(256),
+                   [&] { return launch_token_mlp(t, stream); });
+    }
+
     g = rows_gemm(o, c, b.wproj, c, b.bproj, x_out, c, P, c, c);
     g.b_packed = bs_packs(c, c, EPI_LN_RES);
     g.res = x_in;
@@ -1418,13 +1440,18 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
         const uint64_t wqkv = qkv_attn_fused(A.heads, A.embed / A.heads)
                                   ? (uint64_t)(A.heads / 2) * weight_floats(C, C, EPI_STORE)
                                   : weight_floats(3 * C, C, EPI_STORE);
-        const uint64_t per_block = wqkv + 3 * C                               // fused qkv, its bias
-                                   + NH                                       // logit scale
-                                   + weight_floats(C, C, EPI_LN_RES) + C      // proj
-                                   + 4 * C                                    // norm1, norm2
-                                   + weight_floats(H2, C, EPI_GELU) + H2      // fc1
-                                   + weight_floats(C, H2, EPI_LN_RES) + C     // fc2
-                                   + NH * n * n;                              // the CPB table
+        // the token half: k_token_mlp's stream and parameters, or proj, norm1,
+        // norm2, fc1 and fc2 one by one
+        const uint64_t tok = token_mlp_takes(A.embed, A.mlp_ratio)
+                                 ? token_mlp_weight_floats(A.embed, A.mlp_ratio) +
+                                       token_mlp_param_floats(A.embed, A.mlp_ratio)
+                                 : weight_floats(C, C, EPI_LN_RES) + C + 4 * C +
+                                       weight_floats(H2, C, EPI_GELU) + H2 +
+                                       weight_floats(C, H2, EPI_LN_RES) + C;
+        const uint64_t per_block = wqkv + 3 * C     // fused qkv, its bias
+                                   + NH             // logit scale
+                                   + tok
+                                   + NH * n * n;    // the CPB table
         f += per_block * (uint64_t)A.depths[s];
     }
     const int up = A.upsampler;
@@ -1670,20 +1697,40 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
             rc = rc || ts.get(p + "attn.logit_scale", {NH, 1, 1}, &lsx);
             if (rc) break;
             rc = ctx->upload(vec_of(lsx, NH), &bw.ls);
-            auto up_gemm = [&](const std::string &name, int N, int K, int epi, float **dst) -> int {
-                if (ts.get(name, {N, K}, &x)) return -1;
-                return ctx->upload(gemm_weights(vec_of(x, ts.numel(x)), 1, N, K, epi), dst);
-            };
-            rc = rc || up_gemm(p + "attn.proj.weight", C, C, EPI_LN_RES, &bw.wproj);
-            rc = rc || up(p + "attn.proj.bias", {C}, &bw.bproj);
-            rc = rc || up(p + "norm1.weight", {C}, &bw.n1w);
-            rc = rc || up(p + "norm1.bias", {C}, &bw.n1b);
-            rc = rc || up(p + "norm2.weight", {C}, &bw.n2w);
-            rc = rc || up(p + "norm2.bias", {C}, &bw.n2b);
-            rc = rc || up_gemm(p + "mlp.fc1.weight", H2, C, EPI_GELU, &bw.w1);
-            rc = rc || up(p + "mlp.fc1.bias", {H2}, &bw.b1);
-            rc = rc || up_gemm(p + "mlp.fc2.weight", C, H2, EPI_LN_RES, &bw.w2);
-            rc = rc || up(p + "mlp.fc2.bias", {C}, &bw.b2);
+            if (token_mlp_takes(C, A.mlp_ratio)) {
+                TokMlpWeights tw{};
+                const struct { const char *name; std::vector<int64_t> shape; const float **dst; } parts[] = {
+                    {"attn.proj.weight", {C, C}, &tw.wproj}, {"attn.proj.bias", {C}, &tw.bproj},
+                    {"norm1.weight", {C}, &tw.n1w},          {"norm1.bias", {C}, &tw.n1b},
+                    {"norm2.weight", {C}, &tw.n2w},          {"norm2.bias", {C}, &tw.n2b},
+                    {"mlp.fc1.weight", {H2, C}, &tw.w1},     {"mlp.fc1.bias", {H2}, &tw.b1},
+                    {"mlp.fc2.weight", {C, H2}, &tw.w2},     {"mlp.fc2.bias", {C}, &tw.b2}};
+                for (const auto &e : parts) {
+                    rc = rc || ts.get(p + e.name, e.shape, &x);
+                    if (!rc) *e.dst = x->data;
+                }
+                if (rc) break;
+                std::vector<float> w(token_mlp_weight_floats(C, A.mlp_ratio));
+                std::vector<float> prm(token_mlp_param_floats(C, A.mlp_ratio));
+                token_mlp_pack(tw, C, A.mlp_ratio, w.data(), prm.data(), &bw.ln1_bound, &bw.fc1_l1,
+                               &bw.fc1_bmax);
+                rc = ctx->upload(w, &bw.tok_w) || ctx->upload(prm, &bw.tok_prm);
+            } else {
+                auto up_gemm = [&](const std::string &name, int N, int K, int epi, float **dst) -> int {
+                    if (ts.get(name, {N, K}, &x)) return -1;
+                    return ctx->upload(gemm_weights(vec_of(x, ts.numel(x)), 1, N, K, epi), dst);
+                };
+                rc = rc || up_gemm(p + "attn.proj.weight", C, C, EPI_LN_RES, &bw.wproj);
+                rc = rc || up(p + "attn.proj.bias", {C}, &bw.bproj);
+                rc = rc || up(p + "norm1.weight", {C}, &bw.n1w);
+                rc = rc || up(p + "norm1.bias", {C}, &bw.n1b);
+                rc = rc || up(p + "norm2.weight", {C}, &bw.n2w);
+                rc = rc || up(p + "norm2.bias", {C}, &bw.n2b);
+                rc = rc || up_gemm(p + "mlp.fc1.weight", H2, C, EPI_GELU, &bw.w1);
+                rc = rc || up(p + "mlp.fc1.bias", {H2}, &bw.b1);
+                rc = rc || up_gemm(p + "mlp.fc2.weight", C, H2, EPI_LN_RES, &bw.w2);
+                rc = rc || up(p + "mlp.fc2.bias", {C}, &bw.b2);
+            }
             if (rc) break;
             // The bias table, stored [head][query][key] and scaled by log2(e)
             // for the base-2 softmax. From the converter's cpb_pre when the

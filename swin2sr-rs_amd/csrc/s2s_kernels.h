@@ -214,6 +214,36 @@ inline AttnArgs window_attn_args(const float *qkv, const float *cpbt, const floa
     return a;
 }
 
+// The token half of a Swin block as one kernel (k_token_mlp, s2s_split.hip):
+// out = x1 + LN2(GELU(x1 W1^T + b1) W2^T + b2), x1 = x + LN1(o Wproj^T + b),
+// over [M][C] rows (M a multiple of 16, out may be x), the hidden layer
+// `chunks` * C wide. w, prm and the three bounds come from token_mlp_pack.
+struct TokMlpArgs {
+    const float *o, *x;
+    float *out;
+    const float *w, *prm;
+    float ln1_bound, fc1_l1, fc1_bmax, inv_c;  // inv_c = 1 / C
+    int M, C, chunks;
+};
+struct TokMlpWeights {
+    const float *wproj, *bproj, *n1w, *n1b;  // [C][C], [C], LN1
+    const float *w1, *b1;                    // [ratio C][C], [ratio C]
+    const float *w2, *b2, *n2w, *n2b;        // [C][ratio C], [C], LN2
+};
+// widths k_token_mlp takes; its packed weights' and parameters' floats; the packing
+bool token_mlp_takes(int C, int ratio);
+size_t token_mlp_weight_floats(int C, int ratio);
+size_t token_mlp_param_floats(int C, int ratio);
+void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *prm, float *ln1_bound,
+                    float *fc1_l1, float *fc1_bmax);
+unsigned token_mlp_grid(int M, int C);
+hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st);
+// The power of two that brings the row's largest magnitude into [2^14, 2^15)
+// (1 for a zero row), and 16 weight rows' (null: zeros) k step k0 .. k0 + 31
+// (k < kn) scaled and split into f16 hi and lo fragments, 1 KiB each.
+float split_row_scale(const float *w, int n);
+void split_pack_step(const float *const *rows, const float *scale, int k0, int kn, uint16_t *dst);
+
 #define GEMM_NVARIANTS 6
 hipError_t launch_gemm(const GemmArgs &g, int aload, int epi, hipStream_t st);
 hipError_t launch_gemm_variant(const GemmArgs &g, int aload, int epi, int variant,

@@ -1,0 +1,662 @@
+// s2s_split.hip - fp32 contractions on the f16 matrix cores, by splitting.
+//
+// An fp32 operand x is scaled by a power of two and written as hi + lo, hi =
+// f16(x) and lo = f16(x - hi): 22 bits of it, and a product a b as the three
+// products hi hi + hi lo + lo hi, each exact in the MFMA's fp32 accumulation
+// (the lo lo term is 2^-22 of it and below). v_mfma_f32_16x16x32_f16 takes 32 k
+// where the fp32 v_mfma_f32_16x16x4f32 takes 4 in twice the time, so three of
+// them are 4.4 times the fp32 rate (measured 2,043 / 3 against 154.7 TFLOP/s
+// under pure MFMA load). The error is no larger than the fp32 MFMA's, whose
+// accumulator rounds once per 4 k: on K = 192 dot products of unit normals,
+// rms 1.63e-7 of the result's rms against 2.47e-7, at K = 384 2.24e-7 against
+// 3.56e-7.
+//
+// The scales keep f16's exponent range out of the way. A weight row is scaled
+// at upload so that its largest element lies in [2^14, 2^15); an activation row
+// by 2^(14 - floor(log2 B)), B its largest magnitude or a bound of it. A bound
+// that is loose by 2^10 costs nothing: an element 2^-10 of the row's bound
+// still has both parts normal, and what f16 drops is 2^-39 of B. The products
+// are scaled back in fp32, exactly (powers of two), before the bias.
+//
+// A operand tiles live in LDS in MFMA fragment order: per (row block of 16,
+// k step of 32, part) 1 KiB, lane l = 16 q + r holding row r, k = 8 q .. 8 q + 7,
+// so every operand read is one linear ds_read_b128. Weights are packed in the
+// same order per wave and stream from L2 through registers, each wave reading
+// only its own columns (33-39 TB/s measured with every CU reading the same
+// 737 KB).
+//
+// MFMA 16x16x32 f16 lane layout (checked on the device): lane l supplies
+// A[l%16][8(l/16) .. + 7] and B[l%16][the same k]; accumulator register i of
+// lane l holds D[4(l/16) + i][l%16], rows from A, columns from B. With A =
+// weights and B = tokens a lane holds one token and 4 consecutive columns.
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <type_traits>
+#include <vector>
+
+#include "s2s_device.h"
+#include "s2s_kernels.h"
+
+typedef _Float16 h8v __attribute__((ext_vector_type(8)));
+typedef _Float16 h4v __attribute__((ext_vector_type(4)));
+#define MFMA16H(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16((a), (b), (c), 0, 0, 0)
+
+namespace {
+
+// 2^(14 - floor(log2 b)) for a bound b >= 0 (the exponent clamped so that the
+// scale and its inverse are normal), and that inverse
+__device__ __forceinline__ int bound_exp(float b) {
+    return max((int)(__builtin_bit_cast(unsigned, b) >> 23), 15);
+}
+__device__ __forceinline__ float exp_scale(int e) { return __builtin_bit_cast(float, (268 - e) << 23); }
+__device__ __forceinline__ float exp_unscale(int e) { return __builtin_bit_cast(float, (e - 14) << 23); }
+
+// hi and lo of 4 values. The residuals pass through fp32 registers (the empty
+// asm): the compiler would fuse the subtraction and the conversion into
+// v_fma_mixlo_f16 / v_fma_mixhi_f16, which issue at a quarter of the rate
+// (measured 3.7 ns against 1.9 for v_fma_mix_f32 or the packed conversion and
+// 1.2 for v_fma_f32).
+__device__ __forceinline__ void split4(f4v v, h4v &hi, h4v &lo) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) hi[i] = (_Float16)v[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float r = fmaf((float)hi[i], -1.0f, v[i]);
+        asm("" : "+v"(r));
+        lo[i] = (_Float16)r;
+    }
+}
+
+#define DPP_MAX(v, ctrl)                                                                         \
+    fmaxf((v), __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, (v)), \
+                                                                  (ctrl), 0xF, 0xF, true)))
+__device__ __forceinline__ float row16_max(float v) {
+    v = DPP_MAX(v, 0xB1);
+    v = DPP_MAX(v, 0x4E);
+    v = DPP_MAX(v, 0x141);
+    v = DPP_MAX(v, 0x140);
+    return v;
+}
+// The maximum over lanes j, j+16, j+32, j+48, in every lane (xrow_sum2's swaps).
+__device__ __forceinline__ float xrow_max(float a) {
+    float b = a;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    float c = fmaxf(a, b);
+    float d = c;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+    return fmaxf(c, d);
+}
+
+constexpr int FRAG = 1024;  // bytes of one fragment
+
+// Byte offset within a fragment of row r's 8 k of group q (k = 8 q ..), of k step
+// ks. The row's slot is permuted by q and the parity of ks, within 128 bytes, so
+// that a wave writing a few rows' contiguous columns (operand tiles are loaded
+// so) spreads over the banks: unpermuted, the 8 groups of two k steps are 8-way
+// conflicts.
+__device__ __forceinline__ int frag_slot(int ks, int q, int r) {
+    return (q * 16 + (r ^ (q | (ks & 1) << 2))) * 16;
+}
+// Byte offset in a row block's fragments of the hi part of columns 16 T + 4 q ..
+// + 3 of row j: where an output column tile T lands as the next contraction's
+// operand (the lo part FRAG further on, row block rb 2 KS rb FRAG).
+__device__ __forceinline__ int frag_col(int T, int j, int q) {
+    return (T >> 1) * 2 * FRAG + frag_slot(T >> 1, (T & 1) * 2 + (q >> 1), j) + (q & 1) * 8;
+}
+
+}  // namespace
+
+// ---------------------------------------------------------------------------
+// k_token_mlp: the token half of a Swin block in one kernel,
+//   x1  = x + LN1(o Wproj^T + b),  out = x1 + LN2(GELU(x1 W1^T + b1) W2^T + b2),
+// reading the attention output o and the block input x once and writing the
+// block output once (the three GEMMs it replaces moved 600 MB per block at
+// 264 x 264 x 180 where this moves 150).
+//
+// A workgroup's 4 waves own 16 TN output columns each (C <= 64 TN), all of
+// them the task's rows: RB row blocks of 16 tokens, RB <= RBM, sized so that
+// the two operand tiles (P0: o, then x1; P1: one C-wide chunk of the hidden
+// layer) let two workgroups run per CU. The hidden layer is made and consumed
+// C columns at a time, fc2's accumulators kept across the chunks. x1 stays in
+// registers in fp32 for the last residual.
+//
+// Weights stream through a register ring of WD k steps, refilled as consumed,
+// through GEMM and task boundaries (every task walks the same stream). The row
+// scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(C)
+// max|ln_w| + max|ln_b| (a normalised value is at most sqrt(C)), the hidden
+// layer's from bound(x1) max_j sum_k |W1[j][k]| + max|b1| (|GELU(v)| <= |v|).
+//
+// Every task of a launch has RB row blocks (the launcher's choice), workgroup b
+// taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
+// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 118 us where the
+// three GEMMs took 228 (31.6 GFLOP as three f16 products each: 41 us of MFMA at
+// the rate real data reaches, the rest VALU, which does not overlap MFMA on a
+// SIMD, operand reads and barriers); 2,880 tokens 15 us against 3 launches of
+// about 11.
+// ---------------------------------------------------------------------------
+namespace {
+
+template <int TN, int RB> struct TokCfg {
+    static constexpr int CP = 64 * TN;                // padded width
+    static constexpr int KS = 2 * TN;                 // k steps per GEMM
+    // weight ring, k steps (a divisor of KS); with three row blocks of 180 the
+    // registers go to the operand prefetch instead of a third step (126 -> 119
+    // us at 69,696 tokens), with fewer the ring is what hides L2's latency
+    static constexpr int WD = TN == 3 ? (RB == 3 ? 2 : 3) : (TN == 2 ? 4 : 2);
+    static constexpr bool PRE = TN < 3 || RB == 3;  // operands read a k step ahead
+};
+
+template <int TN, int RB> struct TokState {
+    h8v w[TokCfg<TN, RB>::WD][TN][2];  // the weight ring
+    int wpos;                      // next k step of the stream to load
+};
+
+template <int TN, int RB>
+__device__ __forceinline__ void tok_load(TokState<TN, RB> &s, int slot, __amdgpu_buffer_rsrc_t rw, int wbase,
+                                         int lane) {
+#pragma unroll
+    for (int t = 0; t < TN; ++t)
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+            s.w[slot][t][p] = __builtin_bit_cast(
+                h8v, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16,
+                                                           wbase + ((s.wpos * TN + t) * 2 + p) * FRAG, 0));
+    ++s.wpos;
+}
+
+// acc += tile (RB row blocks, KS k steps) x the stream's next KS k steps
+template <int TN, int RB, bool TAIL>
+__device__ __forceinline__ void tok_gemm(f4v (&acc)[RB][TN], const char *tile, TokState<TN, RB> &s,
+                                         __amdgpu_buffer_rsrc_t rw, int wbase, int lane, int steps) {
+    using K = TokCfg<TN, RB>;
+    h8v a[2][RB][2];  // this k step's operands and the next one's
+    const int fr0 = frag_slot(0, lane >> 4, lane & 15), fr1 = frag_slot(1, lane >> 4, lane & 15);
+    auto read = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 1; p >= 0; --p)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+                a[ks & 1][rb][p] = *reinterpret_cast<const h8v *>(tile + ((rb * K::KS + ks) * 2 + p) * FRAG + (ks & 1 ? fr1 : fr0));
+    };
+    read(0);
+#pragma unroll
+    for (int ks = 0; ks < K::KS; ++ks) {
+        const int slot = ks % K::WD;
+        if (K::PRE && ks + 1 < K::KS) read(ks + 1);
+        if (!K::PRE && ks) read(ks);
+#pragma unroll
+        for (int m = 0; m < 3; ++m)
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int t = 0; t < TN; ++t)
+                    acc[rb][t] = MFMA16H(s.w[slot][t][m == 1], a[ks & 1][rb][m == 0], acc[rb][t]);
+        if (!TAIL || s.wpos < steps) tok_load<TN, RB>(s, slot, rw, wbase, lane);
+        // (without it the compiler hoists later steps' operand reads and spills)
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
+}  // namespace
+
+template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(TokMlpArgs g) {
+    using K = TokCfg<TN, RB>;
+    constexpr int KS = K::KS, CP = K::CP;
+    __shared__ __attribute__((aligned(16))) char P0[RB * KS * 2 * FRAG];
+    __shared__ __attribute__((aligned(16))) char P1[RB * KS * 2 * FRAG];
+    // per row: 4 waves' (sum, sum of squares) of LN2; LN1's, the 4 waves' max
+    // |x| and o's row unscale lie in P1, which is free until the first chunk
+    __shared__ __attribute__((aligned(16))) float red2[RB * 16][8];
+    __shared__ __attribute__((aligned(16))) float lnp[4 * CP];  // LN1, LN2 weights and biases
+    float(*const red1)[8] = reinterpret_cast<float(*)[8]>(P1);
+    float(*const redm)[4] = reinterpret_cast<float(*)[4]>(P1 + RB * 512);
+    float *const osc = reinterpret_cast<float *>(P1 + RB * 768);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    const int C = g.C;
+    const size_t plane = (size_t)g.M * C * 4;
+    const int steps = (1 + 2 * g.chunks) * KS;
+    const __amdgpu_buffer_rsrc_t rw = buf_rsrc(g.w, (size_t)4 * steps * TN * 2 * FRAG);
+    const int wbase = wave * steps * TN * 2 * FRAG;
+    const __amdgpu_buffer_rsrc_t rp = buf_rsrc(g.prm, (size_t)(8 + 2 * g.chunks) * CP * 4);
+    const float inv_c = g.inv_c;
+
+    for (int i = tid; i < CP; i += 256)
+        reinterpret_cast<float4 *>(lnp)[i] = buf_load4(rp, 16 * i);
+
+    TokState<TN, RB> st;
+
+    // o rows of a task: wave w takes rows 4w .. 4w + 3 of each row block, 16
+    // lanes a row, lane c float4s c, c + 16, ...
+    float4 oa[RB][TN];
+    f4v xn[RB][TN];  // the residual x at this lane's output columns
+    int ooff[TN], off[TN], foff[TN];  // o's loads, this lane's output columns, their fragments
+#pragma unroll
+    for (int t = 0; t < TN; ++t) {
+        const int f = j + 16 * t;
+        ooff[t] = 4 * f < C ? ((4 * wave + q) * C + 4 * f) * 4 : BUF_OOB;
+        const int c = 16 * (wave * TN + t) + 4 * q;
+        off[t] = c < C ? (j * C + c) * 4 : BUF_OOB;
+        foff[t] = frag_col(wave * TN + t, j, q);
+    }
+    const int osto = (j >> 3) * 2 * FRAG + frag_slot(j >> 3, (j >> 1) & 3, 4 * wave + q) + (j & 1) * 8;
+    const int nrb = g.M / 16;
+    auto load_rows = [&](int r0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const __amdgpu_buffer_rsrc_t r = buf_rsrc(g.o, r0 + rb < nrb ? plane : 0);
+#pragma unroll
+            for (int i = 0; i < TN; ++i) oa[rb][i] = buf_load4s(r, ooff[i], (r0 + rb) * 16 * C * 4);
+        }
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            const __amdgpu_buffer_rsrc_t r = buf_rsrc(g.x, r0 + rb < nrb ? plane : 0);
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+                xn[rb][t] = __builtin_bit_cast(f4v, buf_load4s(r, off[t], (r0 + rb) * 16 * C * 4));
+        }
+    };
+    // the parameter row `a`'s values at this lane's columns of tile t
+    auto prm4 = [&](int a, int t) __attribute__((always_inline)) {
+        return __builtin_bit_cast(f4v, buf_load4s(rp, 16 * q, (a * CP + 16 * (wave * TN + t)) * 4));
+    };
+    auto store_frag = [&](char *tile, int rb, int t, f4v v) __attribute__((always_inline)) {
+        h4v hi, lo;
+        split4(v, hi, lo);
+        char *d = tile + foff[t] + rb * KS * 2 * FRAG;
+        *reinterpret_cast<h4v *>(d) = hi;
+        *reinterpret_cast<h4v *>(d + FRAG) = lo;
+    };
+
+    load_rows(blockIdx.x * RB);
+    // as many dropped stores as a task's output has: the loop is entered with
+    // the same queue (o's loads, then stores) as it loops back with, so that
+    // the wait for o does not wait for the stores
+#pragma unroll
+    for (int i = 0; i < RB * TN; ++i) buf_store4(buf_rsrc(g.out, 0), 16 * i, make_float4(0.f, 0.f, 0.f, 0.f));
+#pragma unroll 1
+    for (int r0 = blockIdx.x * RB; r0 < nrb; r0 += gridDim.x * RB) {
+        // (a row block past the end reads zeros and stores nothing)
+        auto plane_of = [&](const float *p, int rb) __attribute__((always_inline)) {
+            return buf_rsrc(p, r0 + rb < nrb ? plane : 0);
+        };
+        st.wpos = 0;
+#pragma unroll
+        for (int s = 0; s < K::WD; ++s) tok_load<TN, RB>(st, s, rw, wbase, lane);
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- o into P0 ----
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            float m = 0.f;
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                const float4 v = oa[rb][i];
+                m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+            }
+            const int e = bound_exp(row16_max(m));
+            const float sc = exp_scale(e);
+            const int r = 4 * wave + q;
+            if (j == 0) osc[rb * 16 + r] = exp_unscale(e);
+#pragma unroll
+            for (int i = 0; i < TN; ++i) {
+                h4v hi, lo;
+                split4(__builtin_bit_cast(f4v, oa[rb][i]) * sc, hi, lo);
+                char *d = P0 + osto + (rb * KS * 2 + 4 * i) * FRAG;
+                *reinterpret_cast<h4v *>(d) = hi;
+                *reinterpret_cast<h4v *>(d + FRAG) = lo;
+            }
+        }
+        f4v x1[RB][TN];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) x1[rb][t] = xn[rb][t];
+        lds_sync();
+
+        // ---- proj, LN1, residual ----
+        f4v acc[RB][TN];
+        f4v cs[TN], b[TN];  // the GEMM's column unscales and biases, loaded ahead of it
+        auto load_cb = [&](int a) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                cs[t] = prm4(a, t);
+                b[t] = prm4(a + 1, t);
+            }
+        };
+        load_cb(4);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) acc[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
+        tok_gemm<TN, RB, false>(acc, P0, st, rw, wbase, lane, steps);
+
+        // v = acc scaled back + bias, its row sums (and max |x1|'s part) to
+        // LDS; after the barrier the rows' mean and 1/std
+        float mean[RB], rstd[RB];
+        auto norm_stats = [&](float(*red)[8], const float (&un)[RB]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                float s1 = 0.f, s2 = 0.f;
+#pragma unroll
+                for (int t = 0; t < TN; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = fmaf(acc[rb][t][i] * cs[t][i], un[rb], b[t][i]);
+                        acc[rb][t][i] = v;
+                        s1 += v;
+                        s2 = fmaf(v, v, s2);
+                    }
+                const float s = xrow_sum2(s1, s2);
+                if (lane < 32) red[rb * 16 + j][2 * wave + q] = s;
+            }
+        };
+        auto norm_finish = [&](const float(*red)[8]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const float4 u = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][0]);
+                const float4 v = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][4]);
+                const float m = ((u.x + u.z) + (v.x + v.z)) * inv_c;
+                const float var = fmaxf(((u.y + u.w) + (v.y + v.w)) * inv_c - m * m, 0.f);
+                rstd[rb] = __builtin_amdgcn_rsqf(var + 1e-5f);
+                mean[rb] = m * rstd[rb];
+            }
+        };
+        auto load_ln = [&](int a, f4v(&lw)[TN], f4v(&lb)[TN]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+                const float *d = lnp + a * CP + 16 * (wave * TN + t) + 4 * q;
+                lw[t] = *reinterpret_cast<const f4v *>(d);
+                lb[t] = *reinterpret_cast<const f4v *>(d + CP);
+            }
+        };
+        float un[RB];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) un[rb] = osc[rb * 16 + j];
+        norm_stats(red1, un);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) {
+            float m = 0.f;
+#pragma unroll
+            for (int t = 0; t < TN; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(x1[rb][t][i]));
+            m = xrow_max(m);
+            if (lane < 16) redm[rb * 16 + j][wave] = m;
+        }
+        lds_sync();
+        norm_finish(red1);
+        float hsc[RB];  // the hidden rows' scale (its inverse into un)
+        {
+            f4v lw[TN], lb[TN];
+            load_ln(0, lw, lb);
+            float hun[RB];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const float4 m4 = *reinterpret_cast<const float4 *>(&redm[rb * 16 + j][0]);
+                const float bx = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w)) + g.ln1_bound;
+                const int e = bound_exp(bx);
+                const int eh = bound_exp(fmaf(bx, g.fc1_l1, g.fc1_bmax));
+                const float sc = exp_scale(e);
+                un[rb] = exp_unscale(e);
+                hsc[rb] = exp_scale(eh);
+                hun[rb] = exp_unscale(eh);
+#pragma unroll
+                for (int t = 0; t < TN; ++t) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        x1[rb][t][i] += fmaf(fmaf(acc[rb][t][i], rstd[rb], -mean[rb]), lw[t][i], lb[t][i]);
+                    store_frag(P0, rb, t, x1[rb][t] * sc);
+                    // (kept in the output until LN2: its registers are
+                    // wanted in the MLP loop)
+                    buf_store4s(plane_of(g.out, rb), off[t], (r0 + rb) * 16 * C * 4, __builtin_bit_cast(float4, x1[rb][t]));
+                }
+            }
+            lds_sync();
+
+            // ---- the MLP, a C-wide chunk of the hidden layer at a time ----
+            f4v acc2[RB][TN];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int t = 0; t < TN; ++t) acc2[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int h = 0; h < g.chunks; ++h) {
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) acc[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
+                load_cb(8 + 2 * h);
+                tok_gemm<TN, RB, false>(acc, P0, st, rw, wbase, lane, steps);
+                if (h) lds_sync();  // every wave is past the last chunk's fc2
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int t = 0; t < TN; ++t) {
+                        f4v v;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            v[i] = gelu_erf(fmaf(acc[rb][t][i] * cs[t][i], un[rb], b[t][i])) * hsc[rb];
+                        store_frag(P1, rb, t, v);
+                    }
+                lds_sync();
+                load_cb(6);  // (used after the last chunk)
+                if (h + 1 == g.chunks)
+#pragma unroll
+                    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                        for (int t = 0; t < TN; ++t)
+                            x1[rb][t] = __builtin_bit_cast(f4v, buf_load4s(plane_of(g.out, rb), off[t], (r0 + rb) * 16 * C * 4));
+                tok_gemm<TN, RB, true>(acc2, P1, st, rw, wbase, lane, steps);
+            }
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                un[rb] = hun[rb];
+#pragma unroll
+                for (int t = 0; t < TN; ++t) acc[rb][t] = acc2[rb][t];
+            }
+        }
+        load_rows(r0 + gridDim.x * RB);
+        norm_stats(red2, un);
+        lds_sync();
+        norm_finish(red2);
+        f4v lw[TN], lb[TN];
+        load_ln(2, lw, lb);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int t = 0; t < TN; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    x1[rb][t][i] += fmaf(fmaf(acc[rb][t][i], rstd[rb], -mean[rb]), lw[t][i], lb[t][i]);
+                buf_store4s(plane_of(g.out, rb), off[t], (r0 + rb) * 16 * C * 4, __builtin_bit_cast(float4, x1[rb][t]));
+            }
+    }
+}
+
+// ---- host side ------------------------------------------------------------
+
+namespace {
+
+uint16_t f16_bits(float f) {
+    // round to nearest even; |f| < 2^15 by the scaling
+    uint32_t x;
+    memcpy(&x, &f, 4);
+    const uint32_t sign = (x >> 16) & 0x8000u;
+    const uint32_t a = x & 0x7fffffffu;
+    if (a > 0x7f800000u) return (uint16_t)(sign | 0x7e00u);
+    if (a >= 0x47800000u) return (uint16_t)(sign | 0x7c00u);
+    if (a < 0x38800000u) {
+        // subnormal: units of 2^-24 (the fp32 addition rounds to them)
+        float m;
+        memcpy(&m, &a, 4);
+        const float r = m + 0.5f;
+        uint32_t y;
+        memcpy(&y, &r, 4);
+        return (uint16_t)(sign | (y - 0x3f000000u));
+    }
+    const uint32_t r = a + 0xfffu + ((a >> 13) & 1u);
+    return (uint16_t)(sign | ((r - 0x38000000u) >> 13));
+}
+float f16_value(uint16_t h) {
+    const uint32_t e = (h >> 10) & 31, m = h & 0x3ffu;
+    float v = e == 0 ? ldexpf((float)m, -24) : e == 31 ? (m ? NAN : INFINITY) : ldexpf((float)(m | 0x400u), (int)e - 25);
+    return (h & 0x8000u) ? -v : v;
+}
+
+}  // namespace
+
+float split_row_scale(const float *w, int n) {
+    float m = 0.f;
+    for (int i = 0; i < n; ++i) m = std::max(m, std::fabs(w[i]));
+    if (!(m > 0.f) || !std::isfinite(m)) return 1.f;
+    int e;
+    (void)frexpf(m, &e);  // m = f 2^e, f in [0.5, 1)
+    return ldexpf(1.f, std::min(std::max(15 - e, -126), 126));
+}
+
+void split_pack_step(const float *const *rows, const float *scale, int k0, int kn, uint16_t *dst) {
+    for (int p = 0; p < 2; ++p)
+        for (int l = 0; l < 64; ++l)
+            for (int i = 0; i < 8; ++i) {
+                const int k = k0 + 8 * (l >> 4) + i;
+                const float *row = rows[l & 15];
+                const float v = row && k < kn ? row[k] * scale[l & 15] : 0.f;
+                const uint16_t hi = f16_bits(v);
+                dst[(size_t)p * 512 + l * 8 + i] = p == 0 ? hi : f16_bits(v - f16_value(hi));
+            }
+}
+
+bool token_mlp_takes(int C, int ratio) { return C % 4 == 0 && C <= 192 && ratio >= 1; }
+static int tok_tn(int C) { return (C + 63) / 64; }
+size_t token_mlp_weight_floats(int C, int ratio) {
+    const int tn = tok_tn(C);
+    return (size_t)4 * (1 + 2 * ratio) * 2 * tn * tn * 2 * (FRAG / 4);
+}
+size_t token_mlp_param_floats(int C, int ratio) { return (size_t)(8 + 2 * ratio) * 64 * tok_tn(C); }
+
+void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *prm, float *ln1_bound,
+                    float *fc1_l1, float *fc1_bmax) {
+    const int tn = tok_tn(C), CP = 64 * tn, ks = 2 * tn;
+    uint16_t *dst = reinterpret_cast<uint16_t *>(w);
+    std::fill(prm, prm + token_mlp_param_floats(C, ratio), 0.f);
+    std::vector<float> sp(C), s2(C), s1((size_t)ratio * C);
+    for (int c = 0; c < C; ++c) {
+        sp[c] = split_row_scale(h.wproj + (size_t)c * C, C);
+        s2[c] = split_row_scale(h.w2 + (size_t)c * ratio * C, ratio * C);
+        prm[c] = h.n1w[c];
+        prm[CP + c] = h.n1b[c];
+        prm[2 * CP + c] = h.n2w[c];
+        prm[3 * CP + c] = h.n2b[c];
+        prm[4 * CP + c] = 1.f / sp[c];
+        prm[5 * CP + c] = h.bproj[c];
+        prm[6 * CP + c] = 1.f / s2[c];
+        prm[7 * CP + c] = h.b2[c];
+    }
+    float l1 = 0.f, bmax = 0.f, nw = 0.f, nb = 0.f;
+    for (int o = 0; o < ratio * C; ++o) {
+        const float *row = h.w1 + (size_t)o * C;
+        s1[o] = split_row_scale(row, C);
+        const int ch = o / C, c = o % C;
+        prm[(8 + 2 * ch) * CP + c] = 1.f / s1[o];
+        prm[(9 + 2 * ch) * CP + c] = h.b1[o];
+        double a = 0.0;
+        for (int k = 0; k < C; ++k) a += std::fabs((double)row[k]);
+        l1 = std::max(l1, (float)a);
+        bmax = std::max(bmax, std::fabs(h.b1[o]));
+    }
+    for (int c = 0; c < C; ++c) {
+        nw = std::max(nw, std::fabs(h.n1w[c]));
+        nb = std::max(nb, std::fabs(h.n1b[c]));
+    }
+    *ln1_bound = sqrtf((float)C) * nw + nb;
+    *fc1_l1 = l1;
+    *fc1_bmax = bmax;
+    // the stream of each wave: proj, then per chunk fc1 and fc2
+    for (int wave = 0; wave < 4; ++wave)
+        for (int gm = 0; gm < 1 + 2 * ratio; ++gm)
+            for (int s = 0; s < ks; ++s)
+                for (int t = 0; t < tn; ++t, dst += FRAG) {
+                    const float *rows[16];
+                    float sc[16];
+                    const int ch = (gm - 1) / 2;
+                    for (int r = 0; r < 16; ++r) {
+                        const int c = 16 * (wave * tn + t) + r;
+                        rows[r] = nullptr;
+                        sc[r] = 0.f;
+                        if (c >= C) continue;
+                        if (gm == 0) {
+                            rows[r] = h.wproj + (size_t)c * C;
+                            sc[r] = sp[c];
+                        } else if (gm % 2 == 1) {
+                            rows[r] = h.w1 + ((size_t)ch * C + c) * C;
+                            sc[r] = s1[(size_t)ch * C + c];
+                        } else {
+                            rows[r] = h.w2 + (size_t)c * ratio * C + (size_t)ch * C;
+                            sc[r] = s2[c];
+                        }
+                    }
+                    split_pack_step(rows, sc, 32 * s, C, dst);
+                }
+}
+
+static int split_cus() {
+    static thread_local int dev_of = -1, cus = 0;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 256;
+    if (dev != dev_of) {
+        int n = 0;
+        cus = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
+        dev_of = dev;
+    }
+    return cus;
+}
+
+// Workgroups of a task size that run at once (by registers and LDS).
+static int tok_slots(int C, int rb) { return split_cus() * (tok_tn(C) > 1 ? 2 : rb < 4 ? 4 : 3); }
+// Row blocks per task: the count whose rounds over those slots take least, a
+// round costing its row blocks plus a constant of about one (its weight stream,
+// barriers and latencies).
+static int tok_rb(int M, int C) {
+    const int nrb = M / 16;
+    int best = 1;
+    long best_cost = 0;
+    for (int rb = 1; rb <= (tok_tn(C) == 1 ? 4 : 3); ++rb) {
+        const int tasks = (nrb + rb - 1) / rb, slots = tok_slots(C, rb);
+        const long cost = (long)((tasks + slots - 1) / slots) * (rb + 1);
+        if (rb == 1 || cost <= best_cost) {
+            best = rb;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+unsigned token_mlp_grid(int M, int C) {
+    const int rb = tok_rb(M, C), tasks = (M / 16 + rb - 1) / rb;
+    return (unsigned)std::max(1, std::min(tasks, tok_slots(C, rb)));
+}
+
+template <int TN> static void tok_launch(const TokMlpArgs &g, int rb, dim3 grid, hipStream_t st) {
+    switch (rb) {
+    case 1: hipLaunchKernelGGL((k_token_mlp<TN, 1>), grid, dim3(256), 0, st, g); break;
+    case 2: hipLaunchKernelGGL((k_token_mlp<TN, 2>), grid, dim3(256), 0, st, g); break;
+    case 3: hipLaunchKernelGGL((k_token_mlp<TN, 3>), grid, dim3(256), 0, st, g); break;
+    default:
+        if constexpr (TN == 1) hipLaunchKernelGGL((k_token_mlp<TN, 4>), grid, dim3(256), 0, st, g);
+        break;
+    }
+}
+
+hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st) {
+    if (g.M <= 0 || g.M % 16 || !token_mlp_takes(g.C, g.chunks)) return hipErrorInvalidValue;
+    const dim3 grid(token_mlp_grid(g.M, g.C));
+    const int rb = tok_rb(g.M, g.C);
+    switch (tok_tn(g.C)) {
+    case 1: tok_launch<1>(g, rb, grid, st); break;
+    case 2: tok_launch<2>(g, rb, grid, st); break;
+    default: tok_launch<3>(g, rb, grid, st); break;
+    }
+    return hipGetLastError();
+}

@@ -20,7 +20,7 @@ fn build_hip() {
     let out = std::env::var("OUT_DIR").expect("OUT_DIR");
     let hipcc = std::env::var("HIPCC").unwrap_or_else(|_| "/opt/rocm/bin/hipcc".into());
     let arch = std::env::var("SWIN2SR_HIP_ARCH").unwrap_or_else(|_| "gfx950".into());
-    let srcs = ["s2s_kernels.hip", "s2s_api.cpp", "s2s_test_api.cpp", "s2s_selftest.cpp"];
+    let srcs = ["s2s_kernels.hip", "s2s_split.hip", "s2s_api.cpp", "s2s_test_api.cpp", "s2s_selftest.cpp"];
     let status = Command::new(&hipcc)
         .arg(format!("--offload-arch={arch}"))
         .args(["-O3", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
@@ -39,7 +39,7 @@ fn build_hip() {
     println!("cargo:rustc-link-search=native={out}");
     println!("cargo:rustc-link-lib=dylib=swin2sr_hip");
     println!("cargo:rustc-link-arg=-Wl,-rpath,{out}");
-    for s in srcs.iter().chain(["s2s_kernels.h", "swin2sr_hip.h"].iter()) {
+    for s in srcs.iter().chain(["s2s_kernels.h", "s2s_device.h", "swin2sr_hip.h"].iter()) {
         println!("cargo:rerun-if-changed=hip/{s}");
     }
     println!("cargo:rerun-if-env-changed=HIPCC");
