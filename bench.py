@@ -46,7 +46,9 @@ METRIC = "output Mpix/s classical-x4 256²→1024² fp32 @1 GPU; % MFMA / HBM ro
 MFMA_FP32_PEAK = 157.3e12   # MI355X dense fp32 matrix, FLOP/s (AMD spec)
 HBM_PEAK = 8.0e12           # MI355X HBM3E, B/s (AMD spec)
 VALU_FP32_PEAK = 78.6e12    # MI355X fp32 vector FMA (256 CUs x 4 SIMDs x 16 lanes x 2 x 2.4 GHz)
-FLOP_PEAK = {"mfma": MFMA_FP32_PEAK, "valu": VALU_FP32_PEAK}
+MFMA_F16_PEAK = 2516.6e12   # MI355X dense f16 matrix, FLOP/s (AMD spec)
+# "split": fp32 contractions as three f16 products each (s2s_split.hip)
+FLOP_PEAK = {"mfma": MFMA_FP32_PEAK, "split": MFMA_F16_PEAK / 3, "valu": VALU_FP32_PEAK}
 
 
 def log(*a):
@@ -67,14 +69,14 @@ def kernel_work(arch, h, w, hp=None, wp=None):
     f = 4
     work = {
         "qkv": ("mfma", 2 * P * 3 * C * C, f * P * (C + 3 * C)),
-        # 6 heads of 30: the qkv projection and the window attention as one
+        # 6 heads of 30 or 10: the qkv projection and the window attention as one
         # kernel (x in, the attention output out; q, k, v stay on the CU)
-        "qkv_window_attention": ("mfma", 2 * P * 3 * C * C + 4 * P * win * win * C,
+        "qkv_window_attention": ("split", 2 * P * 3 * C * C + 4 * P * win * win * C,
                                  f * (P * 2 * C + 3 * C * C)),
         "window_attention": ("mfma", 4 * P * win * win * C, f * P * (3 * C + C)),
         # proj + LayerNorm + residual, fc1 + GELU, fc2 + LayerNorm + residual as
         # one kernel (the attention output and the block input in, the block out)
-        "token_mlp": ("mfma", 2 * P * (C * C + 2 * Hd * C), f * P * 3 * C),
+        "token_mlp": ("split", 2 * P * (C * C + 2 * Hd * C), f * P * 3 * C),
         "proj_ln_res": ("mfma", 2 * P * C * C, f * P * 3 * C),
         "fc1_gelu": ("mfma", 2 * P * Hd * C, f * P * (C + Hd)),
         "fc2_ln_res": ("mfma", 2 * P * C * Hd, f * P * (Hd + 2 * C)),
@@ -230,7 +232,7 @@ def roofline_of(work, kernel, ms, n, traffic=True):
         achieved, peak, unit = fl / avg_s / 1e12, FLOP_PEAK[bound] / 1e12, "TFLOP/s"
     else:
         achieved, peak, unit = by / avg_s / 1e9, HBM_PEAK / 1e9, "GB/s"
-    return {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": unit,
+    return {"bound": "mfma" if bound == "split" else bound, "achieved": round(achieved, 3), "peak": peak, "unit": unit,
             "frac": round(achieved / peak, 4),
             "traffic": traffic_from_profiles(kernel) if traffic else None,
             "kernel": kernel, "avg_ms": round(avg_s * 1e3, 4), "launches": n,

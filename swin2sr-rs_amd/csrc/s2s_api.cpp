@@ -62,6 +62,9 @@ struct BlockW {
     float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr;
     float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
     float *ls = nullptr, *cpbt = nullptr;
+    // wqkv as k_qkv_attn reads it (qkv_attn_pack) for the head shapes it takes
+    float *qkv_prm = nullptr;
+    float v_l1 = 0.f, v_bmax = 0.f;
     // the token half as k_token_mlp reads it (token_mlp_pack), for the widths
     // it takes; wproj .. b2 above are then not uploaded
     float *tok_w = nullptr, *tok_prm = nullptr;
@@ -766,20 +769,22 @@ int s2s_ctx::block_fwd(const BlockW &b, int hp, int wp, int shift, const float *
     const int P = hp * wp;
     GemmArgs g;
     if (qkv_attn_fused(arch.heads, hd)) {
-        // 6 heads of 30: the qkv projection and the window attention as one
-        // kernel (the head pair's q, k, v never leave the CU)
+        // 6 heads of 30 or 10: the qkv projection and the window attention as
+        // one kernel (a window's q, k, v never leave the CU)
         QkvAttnArgs a{};
         a.x = x_in;
         a.w = b.wqkv;
-        a.bias = b.bqkv;
+        a.prm = b.qkv_prm;
+        a.v_l1 = b.v_l1;
+        a.v_bmax = b.v_bmax;
         a.cpbt = b.cpbt;
         a.logit_scale = b.ls;
         a.out = o;
         a.hp = hp;
         a.wp = wp;
         a.shift = shift;
-        if (run("qkv_window_attention", dim3(qkv_attention_grid(hp, wp)), dim3(256),
-                [&] { return launch_qkv_attention(a, stream, nullptr); }))
+        if (run("qkv_window_attention", dim3(qkv_attention_grid(hp, wp, hd)), dim3(hd == 30 ? 256 : 384),
+                [&] { return launch_qkv_attention(a, hd, stream); }))
             return -1;
     } else {
         // qkv straight into the window attention's unit layout where its
@@ -1435,11 +1440,11 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
     f += body_conv + C;         // conv_after_body
     for (int s = 0; s < A.n_stages; ++s) {
         f += body_conv + C;     // the stage close (3x3 with the 1x1 folded in)
-        // the fused qkv (per head pair when the qkv + attention kernel takes
-        // the head shape), proj, fc1, fc2 in their GEMMs' layouts
-        const uint64_t wqkv = qkv_attn_fused(A.heads, A.embed / A.heads)
-                                  ? (uint64_t)(A.heads / 2) * weight_floats(C, C, EPI_STORE)
-                                  : weight_floats(3 * C, C, EPI_STORE);
+        // the fused qkv in the qkv + attention kernel's layout, or the GEMM's
+        const int hd = A.embed / A.heads;
+        const uint64_t wqkv = qkv_attn_fused(A.heads, hd)
+                                  ? qkv_attn_weight_floats(hd) + qkv_attn_param_floats(hd)
+                                  : weight_floats(3 * C, C, EPI_STORE) + 3 * C;
         // the token half: k_token_mlp's stream and parameters, or proj, norm1,
         // norm2, fc1 and fc2 one by one
         const uint64_t tok = token_mlp_takes(A.embed, A.mlp_ratio)
@@ -1448,7 +1453,7 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
                                  : weight_floats(C, C, EPI_LN_RES) + C + 4 * C +
                                        weight_floats(H2, C, EPI_GELU) + H2 +
                                        weight_floats(C, H2, EPI_LN_RES) + C;
-        const uint64_t per_block = wqkv + 3 * C     // fused qkv, its bias
+        const uint64_t per_block = wqkv             // fused qkv, its bias
                                    + NH             // logit scale
                                    + tok
                                    + NH * n * n;    // the CPB table
@@ -1682,17 +1687,13 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
             std::copy(qb->data, qb->data + C, bqkv.begin());
             std::copy(vb->data, vb->data + C, bqkv.begin() + 2 * C);
             if (qkv_attn_fused(NH, C / NH)) {
-                // the fused qkv + attention kernel's order: each head pair's
-                // q|k|v rows as the attention unit's columns, each pair's
-                // C x C rows in register order
-                std::vector<float> wp(wqkv.size()), bp(bqkv.size());
-                qkv_pair_weights(wqkv.data(), bqkv.data(), NH, C / NH, wp.data(), bp.data());
-                wqkv = gemm_weights(wp, NH / 2, C, C, EPI_STORE);
-                bqkv.swap(bp);
+                std::vector<float> w(qkv_attn_weight_floats(C / NH)), prm(qkv_attn_param_floats(C / NH));
+                qkv_attn_pack(wqkv.data(), bqkv.data(), C / NH, w.data(), prm.data(), &bw.v_l1, &bw.v_bmax);
+                rc = rc || ctx->upload(w, &bw.wqkv) || ctx->upload(prm, &bw.qkv_prm);
             } else {
                 wqkv = gemm_weights(wqkv, 1, 3 * C, C, EPI_STORE);
+                rc = rc || ctx->upload(wqkv, &bw.wqkv) || ctx->upload(bqkv, &bw.bqkv);
             }
-            rc = rc || ctx->upload(wqkv, &bw.wqkv) || ctx->upload(bqkv, &bw.bqkv);
             const s2s_tensor *lsx;
             rc = rc || ts.get(p + "attn.logit_scale", {NH, 1, 1}, &lsx);
             if (rc) break;

@@ -42,6 +42,9 @@ typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 #define MFMA16H(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16((a), (b), (c), 0, 0, 0)
 
+#ifndef QOCC
+#define QOCC 2
+#endif
 namespace {
 
 // 2^(14 - floor(log2 b)) for a bound b >= 0 (the exponent clamped so that the
@@ -52,14 +55,20 @@ __device__ __forceinline__ int bound_exp(float b) {
 __device__ __forceinline__ float exp_scale(int e) { return __builtin_bit_cast(float, (268 - e) << 23); }
 __device__ __forceinline__ float exp_unscale(int e) { return __builtin_bit_cast(float, (e - 14) << 23); }
 
-// hi and lo of 4 values. The residuals pass through fp32 registers (the empty
-// asm): the compiler would fuse the subtraction and the conversion into
-// v_fma_mixlo_f16 / v_fma_mixhi_f16, which issue at a quarter of the rate
-// (measured 3.7 ns against 1.9 for v_fma_mix_f32 or the packed conversion and
-// 1.2 for v_fma_f32).
+// hi and lo of 4 values. Values and residuals pass through fp32 registers (the
+// empty asm). Left to itself the compiler folds a scaling into the conversions
+// (v_fma_mixlo_f16 rounds once where the packed conversion of the rounded
+// product rounds twice, so the stored hi could differ from the one subtracted),
+// and those issue at a quarter of the rate: measured 3.7 ns against 1.9 for
+// v_fma_mix_f32 or the packed conversion and 1.2 for v_fma_f32.
 __device__ __forceinline__ void split4(f4v v, h4v &hi, h4v &lo) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) hi[i] = (_Float16)v[i];
+    for (int i = 0; i < 4; ++i) {
+        float x = v[i];
+        asm("" : "+v"(x));
+        v[i] = x;
+        hi[i] = (_Float16)x;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float r = fmaf((float)hi[i], -1.0f, v[i]);
@@ -86,6 +95,16 @@ __device__ __forceinline__ float xrow_max(float a) {
     float d = c;
     asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
     return fmaxf(c, d);
+}
+
+// ... and the sum.
+__device__ __forceinline__ float xrow_sum(float a) {
+    float b = a;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(a), "+v"(b));
+    float c = a + b;
+    float d = c;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(c), "+v"(d));
+    return c + d;
 }
 
 constexpr int FRAG = 1024;  // bytes of one fragment
@@ -475,6 +494,385 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_qkv_attn: a block's qkv projection and window attention in one kernel, for
+// 6 heads of 30 and 6 heads of 10 (every released checkpoint). An item is a
+// window and a group of its heads (two of 30, all six of 10): 64 tokens, 60 q, 60
+// k and 60 v columns. Per item a workgroup
+//   - loads the window's token rows (the block's shifted-window order, with
+//     torch.roll's wrap), an item ahead, scales and splits them into LDS;
+//   - multiplies them by the group's q|k|v weights, streamed from L2 through
+//     registers: each wave owns three 16-column tiles, two of q or k (weights
+//     as the MFMA's A operand: a lane holds a token's consecutive columns) and
+//     one of v (tokens as A: a lane holds a column's consecutive tokens);
+//   - normalises q and k (a head's columns are in one wave, so the norm is one
+//     reduction over the lanes), splits q, k and v and writes them over the
+//     token tile as the operands of the two attention products;
+//   - S^T = K Q^T, the CPB bias, the shift mask and the softmax with a lane
+//     holding one query, then O^T = V^T P^T with P straight from the registers
+//     (the k slots of that product are numbered as S^T's accumulator rows, so
+//     P needs no exchange between lanes); row HD of V^T is ones, so that row of
+//     O^T is the softmax denominator.
+// Head columns are padded to whole tiles: 30 to 32, 10 to 16. The scales: x's
+// rows from their maximum; q and k are unit vectors (2^14); the probabilities
+// are at most 1 (2^14, in the exponent's argument); v from the bound max|x|
+// max_j sum_k |Wv[j][k]| + max|bv| over the window.
+//
+// Items go to workgroups as window w on XCD w % 8, a window's groups one after
+// another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 83
+// us (the fp32 MFMA form with the weights in registers took 146); 2,880 tokens
+// 13.4 (19.9). 6 heads of 10: 5,184 tokens 13.7 us and 526,592 286, where the
+// qkv GEMM and the attention as two kernels took 20.6 and 355. With three
+// workgroups per CU (168 registers) the form of 30 spills 76 registers.
+// ---------------------------------------------------------------------------
+typedef float f16acc __attribute__((ext_vector_type(16)));
+#define MFMA32H(a, b, c) __builtin_amdgcn_mfma_f32_32x32x16_f16((a), (b), (c), 0, 0, 0)
+
+namespace {
+
+template <int HD> struct QaCfg {
+    static constexpr int NW = HD > 16 ? 4 : 6;       // waves
+    static constexpr int NG = HD > 16 ? 3 : 1;       // head groups
+    static constexpr int GH = 6 / NG;                // heads per group
+    static constexpr int C = 6 * HD;
+    static constexpr int TF = (C + 63) / 64;         // float4s of a row per lane of 16
+    static constexpr int KS = 2 * TF;                // k steps of the projection
+    static constexpr int DS = HD > 16 ? 2 : 1;       // k steps of q . k
+    static constexpr int VR = HD > 16 ? 32 : 16;     // rows of a v operand
+    static constexpr int QB = DS * 2 * FRAG;         // bytes of 32 queries of a head
+    static constexpr int VB = 2 * VR * 32;           // bytes of 16 keys of a head's v, both parts
+    static constexpr int HB = 4 * QB + 4 * VB;       // bytes of a head: q, k, v
+    static constexpr int TILE = 4 * KS * 2 * FRAG;   // bytes of the token tile
+    static constexpr int BUF = GH * HB > TILE ? GH * HB : TILE;
+};
+
+}  // namespace
+
+template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, QOCC) void k_qkv_attn(QkvAttnArgs g) {
+    using K = QaCfg<HD>;
+    constexpr int KS = K::KS, C = K::C, NW = K::NW, TF = K::TF, DS = K::DS, NT = 64 * NW;
+    constexpr int SUM_E = 4 * (HD / 8) + (HD % 8) % 4, SUM_HH = (HD % 8) / 4;
+    constexpr int NST = (64 + NT / 16 - 1) / (NT / 16);  // output stores per thread
+    __shared__ __attribute__((aligned(16))) char buf[K::BUF];
+    __shared__ __attribute__((aligned(16))) float xun[64];  // the rows' unscale
+    __shared__ __attribute__((aligned(16))) float xmx[64];  // the rows' max |x|
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    const int r = lane & 31, hh = lane >> 5;
+    const int shift = g.shift;
+    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(g.x, (size_t)g.hp * g.wp * C * 4);
+    const __amdgpu_buffer_rsrc_t ro = buf_rsrc(g.out, (size_t)g.hp * g.wp * C * 4);
+    const __amdgpu_buffer_rsrc_t rw = buf_rsrc(g.w, (size_t)K::NG * NW * KS * 6 * FRAG);
+    const __amdgpu_buffer_rsrc_t rp = buf_rsrc(g.prm, (size_t)K::NG * NW * 3 * 32 * 4);
+
+    // items of this XCD: window xcd + 8 (i / NG), group i % NG
+    const int xcd = blockIdx.x & 7;
+    const int nitem = ((g.nw - xcd + 7) >> 3) * K::NG, istep = gridDim.x >> 3;
+
+    // x rows of an item: wave w < 4 takes tokens 16 rb + 4 w + q, 16 lanes a row
+    float4 xa[4][TF];
+    auto load_x = [&](int it) __attribute__((always_inline)) {
+        const int wi = xcd + 8 * (it / K::NG);
+        const int wh = wi / g.nww, ww = wi - wh * g.nww;
+        const bool on = it < nitem;
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) {
+            const int t = 16 * rb + 4 * wave + q;
+            int y = 8 * wh + (t >> 3) + shift;
+            if (y >= g.hp) y -= g.hp;
+            int x = 8 * ww + (t & 7) + shift;
+            if (x >= g.wp) x -= g.wp;
+            const int o = ((y * g.wp + x) * C + 4 * j) * 4;
+#pragma unroll
+            for (int i = 0; i < TF; ++i) xa[rb][i] = buf_load4(rx, on && 4 * (j + 16 * i) < C ? o + 256 * i : BUF_OOB);
+        }
+    };
+    h8v w[2][3][2];
+    int wbase = 0;
+    auto load_w = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+#pragma unroll
+            for (int p = 0; p < 2; ++p)
+                w[ks & 1][t][p] = __builtin_bit_cast(
+                    h8v, __builtin_amdgcn_raw_buffer_load_b128(rw, lane * 16, wbase + ((ks * 3 + t) * 2 + p) * FRAG, 0));
+    };
+
+    const int fr0 = frag_slot(0, q, j), fr1 = frag_slot(1, q, j);
+    const int osto = (j >> 3) * 2 * FRAG + frag_slot(j >> 3, (j >> 1) & 3, 4 * (wave & 3) + q) + (j & 1) * 8;
+
+    int it = blockIdx.x >> 3;
+    if (wave < 4) load_x(it);
+#pragma unroll 1
+    for (; it < nitem; it += istep) {
+        const int hg = it % K::NG;
+        const int wi = xcd + 8 * (it / K::NG);
+        const int wh = wi / g.nww, ww = wi - wh * g.nww;
+        wbase = (hg * NW + wave) * KS * 6 * FRAG;
+        load_w(0);
+        load_w(1);
+        // the tiles' column unscales and biases: q and k tiles as the lane's 4
+        // columns, the v tile as its one
+        f4v cs[2], bi[2];
+        float csv, biv;
+        {
+            const int pb = (hg * NW + wave) * 96 * 4;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                cs[t] = __builtin_bit_cast(f4v, buf_load4s(rp, 16 * q, pb + t * 128));
+                bi[t] = __builtin_bit_cast(f4v, buf_load4s(rp, 16 * q, pb + t * 128 + 64));
+            }
+            csv = buf_load1(rp, pb + 256 + 4 * j);
+            biv = buf_load1(rp, pb + 320 + 4 * j);
+        }
+        // ---- x into the token tile ----
+        if (wave < 4) {
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                float m = 0.f;
+#pragma unroll
+                for (int i = 0; i < TF; ++i) {
+                    const float4 v = xa[rb][i];
+                    m = fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+                }
+                m = row16_max(m);
+                const int e = bound_exp(m);
+                const float sc = exp_scale(e);
+                if (j == 0) {
+                    xun[16 * rb + 4 * wave + q] = exp_unscale(e);
+                    xmx[16 * rb + 4 * wave + q] = m;
+                }
+#pragma unroll
+                for (int i = 0; i < TF; ++i) {
+                    h4v hi, lo;
+                    split4(__builtin_bit_cast(f4v, xa[rb][i]) * sc, hi, lo);
+                    char *d = buf + osto + (rb * KS * 2 + 4 * i) * FRAG;
+                    *reinterpret_cast<h4v *>(d) = hi;
+                    *reinterpret_cast<h4v *>(d + FRAG) = lo;
+                }
+            }
+        }
+        lds_sync();
+
+        // ---- q | k | v ----
+        f4v acc[4][3];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) acc[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            h8v a[4][2];
+#pragma unroll
+            for (int p = 1; p >= 0; --p)
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb)
+                    a[rb][p] = *reinterpret_cast<const h8v *>(buf + ((rb * KS + ks) * 2 + p) * FRAG + (ks & 1 ? fr1 : fr0));
+#pragma unroll
+            for (int m = 0; m < 3; ++m)
+#pragma unroll
+                for (int rb = 0; rb < 4; ++rb) {
+#pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        acc[rb][t] = MFMA16H(w[ks & 1][t][m == 1], a[rb][m == 0], acc[rb][t]);
+                    acc[rb][2] = MFMA16H(a[rb][m == 0], w[ks & 1][2][m == 1], acc[rb][2]);
+                }
+            if (ks + 2 < KS) load_w(ks + 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (wave < 4) load_x(it + istep);
+        // v's scale: the largest row maximum of the window
+        float vmx = xmx[lane];
+        vmx = xrow_max(row16_max(vmx));
+        const int ev = bound_exp(fmaf(vmx, g.v_l1, g.v_bmax));
+        const float vsc = exp_scale(ev);
+        lds_sync();  // every wave has read the token tile
+        {
+            // q and k: unit vectors times 2^14. A head of 30 has both tiles
+            // (q in waves 0-1, k in waves 2-3), a head of 10 one of each
+            char *dq[2];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const int head = DS == 2 ? (wave & 1) : wave;
+                const int isk = DS == 2 ? (wave >> 1) : t;
+                const int st = DS == 2 ? t : 0;
+                dq[t] = buf + head * K::HB + isk * 2 * K::QB + st * 2 * FRAG + ((q >> 1) * 32 + j) * 16 + (q & 1) * 8;
+            }
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                const float un = xun[16 * rb + j];
+                float ss[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    ss[t] = 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float v = fmaf(acc[rb][t][i] * cs[t][i], un, bi[t][i]);
+                        acc[rb][t][i] = v;
+                        ss[t] = fmaf(v, v, ss[t]);
+                    }
+                }
+                if (DS == 2) ss[0] = ss[1] = xrow_sum(ss[0] + ss[1]);
+                else {
+                    ss[0] = xrow_sum(ss[0]);
+                    ss[1] = xrow_sum(ss[1]);
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const float n = 16384.f * __builtin_amdgcn_rsqf(fmaxf(ss[t], 1e-24f));
+                    h4v hi, lo;
+                    split4(acc[rb][t] * n, hi, lo);
+                    char *d = dq[t] + (rb >> 1) * K::QB + (rb & 1) * 256;
+                    *reinterpret_cast<h4v *>(d) = hi;
+                    *reinterpret_cast<h4v *>(d + FRAG) = lo;
+                }
+            }
+            // v: row d, 16 keys 16 rb .. a fragment, the ones row at d = HD
+            const int vh = DS == 2 ? (wave >> 1) : wave, d = DS == 2 ? 16 * (wave & 1) + j : j;
+            char *dv = buf + vh * K::HB + 4 * K::QB + ((q & 1) * K::VR + d) * 16 + (q >> 1) * 8;
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+                const f4v un = *reinterpret_cast<const f4v *>(&xun[16 * rb + 4 * q]);
+                f4v v;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    v[i] = fmaf(acc[rb][2][i] * csv, un[i], biv) * vsc;
+                    v[i] = d == HD ? 1.0f : v[i];
+                }
+                h4v hi, lo;
+                split4(v, hi, lo);
+                *reinterpret_cast<h4v *>(dv + rb * K::VB) = hi;
+                *reinterpret_cast<h4v *>(dv + rb * K::VB + K::VB / 2) = lo;
+            }
+        }
+        lds_sync();
+
+        // ---- attention: this wave's head, 32 queries at a time ----
+#pragma unroll
+        for (int jb = 0; jb < 3 - DS; ++jb) {
+            const int hl = DS == 2 ? (wave >> 1) : wave, qt = DS == 2 ? (wave & 1) : jb;
+            const int head = hg * K::GH + hl, qtok = 32 * qt + r;
+            char *const hb = buf + hl * K::HB;
+            const float *cp = g.cpbt + ((size_t)head * 64 + qtok) * 64 + 4 * hh;
+            f4v cb[2][4];
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) cb[kt][a] = *reinterpret_cast<const f4v *>(cp + 32 * kt + 8 * a);
+            // logit scale x log2(e), the two 2^14 taken out
+            const float ls = ATTN_LOG2E * __expf(fminf(g.logit_scale[head], 4.605170185988092f)) * (1.0f / 268435456.0f);
+            h8v qf[DS][2];
+#pragma unroll
+            for (int s = 0; s < DS; ++s)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+                    qf[s][p] = *reinterpret_cast<const h8v *>(hb + qt * K::QB + (s * 2 + p) * FRAG + lane * 16);
+            f16acc sa[2];
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                h8v kf[DS][2];
+#pragma unroll
+                for (int s = 0; s < DS; ++s)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p)
+                        kf[s][p] = *reinterpret_cast<const h8v *>(hb + (2 + kt) * K::QB + (s * 2 + p) * FRAG + lane * 16);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) sa[kt][e] = 0.f;
+#pragma unroll
+                for (int m = 0; m < 3; ++m)
+#pragma unroll
+                    for (int s = 0; s < DS; ++s) sa[kt] = MFMA32H(kf[s][m == 1], qf[s][m == 0], sa[kt]);
+            }
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) sa[kt][e] = fmaf(sa[kt][e], ls, cb[kt][e >> 2][e & 3]);
+            // shift mask (last window row / column of a shifted block)
+            const bool ey = shift && (wh * 8 + 8 >= g.hp);
+            const bool ex = shift && (ww * 8 + 8 >= g.wp);
+            if (ey || ex) {
+                const bool qy = (qtok >> 3) < 8 - shift;
+                const bool qx = (qtok & 7) < 8 - shift;
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const int krw = 4 * kt + (e >> 2);
+                        const int kcl = 4 * hh + (e & 3);
+                        const bool dy = ey && ((krw < 8 - shift) != qy);
+                        const bool dx = ex && ((kcl < 8 - shift) != qx);
+                        if (dy || dx) sa[kt][e] -= 100.f * ATTN_LOG2E;
+                    }
+            }
+            float mx = -INFINITY;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sa[kt][e]);
+            mx = half_max(mx) - 14.0f;  // (probabilities times 2^14)
+            f16acc o;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) o[e] = 0.f;
+            const char *vb = hb + 4 * K::QB + (hh * K::VR + (r & (K::VR - 1))) * 16;
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) {
+                    const h8v vh = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB);
+                    const h8v vl = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB + K::VB / 2);
+                    h4v ph[2], pl[2];
+#pragma unroll
+                    for (int a = 0; a < 2; ++a) {
+                        f4v p;
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) p[b] = __builtin_amdgcn_exp2f(sa[kt][8 * s + 4 * a + b] - mx);
+                        split4(p, ph[a], pl[a]);
+                    }
+                    const h8v p8 = __builtin_shufflevector(ph[0], ph[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    const h8v l8 = __builtin_shufflevector(pl[0], pl[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                    o = MFMA32H(vh, l8, o);
+                    o = MFMA32H(vl, p8, o);
+                    o = MFMA32H(vh, p8, o);
+                }
+            float lo, hi;
+            halves(o[SUM_E], lo, hi);
+            const float inv = exp_unscale(ev) / (SUM_HH ? hi : lo);
+            // O over this wave's own q operands, [32][HD] floats
+            float *orow = reinterpret_cast<float *>(hb + qt * K::QB) + r * HD;
+#pragma unroll
+            for (int e = 0; e < 16; e += 2) {
+                const int dd = 8 * (e >> 2) + 4 * hh + (e & 3);
+                if (dd < HD) *reinterpret_cast<float2 *>(orow + dd) = make_float2(o[e] * inv, o[e + 1] * inv);
+            }
+        }
+        lds_sync();
+        // ---- out: 16 lanes a token, lane c float4 c of its 60 floats ----
+        float4 ov[NST];
+#pragma unroll
+        for (int u = 0; u < NST; ++u) {
+            const int t = min(u * (NT / 16) + (tid >> 4), 63), c4 = min(j, 14);
+            float2 p[2];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int f = 2 * c4 + k, hl = f / (HD / 2), d2 = f - hl * (HD / 2);
+                p[k] = *reinterpret_cast<const float2 *>(buf + hl * K::HB + (t >> 5) * K::QB + ((t & 31) * HD + 2 * d2) * 4);
+            }
+            ov[u] = make_float4(p[0].x, p[0].y, p[1].x, p[1].y);
+        }
+        lds_sync();  // every wave has read the buffer: the next token tile may land
+#pragma unroll
+        for (int u = 0; u < NST; ++u) {
+            const int t = u * (NT / 16) + (tid >> 4);
+            int y = 8 * wh + (t >> 3) + shift;
+            if (y >= g.hp) y -= g.hp;
+            int x = 8 * ww + (t & 7) + shift;
+            if (x >= g.wp) x -= g.wp;
+            buf_store4(ro, t < 64 && j < 15 ? ((y * g.wp + x) * C + hg * 60 + 4 * j) * 4 : BUF_OOB, ov[u]);
+        }
+    }
+}
+
 // ---- host side ------------------------------------------------------------
 
 namespace {
@@ -658,5 +1056,75 @@ hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st) {
     case 2: tok_launch<2>(g, rb, grid, st); break;
     default: tok_launch<3>(g, rb, grid, st); break;
     }
+    return hipGetLastError();
+}
+
+size_t qkv_attn_weight_floats(int hd) { return (size_t)(hd == 30 ? 3 * 4 * 6 : 6 * 2) * 6 * (FRAG / 4); }
+size_t qkv_attn_param_floats(int hd) { return (size_t)(hd == 30 ? 12 : 6) * 96; }
+
+void qkv_attn_pack(const float *wqkv, const float *bqkv, int hd, float *w, float *prm, float *v_l1, float *v_bmax) {
+    const int c = 6 * hd, ks = c > 64 ? 6 : 2, nw = hd == 30 ? 4 : 6, ng = hd == 30 ? 3 : 1;
+    uint16_t *dst = reinterpret_cast<uint16_t *>(w);
+    // the qkv row of column n of tile t of wave wv, group g; -1: padding
+    auto row_of = [&](int g, int wv, int t, int n) {
+        int seg, head, d;
+        if (hd == 30) {
+            seg = t == 2 ? 2 : wv >> 1;
+            head = 2 * g + (t == 2 ? wv >> 1 : wv & 1);
+            d = 16 * (t == 2 ? wv & 1 : t) + n;
+        } else {
+            seg = t;
+            head = wv;
+            d = n;
+        }
+        return d < hd ? seg * c + head * hd + d : -1;
+    };
+    for (int g = 0; g < ng; ++g)
+        for (int wv = 0; wv < nw; ++wv) {
+            float sc[3][16];
+            const float *rows[3][16];
+            for (int t = 0; t < 3; ++t)
+                for (int n = 0; n < 16; ++n) {
+                    const int r = row_of(g, wv, t, n);
+                    rows[t][n] = r < 0 ? nullptr : wqkv + (size_t)r * c;
+                    sc[t][n] = r < 0 ? 1.f : split_row_scale(rows[t][n], c);
+                    float *p = prm + ((size_t)(g * nw + wv) * 3 + t) * 32;
+                    p[n] = 1.f / sc[t][n];
+                    p[16 + n] = r < 0 ? 0.f : bqkv[r];
+                }
+            for (int s = 0; s < ks; ++s)
+                for (int t = 0; t < 3; ++t, dst += FRAG) split_pack_step(rows[t], sc[t], 32 * s, c, dst);
+        }
+    float l1 = 0.f, bm = 0.f;
+    for (int n = 0; n < c; ++n) {
+        double a = 0.0;
+        for (int k = 0; k < c; ++k) a += std::fabs((double)wqkv[(size_t)(2 * c + n) * c + k]);
+        l1 = std::max(l1, (float)a);
+        bm = std::max(bm, std::fabs(bqkv[2 * c + n]));
+    }
+    *v_l1 = l1;
+    *v_bmax = bm;
+}
+
+// Workgroups: whole XCDs' worth of slots (a multiple of 8), at most three per CU
+// (two of the six-wave form), no more than the items.
+unsigned qkv_attention_grid(int hp, int wp, int hd) {
+    const int nw = (hp / 8) * (wp / 8), ng = hd == 30 ? 3 : 1;
+    const int per_xcd = ((nw + 7) / 8) * ng;
+    const int slots = std::max(1, split_cus() * (hd == 30 ? QOCC : 2) / 8);
+    return 8u * (unsigned)std::min(per_xcd, slots);
+}
+
+hipError_t launch_qkv_attention(const QkvAttnArgs &g0, int hd, hipStream_t st) {
+    if (g0.hp <= 0 || g0.wp <= 0 || g0.hp % 8 || g0.wp % 8 || g0.shift < 0 || g0.shift >= 8 || !qkv_attn_fused(6, hd))
+        return hipErrorInvalidValue;
+    QkvAttnArgs g = g0;
+    g.nww = g.wp / 8;
+    g.nw = (g.hp / 8) * g.nww;
+    const dim3 grid(qkv_attention_grid(g.hp, g.wp, hd));
+    if (hd == 30)
+        hipLaunchKernelGGL(k_qkv_attn<30>, grid, dim3(64 * QaCfg<30>::NW), 0, st, g);
+    else
+        hipLaunchKernelGGL(k_qkv_attn<10>, grid, dim3(64 * QaCfg<10>::NW), 0, st, g);
     return hipGetLastError();
 }

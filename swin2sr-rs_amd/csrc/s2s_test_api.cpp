@@ -221,28 +221,21 @@ int s2s_test_block_attention(int hp, int wp, int heads, int head_dim, int shift,
         return fail("hipMalloc failed: out of memory");
     hipError_t e;
     if (qkv_attn_fused(heads, head_dim)) {
-        // the forward's fused kernel, with the weights in its order: each head
-        // pair's q|k|v rows as the unit's columns, each pair's c x c rows in
-        // k_bsgemm's register order
-        std::vector<float> wp_((size_t)3 * c * c), bp_((size_t)3 * c);
-        qkv_pair_weights(wqkv, bqkv, heads, head_dim, wp_.data(), bp_.data());
-        const size_t pf = bs_weight_floats(c, c, EPI_STORE);
-        std::vector<float> wk((size_t)(heads / 2) * pf);
-        for (int pr = 0; pr < heads / 2; ++pr)
-            bs_pack_weights(wp_.data() + (size_t)pr * c * c, c, c, c, EPI_STORE, wk.data() + pr * pf);
-        const float *dwp = d.up(wk.data(), wk.size()), *dbp = d.up(bp_.data(), bp_.size());
-        if (!dwp || !dbp) return fail("hipMalloc failed: out of memory");
+        // the forward's fused kernel, with the weights in its order
         QkvAttnArgs a{};
+        std::vector<float> w(qkv_attn_weight_floats(head_dim)), prm(qkv_attn_param_floats(head_dim));
+        qkv_attn_pack(wqkv, bqkv, head_dim, w.data(), prm.data(), &a.v_l1, &a.v_bmax);
         a.x = dx;
-        a.w = dwp;
-        a.bias = dbp;
+        a.w = d.up(w.data(), w.size());
+        a.prm = d.up(prm.data(), prm.size());
+        if (!a.w || !a.prm) return fail("hipMalloc failed: out of memory");
         a.cpbt = dcp;
         a.logit_scale = dls;
         a.out = dout;
         a.hp = hp;
         a.wp = wp;
         a.shift = shift;
-        e = launch_qkv_attention(a, 0, nullptr);
+        e = launch_qkv_attention(a, head_dim, 0);
     } else {
         GemmArgs g;
         const int epi = qkv_gemm_args(dx, nullptr, db, dq, hp, wp, shift, heads, head_dim, &g);

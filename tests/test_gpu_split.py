@@ -47,3 +47,56 @@ def test_token_half_sizes(pkg, orc, c, heads, ratio, hp, wp):
 @pytest.mark.parametrize("scale", [0.0, 1e-20, 1e-6, 1e6, 1e15])
 def test_token_half_magnitudes(pkg, orc, c, scale):
     assert run_stage(pkg, orc, c, 6, 2, 2, 16, 24, scale) < 1e-4
+
+
+def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift):
+    """qkv projection and window attention in 64 bits, on [hp*wp][c] rows."""
+    c = heads * hd
+    X = x.astype(np.float64).reshape(hp, wp, c)
+    X = np.roll(X, (-shift, -shift), (0, 1))
+    win = lambda t: t.reshape(hp // 8, 8, wp // 8, 8, -1).transpose(0, 2, 1, 3, 4).reshape(-1, 64, t.shape[-1])
+    qkv = win(X) @ w.astype(np.float64).T + b
+    q, k, v = (t.reshape(-1, 64, heads, hd).transpose(0, 2, 1, 3) for t in np.split(qkv, 3, -1))
+    q, k = (t / np.maximum(np.linalg.norm(t, axis=-1, keepdims=True), 1e-12) for t in (q, k))
+    s = q @ k.transpose(0, 1, 3, 2)
+    s = s * np.exp(np.minimum(ls.astype(np.float64), np.log(100.0)))[None, :, None, None]
+    s += cpb.astype(np.float64).reshape(64, 64, heads).transpose(2, 0, 1)
+    if shift:
+        band = lambda n: (np.arange(n) >= n - 8).astype(int) + (np.arange(n) >= n - shift)
+        reg = win((band(hp)[:, None] * 3 + band(wp)[None, :])[..., None])[..., 0]
+        s -= 100.0 * (reg[:, :, None] != reg[:, None, :])[:, None]
+    p = np.exp(s - s.max(-1, keepdims=True))
+    o = (p / p.sum(-1, keepdims=True)) @ v
+    o = o.transpose(0, 2, 1, 3).reshape(hp // 8, wp // 8, 8, 8, c).transpose(0, 2, 1, 3, 4)
+    return np.roll(o.reshape(hp, wp, c), (shift, shift), (0, 1)).reshape(hp * wp, c)
+
+
+# planes of one window, of fewer windows than XCDs, of one window column, and of
+# more items than workgroups at once (256 CUs x 2, a third of it windows). The
+# bar is per window: x of each window scaled by its own power of ten. A logit of
+# 100 x 1.44 in fp32 carries 100 x 1.44 x 6e-8 = 9e-6 into each probability, and
+# a cosine of 30 terms a few roundings more: 5e-5 of the window's largest value.
+@pytest.mark.parametrize("hd", [30, 10])
+@pytest.mark.parametrize("hp,wp", [(8, 8), (8, 40), (72, 8), (120, 136)])
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("spread", [0, 12])
+def test_window_attention(pkg, hd, hp, wp, shift, spread):
+    heads, c = 6, 6 * hd
+    rng = np.random.default_rng(hp * 1000 + wp + hd + shift + spread)
+    x = rng.standard_normal((hp, wp, c))
+    mag = 10.0 ** rng.uniform(-spread, spread, size=(hp // 8, wp // 8))
+    x = np.roll(x, (-shift, -shift), (0, 1)) * np.kron(mag, np.ones((8, 8)))[..., None]
+    x = np.roll(x, (shift, shift), (0, 1)).reshape(hp * wp, c).astype(np.float32)
+    w = (rng.standard_normal((3 * c, c)) * 0.05).astype(np.float32)
+    b = np.zeros(3 * c, np.float32)
+    if not spread:
+        b = rng.uniform(-0.1, 0.1, 3 * c).astype(np.float32)
+        b[c:2 * c] = 0
+    ls = np.linspace(0.0, 5.5, heads).astype(np.float32)
+    cpb = (16 / (1 + np.exp(-rng.standard_normal((4096, heads))))).astype(np.float32)
+    got = pkg.abi.test_block_attention(hp, wp, heads, hd, shift, x, w, b, ls, cpb)
+    want = attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift)
+    win = lambda t: np.roll(t.reshape(hp, wp, c), (-shift, -shift), (0, 1)).reshape(
+        hp // 8, 8, wp // 8, 8, c).transpose(0, 2, 1, 3, 4).reshape(-1, 64 * c)
+    err = np.abs(win(got - want)).max(1) / np.abs(win(want)).max(1)
+    assert err.max() < 5e-5, err.max()
