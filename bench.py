@@ -64,7 +64,6 @@ def kernel_work(arch, h, w, hp=None, wp=None):
     if hp is None:
         hp, wp = (h // win + 1) * win, (w // win + 1) * win
     P = hp * wp
-    VT = 36 * ((hp + 3) // 4) * ((wp + 3) // 4)  # rows of the 36 Winograd GEMMs
     Hd = arch.mlp_ratio * C
     f = 4
     work = {
@@ -81,18 +80,9 @@ def kernel_work(arch, h, w, hp=None, wp=None):
         "fc1_gelu": ("mfma", 2 * P * Hd * C, f * P * (C + Hd)),
         "fc2_ln_res": ("mfma", 2 * P * C * Hd, f * P * (Hd + 2 * C)),
         # the body's 3x3 convs (the stage close with the 1x1 folded in, and
-        # conv_after_body) as Winograd F(4x4,3x3) over T = ceil(hp/4) ceil(wp/4)
-        # tiles: the input transform (the plane in, 36 transform planes of T
-        # tiles out), the 36 transform-position GEMMs (T x C x C multiply-adds
-        # each: 72 T C^2 FLOPs, the direct conv's 18 P C^2 / 4 when 4 divides
-        # the plane; M over V in place), then the output transform + bias +
-        # residual (M and the residual in, the plane out)
-        "conv3x3_stage_in": ("hbm", 0, f * (P * C + VT * C)),
-        "conv3x3_stage": ("mfma", 2 * VT * C * C, f * (2 * VT * C + 36 * C * C)),
-        "conv3x3_stage_out": ("hbm", 0, f * (VT * C + 2 * P * C)),
-        "conv_after_body_in": ("hbm", 0, f * (P * C + VT * C)),
-        "conv_after_body": ("mfma", 2 * VT * C * C, f * (2 * VT * C + 36 * C * C)),
-        "conv_after_body_out": ("hbm", 0, f * (VT * C + 2 * P * C)),
+        # conv_after_body), direct: the plane and the residual in, the plane out
+        "conv3x3_stage": ("split", 2 * P * C * 9 * C, f * 3 * P * C),
+        "conv_after_body": ("split", 2 * P * C * 9 * C, f * 3 * P * C),
         # conv_first and patch_embed (its 1x1 folded into conv_first) + LayerNorm
         # in one pass on fp32 MFMA: two K = 27 convs
         "embed": ("mfma", 2 * 2 * P * C * 27, f * P * (4 + 2 * C)),
@@ -126,14 +116,9 @@ def kernel_work(arch, h, w, hp=None, wp=None):
         # 48 outputs of a 5x5xF footprint per border pixel (VALU)
         nb = -(-h * s // 4) + -(-w * s // 4) - 1
         work["up2_last_edge"] = ("valu", 2 * nb * 48 * 25 * F, f * (nb * 25 * F + 4 * 48 * 25 * F))
-    if C in (60, 120, 180) and F % 4 == 0 and F <= 64:
-        # conv_before_upsample (C -> F, LeakyReLU) as Winograd F(4x4,3x3): the
-        # same input transform, 36 GEMMs of T x F x C, the output transform
-        work["conv_before_upsample_in"] = ("hbm", 0, f * (P * C + VT * C))
-        work["conv_before_upsample"] = ("mfma", 2 * VT * F * C, f * (VT * (C + F) + 36 * F * C))
-        work["conv_before_upsample_out"] = ("hbm", 0, f * (VT * F + P * F))
-    else:
-        work["conv_before_upsample"] = ("mfma", 2 * P * F * 9 * C, f * P * (C + F))
+    # conv_before_upsample (C -> F, LeakyReLU)
+    work["conv_before_upsample"] = ("split" if C <= 192 and F <= 64 else "mfma", 2 * P * F * 9 * C,
+                                    f * P * (C + F))
     px = P
     for o in range(arch.octaves):
         work[f"conv3x3_shuffle2_o{o}"] = ("mfma", 2 * px * 4 * F * 9 * F, f * px * 5 * F)
@@ -147,7 +132,7 @@ def kernel_work(arch, h, w, hp=None, wp=None):
     # at 16P
     work["conv_up1"] = ("mfma", 2 * 4 * P * F * 4 * F, f * (P * F + 4 * P * F))
     work["conv_up2"] = ("mfma", 2 * 16 * P * F * 4 * F, f * (4 * P * F + 16 * P * F))
-    work["conv_hr"] = ("mfma", 2 * 16 * P * F * 9 * F, f * 2 * 16 * P * F)
+    work["conv_hr"] = ("split", 2 * 16 * P * F * 9 * F, f * 2 * 16 * P * F)
     # pixelshuffle_aux: conv_aux F -> 3 on the VALU with the aux image's
     # denormalisation (the plane in, the aux plane and image out),
     # conv_after_aux 3 -> F; the bicubic resample of the padded input to s x

@@ -480,7 +480,7 @@ def test_conv3x3_nearest2(x_hwc, h, w, wgt, bias, slope):
 
 
 def test_conv3x3_winograd(x_hwc, h, w, wgt, bias, epilogue=0, res=None, slope=0.0):
-    """The Winograd F(4x4,3x3) conv path: the body's C -> C convs (c_in ==
+    """The forward's 3x3 convs (k_split_conv): the body's C -> C convs (c_in ==
     c_out in {60, 120, 180}) and conv_before_upsample's C -> F (F <= 64)."""
     lib = load_library()
     cout, cin = wgt.shape[0], wgt.shape[1]

@@ -75,6 +75,7 @@ struct StageW {
     std::vector<BlockW> blocks;
     // the stage close: its 3x3 conv with the 1x1 patch_embed conv folded in
     float *conv_w = nullptr, *conv_b = nullptr;
+    float conv_un = 0.f;  // k_split_conv's unscale of conv_w
 };
 
 struct ProfKey {
@@ -130,7 +131,8 @@ static bool fits_in(const AllocList &l, const std::vector<BufSpec> &v) {
 struct s2s_ctx {
     s2s_arch arch{};
     int c = 0, hd = 0, hidden = 0, feat = 0, octaves = 0;
-    bool cbu_wino = false;  // conv_before_upsample as Winograd (weights U [36][F][C])
+    // the unscales of the convs that run on k_split_conv (0: the implicit GEMM)
+    float cab_un = 0.f, cbu_un = 0.f, hr_un = 0.f;
     int device = 0;
     hipStream_t stream = nullptr;
     AllocList weight_allocs;
@@ -141,9 +143,9 @@ struct s2s_ctx {
     // [2][9][4][C], the folded bias [C], patch_embed's LayerNorm
     float *emb_w = nullptr, *pe_b = nullptr, *pe_nw = nullptr, *pe_nb = nullptr;
     float *norm_w = nullptr, *norm_b = nullptr;
-    float *cab_w = nullptr, *cab_b = nullptr;  // conv_after_body (body_conv_weights)
+    float *cab_w = nullptr, *cab_b = nullptr;  // conv_after_body (conv_weights)
     std::vector<StageW> stages;
-    float *cbu_w = nullptr, *cbu_b = nullptr;  // conv_before_upsample [F][9*C] or [36][F][C]
+    float *cbu_w = nullptr, *cbu_b = nullptr;  // conv_before_upsample (conv_weights)
     std::vector<float *> up_w, up_b;           // octave convs, shuffle-permuted [4F][9*F]
     float *last_w = nullptr, *last_b = nullptr;  // conv_last [9][F][3]
     // pixelshuffle: the last octave's conv and conv_last composed (k_up_last):
@@ -244,24 +246,24 @@ struct s2s_ctx {
     int upload(const std::vector<float> &host, float **dev);
     int alloc(AllocList &list, size_t floats, float **dev, const char *what, bool wide = false,
               bool planned = false);
-    // qkv buffer floats: the plane layout, or the attention unit layout; it
-    // also holds the body's Winograd convs' transform-domain products (36
-    // planes of wino_tiles(hp, wp) tiles x C) between blocks, and the head's
+    // qkv buffer floats: the plane layout or the attention unit layout, and at
+    // least 36 planes of 4x4-pixel tiles x C (the plan's size is part of what
+    // callers budget with); in the x4 head the Winograd 5x5 conv's V and M
+    // (stride F), at most the whole plane's tiles
     size_t qkv_floats(int hp, int wp) const {
         const size_t plane = (size_t)hp * wp * 3 * c;
         const size_t q = qkv_unit_layout(arch.heads, hd, c)
                              ? std::max(plane, attn_unit_floats(hp, wp, arch.heads, hd))
                              : plane;
         const size_t qb = wino_body(c) ? std::max(q, WINO_POS * wino_tiles(hp, wp) * c) : q;
-        // the x4 head's Winograd 5x5 conv: V and M (stride F) at most the
-        // whole plane's tiles
         return up2_wino ? std::max(qb, WINO_POS * wino5_tiles(hp, wp) * feat) : qb;
     }
-    // MLP hidden buffer floats; it also holds conv_before_upsample's Winograd
-    // products (36 planes of wino_tiles(hp, wp) tiles x F) in the head
+    // MLP hidden buffer floats (at least 36 planes of tiles x F with a
+    // conv_before_upsample head, as above)
     size_t hid_floats(int hp, int wp) const {
         const size_t h = (size_t)hp * wp * hidden;
-        return cbu_wino ? std::max(h, WINO_POS * wino_tiles(hp, wp) * feat) : h;
+        const bool head = arch.upsampler != S2S_PIXELSHUFFLE_DIRECT && wino_head(c, feat);
+        return head ? std::max(h, WINO_POS * wino_tiles(hp, wp) * feat) : h;
     }
     // The buffers of a padded plane's body, and of an image's head (with the
     // host path's device copies of the input and output when `io`); `bind`
@@ -305,11 +307,10 @@ struct s2s_ctx {
     int gemm(const char *name, const GemmArgs &g, int aload, int epi);
     int block_fwd(const BlockW &b, int hp, int wp, int shift, const float *x_in, float *x_out);
     int stage_fwd(int s, int hp, int wp, const float *x_in, float *x_out);
-    int conv_body(const char *name, const float *in, int H, int W, const float *u,
+    int conv_body(const char *name, const float *in, int H, int W, const float *w, float un,
                   const float *bias, const float *res, float *out);
-    int conv_wino(const char *name, const float *in, int H, int W, int ci, int co,
-                  const float *u, const float *bias, const float *res, float *mbuf, float *out,
-                  int lrelu, float slope);
+    int split_conv(const char *name, const float *in, int H, int W, int ci, int co, const float *w,
+                   float un, const float *bias, const float *res, float *out, int lrelu, float slope);
     int forward_device(int h, int w, const float *d_in, float *d_out, bool may_graph = true);
     int forward_launches(int h, int w, const float *d_in, float *d_out);
     int head(int h, int w, float *d_out);
@@ -850,65 +851,38 @@ int s2s_ctx::stage_fwd(int s, int hp, int wp, const float *x_in, float *x_out) {
     // The stage close (reference src/gpu.rs:526-528: the 3x3 conv, the 1x1
     // patch_embed conv, the stage's residual) as one conv: the two
     // convolutions are folded into one at upload, and the residual is added
-    // by the output transform element by element, so it may write over x_in
-    // (the transform-domain GEMM has read all of its input before that).
-    return conv_body("conv3x3_stage", src, hp, wp, st.conv_w, st.conv_b, x_in, x_out);
+    // element by element, so it may write over x_in.
+    return conv_body("conv3x3_stage", src, hp, wp, st.conv_w, st.conv_un, st.conv_b, x_in, x_out);
 }
 
 // A C -> C 3x3 conv of the body (the stage close, conv_after_body), + bias +
-// residual. For the released widths (wino_body) as Winograd F(4x4,3x3): the
-// input transform V of every 4x4 output tile into the qkv buffer (free
-// between blocks), the 36 transform-position GEMMs M = V U^T as one batched
-// launch of the weight-stationary kernel (M over V in place), then the output
-// transform with the bias and the residual: 4x fewer multiplies than the
-// direct conv, the same map to fp32 rounding (the reference's own CUDA backend
-// runs these convs as Winograd with 6x6 tiles, src/gpu.rs:161-181). Other
-// widths: the direct implicit-GEMM conv with the residual as its epilogue.
-int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const float *u,
+// residual, on k_split_conv for the widths it takes (un its weights' unscale),
+// else as the implicit-GEMM conv with the residual as its epilogue.
+int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const float *w, float un,
                        const float *bias, const float *res, float *out) {
-    if (!wino_body(c)) {
-        // the epilogue adds the residual element by element; only a conv that
-        // reads the plane it writes (a stage with no blocks) goes through
-        // `o` (free between blocks)
-        float *dst = in == out ? o : out;
-        GemmArgs g = conv_gemm(in, H, W, c, u, bias, dst, c, c);
+    // the residual is added element by element; only a conv that reads the
+    // plane it writes (a stage with no blocks) goes through `o` (free between
+    // blocks)
+    float *dst = in == out ? o : out;
+    if (split_conv_takes(c, c)) {
+        if (split_conv(name, in, H, W, c, c, w, un, bias, res, dst, 0, 0.f)) return -1;
+    } else {
+        GemmArgs g = conv_gemm(in, H, W, c, w, bias, dst, c, c);
         g.res = res;
         g.ldr = c;
         if (gemm(name, g, ALOAD_IM2COL, EPI_RES)) return -1;
-        if (dst != out) {
-            const hipError_t e = hipMemcpyAsync(out, dst, (size_t)H * W * c * 4, hipMemcpyDeviceToDevice, stream);
-            if (e != hipSuccess) return fail(hip_msg("hipMemcpyAsync(stage)", e));
-        }
-        return 0;
     }
-    return conv_wino(name, in, H, W, c, c, u, bias, res, qkv, out, 0, 0.f);
+    if (dst != out) {
+        const hipError_t e = hipMemcpyAsync(out, dst, (size_t)H * W * c * 4, hipMemcpyDeviceToDevice, stream);
+        if (e != hipSuccess) return fail(hip_msg("hipMemcpyAsync(stage)", e));
+    }
+    return 0;
 }
 
-// A 3x3 conv ci -> co as Winograd F(4x4,3x3) on the qkv buffer (free outside
-// the blocks): the input transform of `in` [H*W][ci] into V there, the 36
-// transform-position GEMMs into M at `mbuf` (M over V in place when mbuf is
-// the qkv buffer, which takes co == ci: every GEMM task then writes exactly
-// the rows it has read), then the output transform with the bias, the
-// residual `res` if set and LeakyReLU(slope) if `lrelu`, into out [H*W][co].
-int s2s_ctx::conv_wino(const char *name, const float *in, int H, int W, int ci, int co,
-                       const float *u, const float *bias, const float *res, float *mbuf,
-                       float *out, int lrelu, float slope) {
-    if (mbuf == qkv && co != ci) return fail(std::string(name) + ": in-place Winograd needs co == ci");
-    const int T = (int)wino_tiles(H, W);
-    const std::string in_name = std::string(name) + "_in", out_name = std::string(name) + "_out";
-    if (run(in_name.c_str(), dim3(wino_in_grid(H, W, ci)), dim3(256),
-            [&] { return launch_wino_in(in, ci, qkv, H, W, ci, stream); }))
-        return -1;
-    GemmArgs g = rows_gemm(qkv, ci, u, ci, nullptr, mbuf, co, T, co, ci);
-    g.nb = WINO_POS;
-    g.a_bstride = (size_t)T * ci;
-    g.o_bstride = (size_t)T * co;
-    g.b_packed = bs_packs(co, ci, EPI_STORE);
-    g.b_bstride = weight_floats(co, ci, EPI_STORE);
-    if (gemm(name, g, ALOAD_ROWS, EPI_STORE)) return -1;
-    return run(out_name.c_str(), dim3(wino_out_grid(H, W, co)), dim3(256), [&] {
-        return launch_wino_out(mbuf, bias, res, res ? co : 0, out, co, H, W, co, lrelu, slope, stream);
-    });
+int s2s_ctx::split_conv(const char *name, const float *in, int H, int W, int ci, int co, const float *w,
+                        float un, const float *bias, const float *res, float *out, int lrelu, float slope) {
+    const SplitConvArgs g{in, w, un, bias, res, out, H, W, ci, co, lrelu, slope};
+    return run(name, dim3(split_conv_grid(H, W, ci, co)), dim3(256), [&] { return launch_split_conv(g, stream); });
 }
 
 int s2s_ctx::forward_device(int h, int w, const float *d_in, float *d_out, bool may_graph) {
@@ -1011,7 +985,7 @@ int s2s_ctx::forward_launches(int h, int w, const float *d_in, float *d_out) {
             [&] { return launch_layernorm(cur, norm_w, norm_b, nullptr, o, P, c, stream); }))
         return -1;
     // (the final norm lands in the attention output's plane, free after the blocks)
-    if (conv_body("conv_after_body", o, hp, wp, cab_w, cab_b, body, cur)) return -1;
+    if (conv_body("conv_after_body", o, hp, wp, cab_w, cab_un, cab_b, body, cur)) return -1;
     return head(h, w, d_out);
 }
 
@@ -1024,9 +998,9 @@ int s2s_ctx::head(int h, int w, float *d_out) {
     GemmArgs g{};
     // conv_before_upsample + LeakyReLU(0.01) into the first feature plane
     auto before_upsample = [&]() -> int {
-        if (cbu_wino)
-            return conv_wino("conv_before_upsample", cur, hp, wp, c, feat, cbu_w, cbu_b, nullptr,
-                             hid, fplanes[0], 1, 0.01f);
+        if (split_conv_takes(c, feat))
+            return split_conv("conv_before_upsample", cur, hp, wp, c, feat, cbu_w, cbu_un, cbu_b, nullptr,
+                              fplanes[0], 1, 0.01f);
         g = conv_gemm(cur, hp, wp, c, cbu_w, cbu_b, fplanes[0], feat, feat);
         g.slope = 0.01f;
         return gemm("conv_before_upsample", g, ALOAD_IM2COL, EPI_LRELU);
@@ -1161,9 +1135,15 @@ int s2s_ctx::head(int h, int w, float *d_out) {
         g = sub2_gemm(fplanes[1], 2 * hp, 2 * wp, feat, nu2_w, nu2_b, fplanes[2]);
         g.slope = 0.2f;
         if (gemm("conv_up2", g, ALOAD_SUB2, EPI_LRELU)) return -1;
-        g = conv_gemm(fplanes[2], 4 * hp, 4 * wp, feat, hr_w, hr_b, fplanes[3], feat, feat);
-        g.slope = 0.2f;
-        if (gemm("conv_hr", g, ALOAD_IM2COL, EPI_LRELU)) return -1;
+        if (split_conv_takes(feat, feat)) {
+            if (split_conv("conv_hr", fplanes[2], 4 * hp, 4 * wp, feat, feat, hr_w, hr_un, hr_b, nullptr,
+                           fplanes[3], 1, 0.2f))
+                return -1;
+        } else {
+            g = conv_gemm(fplanes[2], 4 * hp, 4 * wp, feat, hr_w, hr_b, fplanes[3], feat, feat);
+            g.slope = 0.2f;
+            if (gemm("conv_hr", g, ALOAD_IM2COL, EPI_LRELU)) return -1;
+        }
         return last(fplanes[3], 4 * hp, 4 * wp);
     }
     default:
@@ -1225,14 +1205,17 @@ std::vector<float> conv_relayout(const float *w, int co, int ci, const std::vect
     return out;
 }
 
-// A body C -> C conv's weights [co][ci][3][3] as its kernels read them: the
-// Winograd transform [36][C][C] for the released widths (in the batched
-// GEMM's order), else the implicit GEMM's [co][tap][ci_pad4].
-std::vector<float> body_conv_weights(const float *w, int C) {
-    if (!wino_body(C)) return conv_relayout(w, C, C, nullptr);
-    std::vector<float> u((size_t)WINO_POS * C * C);
-    wino_weights(w, C, C, u.data());
-    return gemm_weights(u, WINO_POS, C, C, EPI_STORE);
+// A 3x3 conv's weights [co][ci][3][3] as its kernel reads them: k_split_conv's
+// packing (*un its unscale) for the shapes it takes, else the implicit GEMM's
+// [co][tap][ci_pad4].
+std::vector<float> conv_weights(const float *w, int co, int ci, float *un) {
+    if (!split_conv_takes(ci, co)) return conv_relayout(w, co, ci, nullptr);
+    std::vector<float> p(split_conv_weight_floats(ci, co));
+    *un = split_conv_pack(w, ci, co, p.data());
+    return p;
+}
+uint64_t conv_weight_floats(int co, int ci) {
+    return split_conv_takes(ci, co) ? split_conv_weight_floats(ci, co) : (uint64_t)co * 9 * round4(ci);
 }
 
 // co = 4ch + 2dy + dx  ->  row (2dy+dx)*feat + ch, so a 32-column tile of the
@@ -1434,9 +1417,7 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
     f += C;                     // conv_first's bias (the body skip)
     f += 2 * 9 * 4 * C + C;     // k_embed's two weight sets, the folded bias
     f += 4 * C;                 // patch_embed's LayerNorm, the final LayerNorm
-    // the body's C -> C convs: Winograd weights [36][C][C] (in the batched
-    // GEMM's register order) or direct [C][9][C4]
-    const uint64_t body_conv = wino_body(A.embed) ? WINO_POS * weight_floats(C, C, EPI_STORE) : C * 9 * C4;
+    const uint64_t body_conv = conv_weight_floats(A.embed, A.embed);  // the body's C -> C convs
     f += body_conv + C;         // conv_after_body
     for (int s = 0; s < A.n_stages; ++s) {
         f += body_conv + C;     // the stage close (3x3 with the 1x1 folded in)
@@ -1464,11 +1445,10 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
         int F = 0;
         if (head_feat_of(ts, A.embed, &F)) return -1;
         const uint64_t F_ = F, F4 = round4(F);
-        // conv_before_upsample: Winograd weights [36][F][C4] or direct [F][9][C4]
-        f += (wino_head(A.embed, F) ? WINO_POS * weight_floats(F, C4, EPI_STORE) : F_ * 9 * C4) + F_;
+        f += conv_weight_floats(F, A.embed) + F_;  // conv_before_upsample
         f += 9 * F_ * 3 + 3;            // conv_last
         if (up == S2S_NEAREST_CONV) {
-            f += 2 * (4 * F_ * 4 * F4 + F_) + (F_ * 9 * F4 + F_);  // conv_up1, conv_up2 (by phase), conv_hr
+            f += 2 * (4 * F_ * 4 * F4 + F_) + (conv_weight_floats(F, F) + F_);  // conv_up1, conv_up2 (by phase), conv_hr
         } else {
             const int oct = octaves_of(A.scale);
             f += (uint64_t)oct * (4 * F_ * 9 * F4 + 4 * F_);  // the octave convs
@@ -1568,15 +1548,12 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
         subpixel_weights(x->data, F, F, w.data());
         return ctx->upload(w, dst);
     };
-    // conv_before_upsample [F][C][3][3]: the Winograd transform [36][F][C]
-    // when wino_head takes it, else the implicit GEMM's layout
+    auto up_conv = [&](const std::string &name, int co, int ci, float **dst, float *un) -> int {
+        if (ts.get(name, {co, ci, 3, 3}, &x)) return -1;
+        return ctx->upload(conv_weights(x->data, co, ci, un), dst);
+    };
     auto up_before_upsample = [&](int F) -> int {
-        ctx->cbu_wino = wino_head(C, F);
-        if (!ctx->cbu_wino) return upconv("conv_before_upsample.0.weight", F, C, &ctx->cbu_w, nullptr);
-        if (ts.get("conv_before_upsample.0.weight", {F, C, 3, 3}, &x)) return -1;
-        std::vector<float> u((size_t)WINO_POS * F * round4(C));
-        wino_weights(x->data, F, C, u.data());
-        return ctx->upload(gemm_weights(u, WINO_POS, F, round4(C), EPI_STORE), &ctx->cbu_w);
+        return up_conv("conv_before_upsample.0.weight", F, C, &ctx->cbu_w, &ctx->cbu_un);
     };
 
     rc = rc || up("conv_first.bias", {C}, &ctx->cf_b);
@@ -1622,7 +1599,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
     {
         const s2s_tensor *cw;
         rc = rc || ts.get("conv_after_body.weight", {C, C, 3, 3}, &cw);
-        if (!rc) rc = ctx->upload(body_conv_weights(cw->data, C), &ctx->cab_w);
+        if (!rc) rc = ctx->upload(conv_weights(cw->data, C, C, &ctx->cab_un), &ctx->cab_w);
     }
     rc = rc || up("conv_after_body.bias", {C}, &ctx->cab_b);
 
@@ -1664,7 +1641,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
                 for (size_t k = 0; k < kk; ++k) wf[(size_t)o * kk + k] = (float)acc[k];
                 bf[o] = (float)ab;
             }
-            rc = rc || ctx->upload(body_conv_weights(wf.data(), C), &st.conv_w);
+            rc = rc || ctx->upload(conv_weights(wf.data(), C, C, &st.conv_un), &st.conv_w);
             rc = rc || ctx->upload(bf, &st.conv_b);
         }
         st.blocks.resize(A.depths[s]);
@@ -1901,7 +1878,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
             rc = rc || up("conv_up1.bias", {F}, &ctx->nu1_b);
             rc = rc || up_sub2("conv_up2.weight", F, &ctx->nu2_w);
             rc = rc || up("conv_up2.bias", {F}, &ctx->nu2_b);
-            rc = rc || upconv("conv_hr.weight", F, F, &ctx->hr_w, nullptr);
+            rc = rc || up_conv("conv_hr.weight", F, F, &ctx->hr_w, &ctx->hr_un);
             rc = rc || up("conv_hr.bias", {F}, &ctx->hr_b);
             rc = rc || conv_last(F);
         }

@@ -241,6 +241,26 @@ hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st);
 float split_row_scale(const float *w, int n);
 void split_pack_step(const float *const *rows, const float *scale, int k0, int kn, uint16_t *dst);
 
+// A 3x3 stride-1 zero-pad-1 conv of the channel-last H x W plane `in` [H*W][cin]
+// into out [H*W][cout] (k_split_conv, s2s_split.hip): + bias (or null), + res
+// [H*W][cout] (or null; may be out), then LeakyReLU(slope) if lrelu. w and
+// unscale from split_conv_pack of the [cout][cin][3][3] weights.
+struct SplitConvArgs {
+    const float *in;
+    const float *w;
+    float unscale;
+    const float *bias, *res;
+    float *out;
+    int H, W, cin, cout;
+    int lrelu;
+    float slope;
+};
+bool split_conv_takes(int cin, int cout);
+size_t split_conv_weight_floats(int cin, int cout);
+float split_conv_pack(const float *w, int cin, int cout, float *out);
+unsigned split_conv_grid(int H, int W, int cin, int cout);
+hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st);
+
 #define GEMM_NVARIANTS 6
 hipError_t launch_gemm(const GemmArgs &g, int aload, int epi, hipStream_t st);
 hipError_t launch_gemm_variant(const GemmArgs &g, int aload, int epi, int variant,
@@ -253,16 +273,9 @@ const char *gemm_kernel_name(const GemmArgs &g, int aload, int epi);
 // profiler's rows), and the kernel family name it picks.
 void gemm_geometry(const GemmArgs &g, int aload, int epi, dim3 *grid, dim3 *block);
 hipError_t launch_attention(const AttnArgs &g, hipStream_t st, unsigned *grid_out);
-// Winograd F(4x4,3x3) for a 3x3 stride-1 zero-pad-1 conv on a channel-last
-// H x W plane (C % 4 == 0): wino_weights transforms the [co][ci][3][3]
-// weights to U = G g G^T, the GEMM's B [36][co][round4(ci)] (double
-// accumulation, rounded once); launch_wino_in writes V = B^T d B of every 4x4
-// output tile's 6x6 input patch (zero outside the plane) as [36][T][C] for the
-// T = wino_tiles(H, W) tiles; a batch of 36 row GEMMs M[b] = V[b] U[b]^T (over
-// M's own buffer); launch_wino_out transforms M back (Y = A^T M A), adds the
-// bias, then the residual `res` [H*W][ldr] if set, then LeakyReLU(slope) if
-// `lrelu`, into out [H*W][ldo] (the tiles' pixels inside the plane).
 constexpr int WINO_POS = 36;
+// 4x4-pixel tiles of a plane (the plan's qkv and MLP buffers hold at least 36 of
+// their planes)
 inline size_t wino_tiles(int H, int W) { return (size_t)((H + 3) / 4) * ((W + 3) / 4); }
 // Winograd F(2x2,5x5) for the x4 head's composed 5x5 conv (F = 64 -> 48, the
 // pixel_shuffle(4) finish): the same six points and B^T; the 2x2 output
@@ -282,21 +295,10 @@ hipError_t launch_wino5_finish(const float *m, int ldm, const float *bias, float
                                int Wo, int oh, int ow, float img_range, const float *mean,
                                hipStream_t st);
 unsigned wino5_finish_grid(int Ho, int Wo);
-void wino_weights(const float *w, int co, int ci, float *out);
-// The body's C -> C convs take the Winograd path when the batched GEMM runs on
-// the weight-stationary kernel with every column in one workgroup (so it may
-// write M over V in place): C in {60, 120, 180}, every released width.
+// The released body widths, and their conv_before_upsample: what
+// s2s_test_conv3x3_winograd takes and the plan's minimum sizes are stated for.
 inline bool wino_body(int c) { return c == 60 || c == 120 || c == 180; }
-// conv_before_upsample (C -> F, then LeakyReLU) takes the Winograd path when C
-// is a body width above and F fits one narrow (64-column) group of the
-// weight-stationary kernel; its products go to a buffer of their own.
 inline bool wino_head(int c, int f) { return wino_body(c) && f % 4 == 0 && f <= 64; }
-hipError_t launch_wino_in(const float *in, int ldi, float *v, int H, int W, int C, hipStream_t st);
-unsigned wino_in_grid(int H, int W, int C);   // the launches' 1-D grids of 256 threads
-unsigned wino_out_grid(int H, int W, int C);
-hipError_t launch_wino_out(const float *m, const float *bias, const float *res, int ldr,
-                           float *out, int ldo, int H, int W, int C, int lrelu, float slope,
-                           hipStream_t st);
 unsigned attention_grid(const AttnArgs &g);
 hipError_t launch_pad_input(const float *in, float *out, int h, int w, int hp, int wp,
                             hipStream_t st);

@@ -10,16 +10,15 @@
 //
 // Dense contractions run on fp32 MFMA (fp32 in, fp32 accumulate):
 //   - (s2s_split.hip: the released widths' Swin blocks, on the f16 matrix cores
-//     by operand splitting: k_qkv_attn and k_token_mlp)
+//     by operand splitting: k_qkv_attn, k_token_mlp, and their 3x3 convs,
+//     k_split_conv)
 //   - k_bsgemm: the token GEMMs of other widths and head shapes, weights stationary in registers, with the elementwise work
 //     fused into the epilogue: bias, erf-GELU, residual, LeakyReLU, LayerNorm
 //     (+ residual) over the full row, and the qkv store in the attention's
 //     unit layout; batched, the transform-domain products of the Winograd
 //     convolutions;
-//   - k_wino_in / k_wino_out: the Winograd F(4x4,3x3) input and output
-//     transforms of the body's 3x3 convolutions (bias, residual or LeakyReLU
-//     in the output pass), and, with k_wino5_finish, the F(2x2,5x5) form of the
-//     x4 head's composed last stage;
+//   - k_wino_in / k_wino5_finish: the Winograd F(2x2,5x5) form of the x4 head's
+//     composed last stage;
 //   - k_gemm: 3x3 convolutions as implicit GEMMs (im2col done by the operand
 //     loader) for the widths the Winograd path does not take, with the same
 //     epilogues and the pixel-shuffle store of the head's octaves;
@@ -2930,25 +2929,20 @@ hipError_t launch_cpb(const float *w0, const float *b0, const float *w2, float *
     return hipGetLastError();
 }
 
-// Winograd F(4x4,3x3): a 4x4 output tile from its 6x6 input patch with 36
-// products per (input, output) channel pair instead of 144. The transforms
-// come from the Toom-Cook construction with the interpolation points
-// 0, 3/2, -3/2, 2/3, -2/3 and infinity (on unit-normal data at C = 180 their
-// fp32 error is about a third of that of the points 0, +-1, +-2):
-//   B^T = [1    0    -97/36  0      1  0]    G = [1       0       0    ]
-//         [0  -2/3   -4/9    3/2    1  0]        [8/65    12/65   18/65]
-//         [0   2/3   -4/9   -3/2    1  0]        [8/65   -12/65   18/65]
-//         [0  -3/2   -9/4    2/3    1  0]        [-81/130 -27/65 -18/65]
-//         [0   3/2   -9/4   -2/3    1  0]        [-81/130  27/65 -18/65]
-//         [0    1     0    -97/36   0  1]        [0       0       1    ]
-//   A^T = [1   1     1     1     1    0]
-//         [0  3/2  -3/2   2/3  -2/3   0]
-//         [0  9/4   9/4   4/9   4/9   0]
-//         [0 27/8 -27/8  8/27 -8/27   1]
-// so that, for the cross-correlation the conv layers compute (tap (a, b) of
-// output pixel (y, x) reads input (y + a - 1, x + b - 1)),
-// Y = A^T [ (G g G^T) .* (B^T d B) ] A per tile and channel pair, summed over
-// the input channels by the transform-domain GEMM.
+// Winograd F(2x2,5x5), for the x4 head's composed 5x5 conv: a 2x2 output tile
+// from its 6x6 input patch with 36 products per (input, output) channel pair
+// instead of 100. The transforms come from the Toom-Cook construction with the
+// interpolation points 0, 3/2, -3/2, 2/3, -2/3 and infinity (their fp32 error on
+// unit-normal data is about a third of that of the points 0, +-1, +-2):
+//   B^T = [1    0    -97/36  0      1  0]
+//         [0  -2/3   -4/9    3/2    1  0]
+//         [0   2/3   -4/9   -3/2    1  0]
+//         [0  -3/2   -9/4    2/3    1  0]
+//         [0   3/2   -9/4   -2/3    1  0]
+//         [0    1     0    -97/36   0  1]
+// (G5 at wino5_weights, A^T at k_wino5_finish). For the cross-correlation that
+// the conv layers compute, Y = A^T [ (G g G^T) .* (B^T d B) ] A per tile and
+// channel pair, summed over the input channels by the transform-domain GEMM.
 
 // B^T applied to the 6 values x[0], x[S], ..., x[5S], in place (14 VALU).
 template <int S> __device__ __forceinline__ void wino4_bt(float *x) {
@@ -2962,16 +2956,6 @@ template <int S> __device__ __forceinline__ void wino4_bt(float *x) {
     x[4 * S] = e2 - o2;
     x[5 * S] = fmaf(-97.f / 36.f, d3, d1 + d5);
 }
-// A^T applied to m[0], m[S], ..., m[5S], into y[0], y[T], y[2T], y[3T].
-template <int S, int T> __device__ __forceinline__ void wino4_at(const float *m, float *y) {
-    const float s12 = m[S] + m[2 * S], d12 = m[S] - m[2 * S];
-    const float s34 = m[3 * S] + m[4 * S], d34 = m[3 * S] - m[4 * S];
-    y[0] = m[0] + s12 + s34;
-    y[T] = fmaf(1.5f, d12, (2.f / 3.f) * d34);
-    y[2 * T] = fmaf(2.25f, s12, (4.f / 9.f) * s34);
-    y[3 * T] = fmaf(3.375f, d12, fmaf(8.f / 27.f, d34, m[5 * S]));
-}
-
 // NE consecutive floats (4: a float4, 2: a float2) at p.
 template <int NE> __device__ __forceinline__ void ld_vec(const float *p, float *v) {
     if constexpr (NE == 4) {
@@ -2993,20 +2977,16 @@ template <int NE> __device__ __forceinline__ void st_vec(float *p, const float *
         *reinterpret_cast<float2 *>(p) = make_float2(v[0], v[1]);
 }
 
-// channels per thread of the two transforms
+// channels per thread of the input transform
 #ifndef WINO_IN_NE
 #define WINO_IN_NE 4
-#endif
-#ifndef WINO_OUT_NE
-#define WINO_OUT_NE 2
 #endif
 
 // Input transform: tile (ty, tx) of the grid of MT x MT output tiles that
 // covers Ho x Wo (rounded up), channels c .. c+NE-1: its 6x6 patch d (rows
 // MT ty - PAD .. MT ty - PAD + 5, the same for columns, zero outside the H x W
-// plane) to V = B^T d B, stored as V[6 xi + nu][tile][c]. F(4x4,3x3) takes
-// MT = 4, PAD = 1; F(2x2,5x5) MT = 2, PAD = 2 - the same B^T for the same six
-// points. One thread per (tile, NE channels); consecutive threads read and
+// plane) to V = B^T d B, stored as V[6 xi + nu][tile][c]. F(2x2,5x5) takes
+// MT = 2, PAD = 2. One thread per (tile, NE channels); consecutive threads read and
 // write consecutive channel groups.
 template <int NE, int MT, int PAD>
 __global__ __launch_bounds__(256) void k_wino_in(const float *__restrict__ in, int ldi,
@@ -3055,20 +3035,6 @@ __global__ __launch_bounds__(256) void k_wino_in(const float *__restrict__ in, i
     }
 }
 
-unsigned wino_in_grid(int H, int W, int C) {
-    // (a multiple of 8 workgroups: k_wino_in's XCD-aware order)
-    return (unsigned)(((long long)wino_tiles(H, W) * (C / WINO_IN_NE) + 2047) / 2048 * 8);
-}
-
-hipError_t launch_wino_in(const float *in, int ldi, float *v, int H, int W, int C, hipStream_t st) {
-    if (H < 1 || W < 1 || C % 4 || ldi % 4) return hipErrorInvalidValue;
-    const int tw = (W + 3) / 4;
-    const int T = (int)wino_tiles(H, W);
-    hipLaunchKernelGGL((k_wino_in<WINO_IN_NE, 4, 1>), dim3(wino_in_grid(H, W, C)), dim3(256), 0, st,
-                       in, ldi, v, H, W, C, T, tw);
-    return hipGetLastError();
-}
-
 unsigned wino5_in_grid(int Ho, int Wo, int C) {
     return (unsigned)(((long long)wino5_tiles(Ho, Wo) * (C / WINO_IN_NE) + 255) / 256);
 }
@@ -3080,84 +3046,6 @@ hipError_t launch_wino5_in(const float *in, int ldi, float *v, int H, int W, int
     const int T = (int)wino5_tiles(Ho, Wo);
     hipLaunchKernelGGL((k_wino_in<WINO_IN_NE, 2, 2>), dim3(wino5_in_grid(Ho, Wo, C)), dim3(256), 0,
                        st, in, ldi, v, H, W, C, T, tw);
-    return hipGetLastError();
-}
-
-// Output transform: tile (ty, tx), channels c .. c+NE-1: M[6 xi + nu][tile][c]
-// to Y = A^T M A, + bias, + the residual, then LeakyReLU when asked, into the
-// tile's 4x4 output pixels that lie inside the plane. One thread per (tile,
-// NE channels); M's 36 planes are read with consecutive threads on
-// consecutive channel groups.
-template <int NE>
-__global__ __launch_bounds__(256) void k_wino_out(const float *__restrict__ m,
-                                                   const float *__restrict__ bias,
-                                                   const float *__restrict__ res, int ldr,
-                                                   float *__restrict__ out, int ldo, int H, int W,
-                                                   int C, int T, int tw, int lrelu, float slope) {
-    const int cgn = C / NE;
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)T * cgn) return;
-    const int tile = (int)(i / cgn);
-    const int c = NE * (int)(i - (long long)tile * cgn);
-    const size_t plane = (size_t)T * C;
-    const float *src = m + (size_t)tile * C + c;
-    float t[6][4][NE];  // [xi][output column][channel]: M A, row by row
-#pragma unroll
-    for (int xi = 0; xi < 6; ++xi) {
-        float mr[6][NE];
-#pragma unroll
-        for (int nu = 0; nu < 6; ++nu) ld_vec<NE>(src + (6 * xi + nu) * plane, mr[nu]);
-#pragma unroll
-        for (int e = 0; e < NE; ++e) wino4_at<NE, NE>(&mr[0][e], &t[xi][0][e]);
-    }
-    float y[4][4][NE];  // [output row][output column][channel]
-#pragma unroll
-    for (int cx = 0; cx < 4; ++cx)
-#pragma unroll
-        for (int e = 0; e < NE; ++e) wino4_at<4 * NE, 4 * NE>(&t[0][cx][e], &y[0][cx][e]);
-    float bv[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) bv[e] = 0.f;
-    if (bias) ld_vec<NE>(bias + c, bv);
-    const int ty = tile / tw, tx = tile - (tile / tw) * tw;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int oy = 4 * ty + r;
-        if (oy >= H) break;
-#pragma unroll
-        for (int cx = 0; cx < 4; ++cx) {
-            const int ox = 4 * tx + cx;
-            if (ox >= W) break;
-            const size_t px = (size_t)oy * W + ox;
-            float v[NE], rv[NE];
-#pragma unroll
-            for (int e = 0; e < NE; ++e) v[e] = y[r][cx][e] + bv[e];
-            if (res) {
-                ld_vec<NE>(res + px * ldr + c, rv);
-#pragma unroll
-                for (int e = 0; e < NE; ++e) v[e] += rv[e];
-            }
-            if (lrelu) {
-#pragma unroll
-                for (int e = 0; e < NE; ++e) v[e] = v[e] < 0.f ? v[e] * slope : v[e];
-            }
-            st_vec<NE>(out + px * ldo + c, v);
-        }
-    }
-}
-
-unsigned wino_out_grid(int H, int W, int C) {
-    return (unsigned)(((long long)wino_tiles(H, W) * (C / WINO_OUT_NE) + 255) / 256);
-}
-
-hipError_t launch_wino_out(const float *m, const float *bias, const float *res, int ldr,
-                           float *out, int ldo, int H, int W, int C, int lrelu, float slope,
-                           hipStream_t st) {
-    if (H < 1 || W < 1 || C % 4 || ldo % 4 || (res && ldr % 4)) return hipErrorInvalidValue;
-    const int tw = (W + 3) / 4;
-    const int T = (int)wino_tiles(H, W);
-    hipLaunchKernelGGL(k_wino_out<WINO_OUT_NE>, dim3(wino_out_grid(H, W, C)), dim3(256), 0, st, m,
-                       bias, res, ldr, out, ldo, H, W, C, T, tw, lrelu, slope);
     return hipGetLastError();
 }
 
@@ -3267,30 +3155,6 @@ void wino5_weights(const double *w, int co, int ci, float *out) {
                             u += G[xi][a] * w[((size_t)o * 25 + 5 * a + b) * ci + i] * G[nu][b];
                     out[((size_t)(6 * xi + nu) * co + o) * cp + i] = (float)u;
                 }
-}
-
-// U = G g G^T per (co, ci) with G above, accumulated in double and rounded
-// once, as the GEMM's B: [36][co][round4(ci)] with batch b = 6 xi + nu.
-void wino_weights(const float *w, int co, int ci, float *out) {
-    static const double G[6][3] = {{1, 0, 0},
-                                   {8.0 / 65, 12.0 / 65, 18.0 / 65},
-                                   {8.0 / 65, -12.0 / 65, 18.0 / 65},
-                                   {-81.0 / 130, -27.0 / 65, -18.0 / 65},
-                                   {-81.0 / 130, 27.0 / 65, -18.0 / 65},
-                                   {0, 0, 1}};
-    const int cp = (ci + 3) / 4 * 4;
-    for (size_t i = 0; i < (size_t)WINO_POS * co * cp; ++i) out[i] = 0.f;
-    for (int o = 0; o < co; ++o)
-        for (int i = 0; i < ci; ++i) {
-            const float *g = w + ((size_t)o * ci + i) * 9;
-            for (int xi = 0; xi < 6; ++xi)
-                for (int nu = 0; nu < 6; ++nu) {
-                    double u = 0.0;
-                    for (int a = 0; a < 3; ++a)
-                        for (int b = 0; b < 3; ++b) u += G[xi][a] * (double)g[3 * a + b] * G[nu][b];
-                    out[((size_t)(6 * xi + nu) * co + o) * cp + i] = (float)u;
-                }
-        }
 }
 
 // A 3x3 conv (w [co][ci][3][3]) of the nearest-2x upsampling of a plane, as

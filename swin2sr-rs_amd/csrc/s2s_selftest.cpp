@@ -178,7 +178,7 @@ extern "C" int s2s_selftest(const s2s_arch *arch, const s2s_tensor *tensors, siz
         }
     }
 
-    // the body's Winograd F(4x4,3x3) conv (the stage close, conv_after_body)
+    // the body's 3x3 conv as the forward runs it (the stage close, conv_after_body)
     // at the released widths and the checkpoint's own: a plane that is all
     // border, planes whose sides are not multiples of the 4x4 tile, planes
     // wider than one 64-lane wavefront
@@ -194,13 +194,13 @@ extern "C" int s2s_selftest(const s2s_arch *arch, const s2s_tensor *tensors, siz
                                             0.f, got.data()));
             std::vector<double> want = conv3x3(x, h, w, c, c, wgt, b);
             for (size_t i = 0; i < want.size(); ++i) want[i] += res[i];
-            CHECK(cnt.ok(close("winograd conv3x3 " + std::to_string(c) + "->" + std::to_string(c) +
+            CHECK(cnt.ok(close("body conv3x3 " + std::to_string(c) + "->" + std::to_string(c) +
                                    " + residual at " + std::to_string(h) + "x" + std::to_string(w),
                                want, got, tol)));
         }
     }
 
-    // conv_before_upsample's Winograd conv (C -> F, then LeakyReLU) at the
+    // conv_before_upsample as the forward runs it (C -> F, then LeakyReLU) at the
     // checkpoint's width and a head of 64 features, on a plane ending in
     // partial tiles
     if (wino_head(arch->embed, 64)) {
@@ -212,7 +212,7 @@ extern "C" int s2s_selftest(const s2s_arch *arch, const s2s_tensor *tensors, siz
                                         got.data()));
         std::vector<double> want = conv3x3(x, h, w, c, f, wgt, b);
         for (double &v : want) v = v < 0 ? v * 0.01 : v;
-        CHECK(cnt.ok(close("winograd conv3x3 " + std::to_string(c) + "->64 + LeakyReLU at 11x13",
+        CHECK(cnt.ok(close("body conv3x3 " + std::to_string(c) + "->64 + LeakyReLU at 11x13",
                            want, got, tol)));
     }
 

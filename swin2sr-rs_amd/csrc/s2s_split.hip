@@ -873,6 +873,206 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, QOCC) void k_
     }
 }
 
+// ---------------------------------------------------------------------------
+// k_split_conv: 3x3 stride-1 zero-pad-1 convolution of a channel-last plane, cin
+// and cout at most 192, as one implicit GEMM on the split: + bias, then the
+// residual or LeakyReLU.
+//
+// A workgroup makes a tile of 8 pixels by 2 RBT rows, RBT = RB 4 / WC row blocks
+// of 2 x 8 pixels: WC waves side by side in the output columns (16 TN each), 4 /
+// WC groups of waves below one another, RB row blocks each. The tile's halo is
+// loaded a tile ahead, scaled by its largest magnitude (one scale: a sum runs
+// over the pixels of a footprint), split and kept in LDS as [k step][part][q]
+// [pixel], so that a tap is an offset; the nine taps' weights stream from L2
+// through a register ring as in k_token_mlp. The pixel slots are permuted within
+// 8 by q and the parity of the k step, for the writes' banks (frag_slot).
+//
+// Tiles go to workgroups in plane order within each XCD, so that halos are shared
+// in its L2. MI355X: 264 x 264 x 180 in 133 us, where F(4x4,3x3) Winograd (a
+// quarter of the multiply-adds, in fp32, and 560 MB of transform planes) took 176;
+// 40 x 72 x 180 20.8 (31.7); 544 x 968 x 60 160 (338); 64 -> 64 at 1952 x 2592 1.26
+// ms where the fp32 implicit GEMM took 3.1. 81 us of the first are MFMA issue at
+// the clock the kernel runs at. One workgroup per CU with six row blocks per wave
+// and operands read ahead: 138 us.
+// ---------------------------------------------------------------------------
+namespace {
+
+template <int KSC, int TN, int RB, int WC> struct ConvCfg {
+    static constexpr int RBT = RB * 4 / WC;
+    static constexpr int TH = 2 * RBT;                    // tile rows
+    static constexpr int NPIX = (TH + 2) * 10;            // halo pixels
+    static constexpr int NP = (NPIX + 7) / 8 * 8;
+    static constexpr int F = 8 * KSC;                     // float4s of a pixel
+    static constexpr int NL = (NPIX * F + 255) / 256;     // loads per thread
+    static constexpr int STEP = 4 * NP * 16;              // bytes of a k step's part
+};
+
+}  // namespace
+
+template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) void k_split_conv(SplitConvArgs g) {
+    using K = ConvCfg<KSC, TN, RB, WC>;
+    __shared__ __attribute__((aligned(16))) char buf[2 * KSC * K::STEP];
+    __shared__ float wmx[4];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 15, q = lane >> 4;
+    const int cw = wave % WC, rw = wave / WC;
+    const __amdgpu_buffer_rsrc_t rw_ = buf_rsrc(g.w, (size_t)WC * 9 * KSC * TN * 2 * FRAG);
+    const int wbase = cw * 9 * KSC * TN * 2 * FRAG;
+    const int tx = (g.W + 7) / 8, ty = (g.H + K::TH - 1) / K::TH, nt = tx * ty;
+    // tiles of this XCD: a contiguous eighth
+    const int xcd = blockIdx.x & 7;
+    const int t0 = (int)((unsigned)nt * xcd / 8), t1 = (int)((unsigned)nt * (xcd + 1) / 8);
+    const int istep = gridDim.x >> 3;
+
+    // (an opaque copy per use: hoisted out of the tile loop, the addresses made
+    // from it would not fit the registers)
+    auto tid_of = [&]() __attribute__((always_inline)) {
+        int i = tid;
+        asm("" : "+v"(i));
+        return i;
+    };
+    float4 v[K::NL];
+    auto load_tile = [&](int t) __attribute__((always_inline)) {
+        const int by = t / tx, y0 = by * K::TH - 1, x0 = (t - by * tx) * 8 - 1;
+        // a resource based at the tile's first row (the plane may pass 2 GiB)
+        const size_t row = (size_t)g.W * g.cin * 4;
+        const int ti = tid_of();
+        const int yb = max(y0, 0);
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(g.in + (size_t)yb * g.W * g.cin, t < t1 ? (size_t)(g.H - yb) * row : 0);
+#pragma unroll
+        for (int i = 0; i < K::NL; ++i) {
+            const int c = ti + 256 * i, pix = c / K::F, f = c - pix * K::F;
+            const int py = pix / 10, y = y0 + py, x = x0 + pix - 10 * py;
+            const bool in = pix < K::NPIX && 4 * f < g.cin && y >= 0 && y < g.H && x >= 0 && x < g.W;
+            v[i] = buf_load4(r, in ? (((y - yb) * g.W + x) * g.cin + 4 * f) * 4 : BUF_OOB);
+        }
+    };
+
+    int t = t0 + (blockIdx.x >> 3);
+    load_tile(t);
+#pragma unroll 1
+    for (; t < t1; t += istep) {
+        // ---- the halo's scale, and its split into LDS ----
+        float m = 0.f;
+#pragma unroll
+        for (int i = 0; i < K::NL; ++i)
+            m = fmaxf(m, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+        m = xrow_max(row16_max(m));
+        if (lane == 0) wmx[wave] = m;
+        lds_sync();  // (every wave is also past the last tile's reads)
+        const int e = bound_exp(fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3])));
+        const float sc = exp_scale(e);
+        const int ti = tid_of();
+#pragma unroll
+        for (int i = 0; i < K::NL; ++i) {
+            const int c = ti + 256 * i, pix = c / K::F, f = c - pix * K::F;
+            h4v hi, lo;
+            split4(__builtin_bit_cast(f4v, v[i]) * sc, hi, lo);
+            const int ks = f >> 3, qf = (f >> 1) & 3;
+            char *d = buf + 2 * ks * K::STEP + (qf * K::NP + (pix ^ (qf | (ks & 1) << 2))) * 16 + (f & 1) * 8;
+            if (K::NL * 256 == K::NPIX * K::F || pix < K::NPIX) {
+                *reinterpret_cast<h4v *>(d) = hi;
+                *reinterpret_cast<h4v *>(d + K::STEP) = lo;
+            }
+        }
+        lds_sync();
+        load_tile(t + istep);
+
+        // ---- nine taps ----
+        h8v w[2][TN][2];
+        int wpos = wbase;
+        auto load_w = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+            for (int n = 0; n < TN; ++n)
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
+                    w[slot][n][p] = __builtin_bit_cast(
+                        h8v, __builtin_amdgcn_raw_buffer_load_b128(rw_, lane * 16, wpos + (n * 2 + p) * FRAG, 0));
+            wpos += TN * 2 * FRAG;
+        };
+        load_w(0);
+        load_w(1);
+        // each row of taps is summed by itself, then added: a third as long a
+        // chain of roundings at the sum's full size (a 180-wide conv's error
+        // against 64 bits 2.2e-7 -> 1.3e-7 of its rms; one chain of all taps left
+        // an image 1.1e-7 off where the Winograd form had 8.5e-8 and this 7.7e-8)
+        f4v tot[RB][TN];
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) tot[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
+        const int pix0 = (2 * RB * rw + (j >> 3)) * 10 + (j & 7);
+        int tap = 0;
+#pragma unroll 1
+        for (int dy = 0; dy < 3; ++dy) {
+            f4v acc[RB][TN];
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int n = 0; n < TN; ++n) acc[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+            for (int dx = 0; dx < 3; ++dx, ++tap) {
+                const char *ad[RB][2];
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb) {
+                    const int pix = pix0 + (2 * rb + dy) * 10 + dx;
+                    ad[rb][0] = buf + (q * K::NP + (pix ^ q)) * 16;
+                    ad[rb][1] = buf + (q * K::NP + (pix ^ (q | 4))) * 16;
+                }
+#pragma unroll
+                for (int ks = 0; ks < KSC; ++ks) {
+                    h8v a[RB][2];
+#pragma unroll
+                    for (int p = 1; p >= 0; --p)
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb)
+                            a[rb][p] = *reinterpret_cast<const h8v *>(ad[rb][ks & 1] + (2 * ks + p) * K::STEP);
+#pragma unroll
+                    for (int mm = 0; mm < 3; ++mm)
+#pragma unroll
+                        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                            for (int n = 0; n < TN; ++n)
+                                acc[rb][n] = MFMA16H(w[ks & 1][n][mm == 1], a[rb][mm == 0], acc[rb][n]);
+                    if (ks < KSC - 2 || tap < 8) load_w(ks & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                for (int n = 0; n < TN; ++n) tot[rb][n] += acc[rb][n];
+        }
+
+        // ---- epilogue: lane (j, q) holds pixel j of each row block ----
+        const float un = exp_unscale(e) * g.unscale;
+        const int by = t / tx, x = (t - by * tx) * 8 + (j & 7);
+        const int yt = by * K::TH;
+        const __amdgpu_buffer_rsrc_t ro = buf_rsrc(g.out + (size_t)yt * g.W * g.cout, (size_t)(g.H - yt) * g.W * g.cout * 4);
+        const __amdgpu_buffer_rsrc_t rr =
+            buf_rsrc(g.res + (g.res ? (size_t)yt * g.W * g.cout : 0), g.res ? (size_t)(g.H - yt) * g.W * g.cout * 4 : 0);
+#pragma unroll
+        for (int n = 0; n < TN; ++n) {
+            const int c = 16 * (cw * TN + n) + 4 * q;
+            const f4v b = __builtin_bit_cast(f4v, buf_load4(buf_rsrc(g.bias, g.bias ? (size_t)g.cout * 4 : 0), c * 4));
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const int y = 2 * (RB * rw + rb) + (j >> 3);
+                const int off = x < g.W && yt + y < g.H && c < g.cout ? ((y * g.W + x) * g.cout + c) * 4 : BUF_OOB;
+                const f4v r = __builtin_bit_cast(f4v, buf_load4(rr, off));
+                f4v o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    o[i] = fmaf(tot[rb][n][i], un, b[i]) + r[i];
+                    if (g.lrelu) o[i] = o[i] >= 0.f ? o[i] : o[i] * g.slope;
+                }
+                buf_store4(ro, off, __builtin_bit_cast(float4, o));
+            }
+        }
+    }
+}
+
 // ---- host side ------------------------------------------------------------
 
 namespace {
@@ -1126,5 +1326,97 @@ hipError_t launch_qkv_attention(const QkvAttnArgs &g0, int hd, hipStream_t st) {
         hipLaunchKernelGGL(k_qkv_attn<30>, grid, dim3(64 * QaCfg<30>::NW), 0, st, g);
     else
         hipLaunchKernelGGL(k_qkv_attn<10>, grid, dim3(64 * QaCfg<10>::NW), 0, st, g);
+    return hipGetLastError();
+}
+
+// k_split_conv's shapes: waves side by side and column tiles per wave by cout,
+// k steps per tap by cin (both padded to 64).
+static int conv_tn(int cout) { return cout <= 64 ? 2 : (cout + 63) / 64; }
+static int conv_wc(int cout) { return cout <= 64 ? 2 : 4; }
+static int conv_ks(int cin) { return 2 * ((cin + 63) / 64); }
+bool split_conv_takes(int cin, int cout) {
+    const int a = (cin + 63) / 64, b = (cout + 63) / 64;
+    return cin % 4 == 0 && cout % 4 == 0 && cin > 0 && cout > 0 && a <= 3 && (b == 1 || b == a);
+}
+size_t split_conv_weight_floats(int cin, int cout) {
+    return (size_t)conv_wc(cout) * 9 * conv_ks(cin) * conv_tn(cout) * 2 * (FRAG / 4);
+}
+float split_conv_pack(const float *w, int cin, int cout, float *out) {
+    // one power of two for the whole tensor: a column 2^-15 of the largest still
+    // keeps 24 bits, and the products need no column scale
+    const float sc = split_row_scale(w, cout * cin * 9);
+    const int wc = conv_wc(cout), tn = conv_tn(cout), ks = conv_ks(cin);
+    uint16_t *dst = reinterpret_cast<uint16_t *>(out);
+    std::vector<float> tapw((size_t)9 * cout * cin);
+    for (int o = 0; o < cout; ++o)
+        for (int c = 0; c < cin; ++c)
+            for (int t = 0; t < 9; ++t) tapw[((size_t)t * cout + o) * cin + c] = w[((size_t)o * cin + c) * 9 + t];
+    float scs[16];
+    std::fill(scs, scs + 16, sc);
+    for (int g = 0; g < wc; ++g)
+        for (int t = 0; t < 9; ++t)
+            for (int s = 0; s < ks; ++s)
+                for (int n = 0; n < tn; ++n, dst += FRAG) {
+                    const float *rows[16];
+                    for (int r = 0; r < 16; ++r) {
+                        const int o = 16 * (g * tn + n) + r;
+                        rows[r] = o < cout ? &tapw[((size_t)t * cout + o) * cin] : nullptr;
+                    }
+                    split_pack_step(rows, scs, 32 * s, cin, dst);
+                }
+    return 1.f / sc;
+}
+
+// Row blocks per wave: the count whose rounds over two workgroups per CU take
+// least, a tile costing its row blocks plus its halo rows and a constant; at
+// most what two workgroups' registers and LDS hold.
+static int conv_rb_max(int cin, int cout) {
+    const int a = (cin + 63) / 64;
+    return cout <= 64 ? (a == 1 ? 4 : a == 2 ? 3 : 2) : (a == 2 ? 4 : 3);
+}
+static int conv_rb(int H, int W, int cin, int cout) {
+    const int wr = 4 / conv_wc(cout), slots = 2 * split_cus();
+    int best = 1;
+    double best_cost = 0;
+    for (int rb = 1; rb <= conv_rb_max(cin, cout); ++rb) {
+        const int th = 2 * rb * wr;
+        const long tiles = (long)((W + 7) / 8) * ((H + th - 1) / th);
+        const double cost = (double)((tiles + slots - 1) / slots) * (rb + 0.5);
+        if (rb == 1 || cost <= best_cost) {
+            best = rb;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
+unsigned split_conv_grid(int H, int W, int cin, int cout) {
+    const int th = 2 * conv_rb(H, W, cin, cout) * 4 / conv_wc(cout);
+    const long nt = (long)((W + 7) / 8) * ((H + th - 1) / th);
+    return 8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, split_cus() / 4));
+}
+
+template <int KSC, int TN, int WC, int RBM>
+static void conv_launch(const SplitConvArgs &g, int rb, dim3 grid, hipStream_t st) {
+    if (rb == RBM)
+        hipLaunchKernelGGL((k_split_conv<KSC, TN, RBM, WC>), grid, dim3(256), 0, st, g);
+    else if constexpr (RBM > 1)
+        conv_launch<KSC, TN, WC, RBM - 1>(g, rb, grid, st);
+}
+
+hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st) {
+    if (g.H <= 0 || g.W <= 0 || !split_conv_takes(g.cin, g.cout)) return hipErrorInvalidValue;
+    const int rb = conv_rb(g.H, g.W, g.cin, g.cout);
+    const dim3 grid(split_conv_grid(g.H, g.W, g.cin, g.cout));
+    const int a = (g.cin + 63) / 64;
+    if (g.cout <= 64) {
+        if (a == 1) conv_launch<2, 2, 2, 4>(g, rb, grid, st);
+        else if (a == 2) conv_launch<4, 2, 2, 3>(g, rb, grid, st);
+        else conv_launch<6, 2, 2, 2>(g, rb, grid, st);
+    } else if (a == 2) {
+        conv_launch<4, 2, 4, 4>(g, rb, grid, st);
+    } else {
+        conv_launch<6, 3, 4, 3>(g, rb, grid, st);
+    }
     return hipGetLastError();
 }

@@ -399,49 +399,34 @@ int s2s_test_conv3x3(int h, int w, int c_in, int c_out, const float *x, const fl
 int s2s_test_conv3x3_winograd(int h, int w, int c_in, int c_out, const float *x, const float *wgt,
                               const float *bias, int epilogue, const float *res, float slope,
                               float *out) {
-    if (epilogue != 0 && epilogue != 2 && epilogue != 5) return fail("winograd epilogue must be 0, 2 or 5");
+    if (epilogue != 0 && epilogue != 2 && epilogue != 5) return fail("epilogue must be 0, 2 or 5");
     if (epilogue == 2 && !res) return fail("residual epilogue needs res");
-    if (h <= 0 || w <= 0) return fail("the Winograd conv needs a non-empty plane");
+    if (h <= 0 || w <= 0) return fail("the conv needs a non-empty plane");
     const bool body = c_out == c_in && wino_body(c_in);
     if (!body && !wino_head(c_in, c_out))
-        return fail("the Winograd conv is the body's C -> C conv, C in {60, 120, 180}, or "
+        return fail("the conv is the body's C -> C conv, C in {60, 120, 180}, or "
                     "conv_before_upsample's C -> F, F <= 64 and a multiple of 4");
-    const size_t P = (size_t)h * w, T = wino_tiles(h, w);
-    std::vector<float> u((size_t)WINO_POS * c_out * c_in);
-    wino_weights(wgt, c_out, c_in, u.data());
-    GemmArgs g{};
-    g.lda = c_in;
-    g.ldb = c_in;
-    g.ldo = c_out;
-    g.M = (int)T;
-    g.N = c_out;
-    g.K = c_in;
-    g.nb = WINO_POS;
-    g.a_bstride = T * c_in;
-    g.o_bstride = T * c_out;
-    g.b_bstride = (size_t)c_out * c_in;
-    // U in the batched GEMM's register order, as the forward uploads it
-    const std::vector<float> ug = gemm_weights(g, ALOAD_ROWS, EPI_STORE, u.data(), WINO_POS);
+    const size_t P = (size_t)h * w;
+    SplitConvArgs g{};
+    std::vector<float> wp(split_conv_weight_floats(c_in, c_out));
+    g.unscale = split_conv_pack(wgt, c_in, c_out, wp.data());
     Dev d;
-    const float *dx = d.up(x, P * c_in), *du = d.up(ug.data(), ug.size());
-    const float *db = bias ? d.up(bias, c_out) : nullptr;
-    const float *dr = res ? d.up(res, P * c_out) : nullptr;
-    // V [36][T][C_in], then M [36][T][C_out] - over V row for row for the
-    // body's convs, in a buffer of its own for conv_before_upsample, as the
-    // forward does
-    float *dv = d.alloc<float>(WINO_POS * T * c_in), *dout = d.alloc<float>(P * c_out);
-    float *dm = body ? dv : d.alloc<float>(WINO_POS * T * c_out);
-    if (!dx || !du || !dv || !dm || !dout || (bias && !db) || (res && !dr))
+    float *dout = d.alloc<float>(P * c_out);
+    g.in = d.up(x, P * c_in);
+    g.w = d.up(wp.data(), wp.size());
+    g.bias = bias ? d.up(bias, c_out) : nullptr;
+    g.res = epilogue == 2 ? d.up(res, P * c_out) : nullptr;
+    g.out = dout;
+    g.H = h;
+    g.W = w;
+    g.cin = c_in;
+    g.cout = c_out;
+    g.lrelu = epilogue == 5;
+    g.slope = slope;
+    if (!g.in || !g.w || !dout || (bias && !g.bias) || (epilogue == 2 && !g.res))
         return fail("hipMalloc failed: out of memory");
-    g.A = dv;
-    g.B = du;
-    g.out = dm;
-    hipError_t e = launch_wino_in(dx, c_in, dv, h, w, c_in, 0);
-    if (e == hipSuccess) e = launch_gemm(g, ALOAD_ROWS, EPI_STORE, 0);
-    if (e == hipSuccess)
-        e = launch_wino_out(dm, db, epilogue == 2 ? dr : nullptr, c_out, dout, c_out, h, w, c_out,
-                            epilogue == 5, slope, 0);
-    if (int rc = finish(e, "winograd conv3x3")) return rc;
+    const hipError_t e = launch_split_conv(g, 0);
+    if (int rc = finish(e, "conv3x3 (as the forward)")) return rc;
     if (hipMemcpy(out, dout, P * c_out * 4, hipMemcpyDeviceToHost) != hipSuccess)
         return fail("hipMemcpy failed");
     return 0;

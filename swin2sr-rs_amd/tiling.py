@@ -92,7 +92,7 @@ def _fused_octaves(arch: M.Arch) -> int:
 
 
 def _wino_before_upsample(arch: M.Arch) -> bool:
-    """conv_before_upsample runs as Winograd (its products in the MLP buffer)."""
+    """The MLP buffer is planned for at least 36 planes of tiles x feat."""
     return (arch.upsampler in ("pixelshuffle", "pixelshuffle_aux", "nearest+conv")
             and arch.embed in (60, 120, 180) and arch.feat % 4 == 0 and arch.feat <= 64)
 
@@ -112,14 +112,14 @@ def _plan_terms(arch: M.Arch, h: int, w: int):
     if _unit_layout(arch):
         qkv = max(qkv, P * ((arch.heads + 1) // 2) * (6 * arch.head_dim + 2))
     if c in (60, 120, 180):
-        # the Winograd convs' 36 transform planes of 4x4-pixel tiles
+        # at least 36 planes of 4x4-pixel tiles
         qkv = max(qkv, 36 * ((hp + 3) // 4) * ((wp + 3) // 4) * c)
     if _wino_up2(arch):
         # the x4 head's Winograd 5x5 conv: 36 planes of 2x2-pixel tiles x F
         qkv = max(qkv, 36 * ((hp + 1) // 2) * ((wp + 1) // 2) * f)
     hid = P * arch.mlp_ratio * c
     if _wino_before_upsample(arch):
-        # conv_before_upsample's Winograd products (36 planes of F per tile)
+        # at least 36 planes of F per tile
         hid = max(hid, 36 * ((hp + 3) // 4) * ((wp + 3) // 4) * f)
     terms = [P * c] * 3 + [qkv, P * c, hid]
     terms += [3 * h * w, 3 * h * s * w * s, P * 4]

@@ -100,3 +100,33 @@ def test_window_attention(pkg, hd, hp, wp, shift, spread):
         hp // 8, 8, wp // 8, 8, c).transpose(0, 2, 1, 3, 4).reshape(-1, 64 * c)
     err = np.abs(win(got - want)).max(1) / np.abs(win(want)).max(1)
     assert err.max() < 5e-5, err.max()
+
+
+# the tile is 8 pixels by 2 to 16 rows: planes smaller than one, of one column of
+# tiles, ragged in both directions, and of more tiles than workgroups (2 x 256);
+# widths that end inside a k step and inside a column tile. Sums of 9 cin products
+# in fp32 on unit-normal data: sqrt(1620) roundings of 6e-8 of at most 5 would be
+# 1.2e-5.
+@pytest.mark.parametrize("cin,cout,h,w", [
+    (180, 180, 1, 1), (180, 180, 7, 9), (180, 180, 96, 100), (180, 180, 130, 124),
+    (120, 120, 40, 72), (60, 60, 3, 50), (60, 60, 150, 133), (180, 64, 50, 37),
+    (120, 32, 64, 65), (60, 4, 17, 70),
+])
+@pytest.mark.parametrize("epilogue", [0, 2, 5])
+def test_split_conv(pkg, cin, cout, h, w, epilogue):
+    import torch
+    rng = np.random.default_rng(cin + cout + h + w)
+    x = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = (rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5).astype(np.float32)
+    b = rng.standard_normal(cout, dtype=np.float32)
+    res = rng.standard_normal((h * w, cout), dtype=np.float32)
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, b, epilogue, res if epilogue == 2 else None, 0.2)
+    t = torch.from_numpy
+    want = torch.nn.functional.conv2d(t(x.astype(np.float64).reshape(h, w, cin)).permute(2, 0, 1)[None],
+                                      t(wt.astype(np.float64)), t(b.astype(np.float64)), padding=1)
+    want = want[0].permute(1, 2, 0).reshape(h * w, cout).numpy()
+    if epilogue == 2:
+        want = want + res
+    if epilogue == 5:
+        want = np.where(want < 0, 0.2 * want, want)
+    assert np.abs(got - want).max() < 2e-5
