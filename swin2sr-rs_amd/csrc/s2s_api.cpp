@@ -882,7 +882,7 @@ int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const fl
 int s2s_ctx::split_conv(const char *name, const float *in, int H, int W, int ci, int co, const float *w,
                         float un, const float *bias, const float *res, float *out, int lrelu, float slope) {
     const SplitConvArgs g{in, w, un, bias, res, out, H, W, ci, co, lrelu, slope};
-    return run(name, dim3(split_conv_grid(H, W, ci, co)), dim3(256), [&] { return launch_split_conv(g, stream); });
+    return run(name, split_conv_grid(H, W, ci, co), dim3(256), [&] { return launch_split_conv(g, stream); });
 }
 
 int s2s_ctx::forward_device(int h, int w, const float *d_in, float *d_out, bool may_graph) {

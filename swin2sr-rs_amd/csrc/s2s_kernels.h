@@ -258,7 +258,7 @@ struct SplitConvArgs {
 bool split_conv_takes(int cin, int cout);
 size_t split_conv_weight_floats(int cin, int cout);
 float split_conv_pack(const float *w, int cin, int cout, float *out);
-unsigned split_conv_grid(int H, int W, int cin, int cout);
+dim3 split_conv_grid(int H, int W, int cin, int cout);
 hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st);
 
 #define GEMM_NVARIANTS 6

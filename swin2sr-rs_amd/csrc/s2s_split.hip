@@ -884,7 +884,10 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, QOCC) void k_
 // loaded a tile ahead, scaled by its largest magnitude (one scale: a sum runs
 // over the pixels of a footprint), split and kept in LDS as [k step][part][q]
 // [pixel], so that a tap is an offset; the nine taps' weights stream from L2
-// through a register ring as in k_token_mlp. The pixel slots are permuted within
+// through a register ring as in k_token_mlp. On a plane of few tiles CS workgroups
+// (blockIdx.y) share one, each with its part of every wave's column tiles: a
+// workgroup streams all of its columns' weights, 1.3 MB at 180 wide and 12 us
+// through one CU's cache, however few its pixels. The pixel slots are permuted within
 // 8 by q and the parity of the k step, for the writes' banks (frag_slot).
 //
 // Tiles go to workgroups in plane order within each XCD, so that halos are shared
@@ -909,8 +912,10 @@ template <int KSC, int TN, int RB, int WC> struct ConvCfg {
 
 }  // namespace
 
-template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) void k_split_conv(SplitConvArgs g) {
+template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(256, 2) void k_split_conv(SplitConvArgs g) {
     using K = ConvCfg<KSC, TN, RB, WC>;
+    constexpr int NT = TN / CS;  // this workgroup's column tiles per wave, from n0
+    const int n0 = CS > 1 ? blockIdx.y * NT : 0;
     __shared__ __attribute__((aligned(16))) char buf[2 * KSC * K::STEP];
     __shared__ float wmx[4];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -980,11 +985,11 @@ template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) 
         load_tile(t + istep);
 
         // ---- nine taps ----
-        h8v w[2][TN][2];
-        int wpos = wbase;
+        h8v w[2][NT][2];
+        int wpos = wbase + n0 * 2 * FRAG;
         auto load_w = [&](int slot) __attribute__((always_inline)) {
 #pragma unroll
-            for (int n = 0; n < TN; ++n)
+            for (int n = 0; n < NT; ++n)
 #pragma unroll
                 for (int p = 0; p < 2; ++p)
                     w[slot][n][p] = __builtin_bit_cast(
@@ -997,20 +1002,20 @@ template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) 
         // chain of roundings at the sum's full size (a 180-wide conv's error
         // against 64 bits 2.2e-7 -> 1.3e-7 of its rms; one chain of all taps left
         // an image 1.1e-7 off where the Winograd form had 8.5e-8 and this 7.7e-8)
-        f4v tot[RB][TN];
+        f4v tot[RB][NT];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-            for (int n = 0; n < TN; ++n) tot[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
+            for (int n = 0; n < NT; ++n) tot[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
         const int pix0 = (2 * RB * rw + (j >> 3)) * 10 + (j & 7);
         int tap = 0;
 #pragma unroll 1
         for (int dy = 0; dy < 3; ++dy) {
-            f4v acc[RB][TN];
+            f4v acc[RB][NT];
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int n = 0; n < TN; ++n) acc[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
+                for (int n = 0; n < NT; ++n) acc[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll 1
             for (int dx = 0; dx < 3; ++dx, ++tap) {
                 const char *ad[RB][2];
@@ -1033,7 +1038,7 @@ template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) 
 #pragma unroll
                         for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                            for (int n = 0; n < TN; ++n)
+                            for (int n = 0; n < NT; ++n)
                                 acc[rb][n] = MFMA16H(w[ks & 1][n][mm == 1], a[rb][mm == 0], acc[rb][n]);
                     if (ks < KSC - 2 || tap < 8) load_w(ks & 1);
                     __builtin_amdgcn_sched_barrier(0);
@@ -1042,7 +1047,7 @@ template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) 
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb)
 #pragma unroll
-                for (int n = 0; n < TN; ++n) tot[rb][n] += acc[rb][n];
+                for (int n = 0; n < NT; ++n) tot[rb][n] += acc[rb][n];
         }
 
         // ---- epilogue: lane (j, q) holds pixel j of each row block ----
@@ -1053,8 +1058,8 @@ template <int KSC, int TN, int RB, int WC> __global__ __launch_bounds__(256, 2) 
         const __amdgpu_buffer_rsrc_t rr =
             buf_rsrc(g.res + (g.res ? (size_t)yt * g.W * g.cout : 0), g.res ? (size_t)(g.H - yt) * g.W * g.cout * 4 : 0);
 #pragma unroll
-        for (int n = 0; n < TN; ++n) {
-            const int c = 16 * (cw * TN + n) + 4 * q;
+        for (int n = 0; n < NT; ++n) {
+            const int c = 16 * (cw * TN + n0 + n) + 4 * q;
             const f4v b = __builtin_bit_cast(f4v, buf_load4(buf_rsrc(g.bias, g.bias ? (size_t)g.cout * 4 : 0), c * 4));
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
@@ -1098,9 +1103,18 @@ uint16_t f16_bits(float f) {
     return (uint16_t)(sign | ((r - 0x38000000u) >> 13));
 }
 float f16_value(uint16_t h) {
-    const uint32_t e = (h >> 10) & 31, m = h & 0x3ffu;
-    float v = e == 0 ? ldexpf((float)m, -24) : e == 31 ? (m ? NAN : INFINITY) : ldexpf((float)(m | 0x400u), (int)e - 25);
-    return (h & 0x8000u) ? -v : v;
+    const uint32_t e = (h >> 10) & 31, m = h & 0x3ffu, sign = (uint32_t)(h & 0x8000u) << 16;
+    uint32_t x;
+    if (e == 0) {
+        const float v = (float)m * 5.9604644775390625e-8f;  // 2^-24 units
+        memcpy(&x, &v, 4);
+    } else {
+        x = e == 31 ? 0x7f800000u | m << 13 : (e + 112) << 23 | m << 13;
+    }
+    x |= sign;
+    float v;
+    memcpy(&v, &x, 4);
+    return v;
 }
 
 }  // namespace
@@ -1115,15 +1129,17 @@ float split_row_scale(const float *w, int n) {
 }
 
 void split_pack_step(const float *const *rows, const float *scale, int k0, int kn, uint16_t *dst) {
-    for (int p = 0; p < 2; ++p)
-        for (int l = 0; l < 64; ++l)
-            for (int i = 0; i < 8; ++i) {
-                const int k = k0 + 8 * (l >> 4) + i;
-                const float *row = rows[l & 15];
-                const float v = row && k < kn ? row[k] * scale[l & 15] : 0.f;
-                const uint16_t hi = f16_bits(v);
-                dst[(size_t)p * 512 + l * 8 + i] = p == 0 ? hi : f16_bits(v - f16_value(hi));
-            }
+    for (int l = 0; l < 64; ++l) {
+        const float *row = rows[l & 15];
+        const float sc = scale[l & 15];
+        for (int i = 0; i < 8; ++i) {
+            const int k = k0 + 8 * (l >> 4) + i;
+            const float v = row && k < kn ? row[k] * sc : 0.f;
+            const uint16_t hi = f16_bits(v);
+            dst[l * 8 + i] = hi;
+            dst[512 + l * 8 + i] = f16_bits(v - f16_value(hi));
+        }
+    }
 }
 
 bool token_mlp_takes(int C, int ratio) { return C % 4 == 0 && C <= 192 && ratio >= 1; }
@@ -1390,24 +1406,41 @@ static int conv_rb(int H, int W, int cin, int cout) {
     return best;
 }
 
-unsigned split_conv_grid(int H, int W, int cin, int cout) {
-    const int th = 2 * conv_rb(H, W, cin, cout) * 4 / conv_wc(cout);
-    const long nt = (long)((W + 7) / 8) * ((H + th - 1) / th);
-    return 8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, split_cus() / 4));
+static long conv_tiles(int H, int W, int cout, int rb) {
+    const int th = 2 * rb * 4 / conv_wc(cout);
+    return (long)((W + 7) / 8) * ((H + th - 1) / th);
+}
+// Workgroups that share a tile's columns: all the column tiles of a wave apart
+// while the one-row-block tiles alone leave half the CUs without one (180 wide:
+// 4 tiles 15.2 -> 9.4 us, 96 tiles 15.9 -> 12.6; at 180 and 224 tiles no gain).
+static int conv_split(int H, int W, int cin, int cout) {
+    return conv_rb(H, W, cin, cout) == 1 && conv_tiles(H, W, cout, 1) <= split_cus() / 2 ? conv_tn(cout) : 1;
+}
+dim3 split_conv_grid(int H, int W, int cin, int cout) {
+    const long nt = conv_tiles(H, W, cout, conv_rb(H, W, cin, cout));
+    return dim3(8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, split_cus() / 4)),
+                (unsigned)conv_split(H, W, cin, cout));
 }
 
 template <int KSC, int TN, int WC, int RBM>
 static void conv_launch(const SplitConvArgs &g, int rb, dim3 grid, hipStream_t st) {
-    if (rb == RBM)
-        hipLaunchKernelGGL((k_split_conv<KSC, TN, RBM, WC>), grid, dim3(256), 0, st, g);
-    else if constexpr (RBM > 1)
-        conv_launch<KSC, TN, WC, RBM - 1>(g, rb, grid, st);
+    if (rb != RBM) {
+        if constexpr (RBM > 1) conv_launch<KSC, TN, WC, RBM - 1>(g, rb, grid, st);
+        return;
+    }
+    if constexpr (RBM == 1) {
+        if (grid.y > 1) {
+            hipLaunchKernelGGL((k_split_conv<KSC, TN, 1, WC, TN>), grid, dim3(256), 0, st, g);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((k_split_conv<KSC, TN, RBM, WC, 1>), grid, dim3(256), 0, st, g);
 }
 
 hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st) {
     if (g.H <= 0 || g.W <= 0 || !split_conv_takes(g.cin, g.cout)) return hipErrorInvalidValue;
     const int rb = conv_rb(g.H, g.W, g.cin, g.cout);
-    const dim3 grid(split_conv_grid(g.H, g.W, g.cin, g.cout));
+    const dim3 grid = split_conv_grid(g.H, g.W, g.cin, g.cout);
     const int a = (g.cin + 63) / 64;
     if (g.cout <= 64) {
         if (a == 1) conv_launch<2, 2, 2, 4>(g, rb, grid, st);
