@@ -42,9 +42,6 @@ typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 typedef _Float16 h4v __attribute__((ext_vector_type(4)));
 #define MFMA16H(a, b, c) __builtin_amdgcn_mfma_f32_16x16x32_f16((a), (b), (c), 0, 0, 0)
 
-#ifndef QOCC
-#define QOCC 2
-#endif
 namespace {
 
 // 2^(14 - floor(log2 b)) for a bound b >= 0 (the exponent clamped so that the
@@ -548,7 +545,7 @@ template <int HD> struct QaCfg {
 
 }  // namespace
 
-template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, QOCC) void k_qkv_attn(QkvAttnArgs g) {
+template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv_attn(QkvAttnArgs g) {
     using K = QaCfg<HD>;
     constexpr int KS = K::KS, C = K::C, NW = K::NW, TF = K::TF, DS = K::DS, NT = 64 * NW;
     constexpr int SUM_E = 4 * (HD / 8) + (HD % 8) % 4, SUM_HH = (HD % 8) / 4;
@@ -963,6 +960,16 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
 #pragma unroll
         for (int i = 0; i < K::NL; ++i)
             m = fmaxf(m, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
+        if (m == INFINITY) {  // no scale for the finite values beside it
+            m = 0.f;
+#pragma unroll
+            for (int i = 0; i < K::NL; ++i)
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const float a = fabsf(__builtin_bit_cast(f4v, v[i])[b]);
+                    m = a < INFINITY ? fmaxf(m, a) : m;
+                }
+        }
         m = xrow_max(row16_max(m));
         if (lane == 0) wmx[wave] = m;
         lds_sync();  // (every wave is also past the last tile's reads)
@@ -1322,12 +1329,12 @@ void qkv_attn_pack(const float *wqkv, const float *bqkv, int hd, float *w, float
     *v_bmax = bm;
 }
 
-// Workgroups: whole XCDs' worth of slots (a multiple of 8), at most three per CU
-// (two of the six-wave form), no more than the items.
+// Workgroups: whole XCDs' worth of slots (a multiple of 8), at most two per CU,
+// no more than the items.
 unsigned qkv_attention_grid(int hp, int wp, int hd) {
     const int nw = (hp / 8) * (wp / 8), ng = hd == 30 ? 3 : 1;
     const int per_xcd = ((nw + 7) / 8) * ng;
-    const int slots = std::max(1, split_cus() * (hd == 30 ? QOCC : 2) / 8);
+    const int slots = std::max(1, split_cus() * 2 / 8);
     return 8u * (unsigned)std::min(per_xcd, slots);
 }
 

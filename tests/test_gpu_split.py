@@ -130,3 +130,22 @@ def test_split_conv(pkg, cin, cout, h, w, epilogue):
     if epilogue == 5:
         want = np.where(want < 0, 0.2 * want, want)
     assert np.abs(got - want).max() < 2e-5
+
+
+# A non-finite value reaches the outputs whose footprint holds it and no other.
+@pytest.mark.parametrize("cin,cout", [(180, 180), (60, 60)])
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+def test_split_conv_nonfinite(pkg, cin, cout, bad):
+    h, w = 40, 33
+    rng = np.random.default_rng(7)
+    x = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = (rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5).astype(np.float32)
+    b = rng.standard_normal(cout, dtype=np.float32)
+    clean = pkg.abi.test_conv3x3_winograd(x, h, w, wt, b, 0).reshape(h, w, cout)
+    x[17 * w + 12, 5] = bad
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, b, 0).reshape(h, w, cout)
+    near = np.zeros((h, w), bool)
+    near[16:19, 11:14] = True
+    assert not np.isfinite(got[near]).any()
+    # (the scale may differ by the clean value's part in the maximum)
+    assert np.abs(got[~near] - clean[~near]).max() < 2e-5
