@@ -127,15 +127,15 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 // k_token_mlp: the token half of a Swin block in one kernel,
 //   x1  = x + LN1(o Wproj^T + b),  out = x1 + LN2(GELU(x1 W1^T + b1) W2^T + b2),
 // reading the attention output o and the block input x once and writing the
-// block output once (the three GEMMs it replaces moved 600 MB per block at
-// 264 x 264 x 180 where this moves 150).
+// block output once, and x1 once each way through the output's rows (the three
+// GEMMs it replaces moved 600 MB per block at 264 x 264 x 180 where this moves
+// 244).
 //
 // A workgroup's 4 waves own 16 TN output columns each (C <= 64 TN), all of
 // them the task's rows: RB row blocks of 16 tokens, RB <= RBM, sized so that
 // the two operand tiles (P0: o, then x1; P1: one C-wide chunk of the hidden
 // layer) let two workgroups run per CU. The hidden layer is made and consumed
-// C columns at a time, fc2's accumulators kept across the chunks. x1 stays in
-// registers in fp32 for the last residual.
+// C columns at a time, fc2's accumulators kept across the chunks.
 //
 // Weights stream through a register ring of WD k steps, refilled as consumed,
 // through GEMM and task boundaries (every task walks the same stream). The row
@@ -145,8 +145,8 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
-// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 118 us where the
-// three GEMMs took 228 (31.6 GFLOP as three f16 products each: 41 us of MFMA at
+// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 106 us where the
+// three GEMMs took 228 (22.6 GFLOP as three f16 products each: 41 us of MFMA at
 // the rate real data reaches, the rest VALU, which does not overlap MFMA on a
 // SIMD, operand reads and barriers); 2,880 tokens 15 us against 3 launches of
 // about 11.
@@ -516,7 +516,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
 // max_j sum_k |Wv[j][k]| + max|bv| over the window.
 //
 // Items go to workgroups as window w on XCD w % 8, a window's groups one after
-// another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 83
+// another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 80
 // us (the fp32 MFMA form with the weights in registers took 146); 2,880 tokens
 // 13.4 (19.9). 6 heads of 10: 5,184 tokens 13.7 us and 526,592 286, where the
 // qkv GEMM and the attention as two kernels took 20.6 and 355. With three
