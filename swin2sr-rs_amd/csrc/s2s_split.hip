@@ -139,9 +139,15 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 //
 // Weights stream through a register ring of WD k steps, refilled as consumed,
 // through GEMM and task boundaries (every task walks the same stream). The row
-// scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(C)
-// max|ln_w| + max|ln_b| (a normalised value is at most sqrt(C)), the hidden
-// layer's from bound(x1) max_j sum_k |W1[j][k]| + max|b1| (|GELU(v)| <= |v|).
+// scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(2 C)
+// max|ln_w| + max|ln_b|, the hidden layer's from bound(x1) max_j sum_k |W1[j][k]|
+// + max|b1| (|GELU(v)| <= |v|). A bound that a value passes by more than a factor
+// of two would be an infinite hi, so the LayerNorms sum squares of differences:
+// each wave takes its columns' mean, the squares about it, and the four (mean,
+// sum) pairs are combined. Every normalised value is then at most sqrt(C) in exact
+// arithmetic and sqrt(2 C) with any rounding of the means (the squares left out
+// are twice a product whose two squares are in). E[v^2] - mean^2 has no such
+// bound: emulated, rows of 180 with mean 2,000 times their deviation reach 870.
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
@@ -221,7 +227,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
     constexpr int KS = K::KS, CP = K::CP;
     __shared__ __attribute__((aligned(16))) char P0[RB * KS * 2 * FRAG];
     __shared__ __attribute__((aligned(16))) char P1[RB * KS * 2 * FRAG];
-    // per row: 4 waves' (sum, sum of squares) of LN2; LN1's, the 4 waves' max
+    // per row: 4 waves' means and sums of squares of LN2; LN1's, the 4 waves' max
     // |x| and o's row unscale lie in P1, which is free until the first chunk
     __shared__ __attribute__((aligned(16))) float red2[RB * 16][8];
     __shared__ __attribute__((aligned(16))) float lnp[4 * CP];  // LN1, LN2 weights and biases
@@ -237,7 +243,15 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
     const __amdgpu_buffer_rsrc_t rw = buf_rsrc(g.w, (size_t)4 * steps * TN * 2 * FRAG);
     const int wbase = wave * steps * TN * 2 * FRAG;
     const __amdgpu_buffer_rsrc_t rp = buf_rsrc(g.prm, (size_t)(8 + 2 * g.chunks) * CP * 4);
+    // the waves' columns: this wave's 1 / count, and each one's share of the row
+    auto cols_of = [&](int w) __attribute__((always_inline)) { return min(max(C - 16 * TN * w, 0), 16 * TN); };
+    auto uniform = [](float v) __attribute__((always_inline)) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+    };
     const float inv_c = g.inv_c;
+    const float inv_n = uniform(1.0f / (float)max(cols_of(wave), 1));
+    const float share[4] = {uniform((float)cols_of(0) * inv_c), uniform((float)cols_of(1) * inv_c),
+                            uniform((float)cols_of(2) * inv_c), uniform((float)cols_of(3) * inv_c)};
 
     for (int i = tid; i < CP; i += 256)
         reinterpret_cast<float4 *>(lnp)[i] = buf_load4(rp, 16 * i);
@@ -348,35 +362,53 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
             for (int t = 0; t < TN; ++t) acc[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
         tok_gemm<TN, RB, false>(acc, P0, st, rw, wbase, lane, steps);
 
-        // v = acc scaled back + bias, its row sums (and max |x1|'s part) to
-        // LDS; after the barrier the rows' mean and 1/std
+        // v = acc scaled back + bias, less the wave's mean of the row (acc; the
+        // padding stays 0), the mean and the sum of squares to LDS; after the
+        // barrier the rows' 1/std, and what is left of the mean times it
         float mean[RB], rstd[RB];
         auto norm_stats = [&](float(*red)[8], const float (&un)[RB]) __attribute__((always_inline)) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                float s1 = 0.f, s2 = 0.f;
+                float s = 0.f;
 #pragma unroll
                 for (int t = 0; t < TN; ++t)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float v = fmaf(acc[rb][t][i] * cs[t][i], un[rb], b[t][i]);
                         acc[rb][t][i] = v;
-                        s1 += v;
-                        s2 = fmaf(v, v, s2);
+                        s += v;
                     }
-                const float s = xrow_sum2(s1, s2);
-                if (lane < 32) red[rb * 16 + j][2 * wave + q] = s;
+                mean[rb] = xrow_sum(s) * inv_n;
+            }
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                float s = 0.f;
+#pragma unroll
+                for (int t = 0; t < TN; ++t) {
+                    const float m = off[t] != BUF_OOB ? mean[rb] : 0.f;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float d = acc[rb][t][i] - m;
+                        acc[rb][t][i] = d;
+                        s = fmaf(d, d, s);
+                    }
+                }
+                s = xrow_sum(s);
+                if (lane < 32) red[rb * 16 + j][4 * q + wave] = q ? s : mean[rb];
             }
         };
         auto norm_finish = [&](const float(*red)[8]) __attribute__((always_inline)) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                const float4 u = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][0]);
-                const float4 v = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][4]);
-                const float m = ((u.x + u.z) + (v.x + v.z)) * inv_c;
-                const float var = fmaxf(((u.y + u.w) + (v.y + v.w)) * inv_c - m * m, 0.f);
+                const f4v u = *reinterpret_cast<const f4v *>(&red[rb * 16 + j][0]);
+                const f4v v = *reinterpret_cast<const f4v *>(&red[rb * 16 + j][4]);
+                float m = 0.f, var = ((v[0] + v[1]) + (v[2] + v[3])) * inv_c;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) m = fmaf(u[w], share[w], m);
+#pragma unroll
+                for (int w = 0; w < 4; ++w) var = fmaf((u[w] - m) * share[w], u[w] - m, var);
                 rstd[rb] = __builtin_amdgcn_rsqf(var + 1e-5f);
-                mean[rb] = m * rstd[rb];
+                mean[rb] = (m - mean[rb]) * rstd[rb];
             }
         };
         auto load_ln = [&](int a, f4v(&lw)[TN], f4v(&lb)[TN]) __attribute__((always_inline)) {
@@ -1191,7 +1223,7 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
         nw = std::max(nw, std::fabs(h.n1w[c]));
         nb = std::max(nb, std::fabs(h.n1b[c]));
     }
-    *ln1_bound = sqrtf((float)C) * nw + nb;
+    *ln1_bound = sqrtf(2.0f * (float)C) * nw + nb;
     *fc1_l1 = l1;
     *fc1_bmax = bmax;
     // the stream of each wave: proj, then per chunk fc1 and fc2

@@ -5,6 +5,8 @@ input magnitudes far outside f16's range."""
 import numpy as np
 import pytest
 
+import refimpl as R
+
 pytestmark = pytest.mark.gpu
 
 
@@ -47,6 +49,42 @@ def test_token_half_sizes(pkg, orc, c, heads, ratio, hp, wp):
 @pytest.mark.parametrize("scale", [0.0, 1e-20, 1e-6, 1e6, 1e15])
 def test_token_half_magnitudes(pkg, orc, c, scale):
     assert run_stage(pkg, orc, c, 6, 2, 2, 16, 24, scale) < 1e-4
+
+
+# A bias far above the rows' deviation in front of each LayerNorm (the mean thousands
+# of times it, then a deviation below fp32's resolution of the mean). v = sum + bias,
+# the wave's mean and the row's are each rounded at the bias' magnitude, 2^-24 of it,
+# and the difference's rounding is no larger: 4 of them, over the deviation. The 1e-4
+# of the stage tests stands for the rest.
+@pytest.mark.parametrize("c", [180, 60, 24])
+@pytest.mark.parametrize("where", ["attn.proj.bias", "mlp.fc2.bias"])
+@pytest.mark.parametrize("offset", [3e2, -3e3, 3e4, 1e8])
+def test_token_half_row_offset(pkg, monkeypatch, c, where, offset):
+    M = pkg.model
+    hp, wp, heads = 8, 16, 2 if c == 24 else 6
+    arch = M.Arch(upsampler="pixelshuffle", scale=2, embed=c, heads=heads, mlp_ratio=2, depths=[1])
+    wts = M.make_weights(arch, seed=5, perturb=True)
+    bias = "layers.0.residual_group.blocks.0." + where
+    wts[bias] = (wts[bias] + np.float32(offset)).astype(np.float32)
+    x = np.random.default_rng(c).standard_normal((c, hp, wp)).astype(np.float32)
+    std, norm = [], R.layer_norm
+
+    def layer_norm(v, *args, **kw):
+        std.append(np.asarray(v).std(0).min())
+        return norm(v, *args, **kw)
+
+    monkeypatch.setattr(R, "layer_norm", layer_norm)
+    want = R.rstb(x.astype(np.float64), wts, 0, 1, 8, heads)
+    be = pkg.HipBackend(arch, wts)
+    try:
+        got = be.test_rstb(0, hp, wp, np.ascontiguousarray(x.transpose(1, 2, 0).reshape(hp * wp, c)))
+    finally:
+        be.close()
+    assert np.isfinite(got).all()
+    if abs(offset) < 1e6:
+        err = np.abs(got.reshape(hp, wp, c).transpose(2, 0, 1) - want).max() / np.abs(want).max()
+        bar = 1e-4 + 4 * 2.0 ** -24 * abs(offset) / std[where == "mlp.fc2.bias"]
+        assert err < bar, (err, bar)
 
 
 def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift):
