@@ -910,9 +910,11 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
 // A workgroup makes a tile of 8 pixels by 2 RBT rows, RBT = RB 4 / WC row blocks
 // of 2 x 8 pixels: WC waves side by side in the output columns (16 TN each), 4 /
 // WC groups of waves below one another, RB row blocks each. The tile's halo is
-// loaded a tile ahead, scaled by its largest magnitude (one scale: a sum runs
-// over the pixels of a footprint), split and kept in LDS as [k step][part][q]
-// [pixel], so that a tap is an offset; the nine taps' weights stream from L2
+// loaded a tile ahead, 16 lanes a pixel, each pixel scaled by its largest
+// magnitude, split and kept in LDS as [k step][part][q][pixel], so that a tap is
+// an offset; a tap's products are scaled back as they are added to the output's
+// sum, a lane's products all being of one pixel, so what a pixel holds bears on
+// its own footprint only, as in fp32. The nine taps' weights stream from L2
 // through a register ring as in k_token_mlp. On a plane of few tiles CS workgroups
 // (blockIdx.y) share one, each with its part of every wave's column tiles: a
 // workgroup streams all of its columns' weights, 1.3 MB at 180 wide and 12 us
@@ -934,8 +936,8 @@ template <int KSC, int TN, int RB, int WC> struct ConvCfg {
     static constexpr int TH = 2 * RBT;                    // tile rows
     static constexpr int NPIX = (TH + 2) * 10;            // halo pixels
     static constexpr int NP = (NPIX + 7) / 8 * 8;
-    static constexpr int F = 8 * KSC;                     // float4s of a pixel
-    static constexpr int NL = (NPIX * F + 255) / 256;     // loads per thread
+    static constexpr int NV = KSC / 2;                    // float4s of a pixel per lane of 16
+    static constexpr int NG = (NPIX + 15) / 16;           // pixels per 16 lanes
     static constexpr int STEP = 4 * NP * 16;              // bytes of a k step's part
 };
 
@@ -946,7 +948,7 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
     constexpr int NT = TN / CS;  // this workgroup's column tiles per wave, from n0
     const int n0 = CS > 1 ? blockIdx.y * NT : 0;
     __shared__ __attribute__((aligned(16))) char buf[2 * KSC * K::STEP];
-    __shared__ float wmx[4];
+    __shared__ float pun[K::NP];  // the pixels' unscale, less what the weights' scale adds
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, q = lane >> 4;
@@ -966,7 +968,7 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
         asm("" : "+v"(i));
         return i;
     };
-    float4 v[K::NL];
+    float4 v[K::NG][K::NV];
     auto load_tile = [&](int t) __attribute__((always_inline)) {
         const int by = t / tx, y0 = by * K::TH - 1, x0 = (t - by * tx) * 8 - 1;
         // a resource based at the tile's first row (the plane may pass 2 GiB)
@@ -975,11 +977,12 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
         const int yb = max(y0, 0);
         const __amdgpu_buffer_rsrc_t r = buf_rsrc(g.in + (size_t)yb * g.W * g.cin, t < t1 ? (size_t)(g.H - yb) * row : 0);
 #pragma unroll
-        for (int i = 0; i < K::NL; ++i) {
-            const int c = ti + 256 * i, pix = c / K::F, f = c - pix * K::F;
-            const int py = pix / 10, y = y0 + py, x = x0 + pix - 10 * py;
-            const bool in = pix < K::NPIX && 4 * f < g.cin && y >= 0 && y < g.H && x >= 0 && x < g.W;
-            v[i] = buf_load4(r, in ? (((y - yb) * g.W + x) * g.cin + 4 * f) * 4 : BUF_OOB);
+        for (int i = 0; i < K::NG; ++i) {
+            const int pix = (ti >> 4) + 16 * i, f = ti & 15, py = pix / 10, y = y0 + py, x = x0 + pix - 10 * py;
+            const bool in = pix < K::NPIX && y >= 0 && y < g.H && x >= 0 && x < g.W;
+            const int o = (((y - yb) * g.W + x) * g.cin + 4 * f) * 4;
+#pragma unroll
+            for (int u = 0; u < K::NV; ++u) v[i][u] = buf_load4(r, in && 4 * (f + 16 * u) < g.cin ? o + 256 * u : BUF_OOB);
         }
     };
 
@@ -987,35 +990,44 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
     load_tile(t);
 #pragma unroll 1
     for (; t < t1; t += istep) {
-        // ---- the halo's scale, and its split into LDS ----
-        float m = 0.f;
-#pragma unroll
-        for (int i = 0; i < K::NL; ++i)
-            m = fmaxf(m, fmaxf(fmaxf(fabsf(v[i].x), fabsf(v[i].y)), fmaxf(fabsf(v[i].z), fabsf(v[i].w))));
-        if (m == INFINITY) {  // no scale for the finite values beside it
-            m = 0.f;
-#pragma unroll
-            for (int i = 0; i < K::NL; ++i)
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const float a = fabsf(__builtin_bit_cast(f4v, v[i])[b]);
-                    m = a < INFINITY ? fmaxf(m, a) : m;
-                }
-        }
-        m = xrow_max(row16_max(m));
-        if (lane == 0) wmx[wave] = m;
-        lds_sync();  // (every wave is also past the last tile's reads)
-        const int e = bound_exp(fmaxf(fmaxf(wmx[0], wmx[1]), fmaxf(wmx[2], wmx[3])));
-        const float sc = exp_scale(e);
+        // ---- the pixels' scales, and their split into LDS ----
+        lds_sync();  // every wave is past the last tile's reads
         const int ti = tid_of();
 #pragma unroll
-        for (int i = 0; i < K::NL; ++i) {
-            const int c = ti + 256 * i, pix = c / K::F, f = c - pix * K::F;
-            h4v hi, lo;
-            split4(__builtin_bit_cast(f4v, v[i]) * sc, hi, lo);
-            const int ks = f >> 3, qf = (f >> 1) & 3;
-            char *d = buf + 2 * ks * K::STEP + (qf * K::NP + (pix ^ (qf | (ks & 1) << 2))) * 16 + (f & 1) * 8;
-            if (K::NL * 256 == K::NPIX * K::F || pix < K::NPIX) {
+        for (int i = 0; i < K::NG; ++i) {
+            const int pix = (ti >> 4) + 16 * i, f = ti & 15;
+            f4v p[K::NV];
+            float m = 0.f;
+#pragma unroll
+            for (int u = 0; u < K::NV; ++u) {
+                p[u] = __builtin_bit_cast(f4v, v[i][u]);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) m = fmaxf(m, fabsf(p[u][b]));
+            }
+            m = row16_max(m);
+            const int e = bound_exp(m);
+            float sc = exp_scale(e), un = exp_unscale(e) * 0x1p-15f;
+            if (m == INFINITY) {
+                // its infinities (as 1) and NaNs alone count, its sums times
+                // infinity
+                sc = 16384.f;
+                un = INFINITY;
+#pragma unroll
+                for (int u = 0; u < K::NV; ++u)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) {
+                        const float x = p[u][b];
+                        p[u][b] = fabsf(x) == INFINITY ? copysignf(1.f, x) : x != x ? x : 0.f;
+                    }
+            }
+            if (16 * (i + 1) > K::NPIX && pix >= K::NPIX) continue;
+            if (f == 0) pun[pix] = un;
+#pragma unroll
+            for (int u = 0; u < K::NV; ++u) {
+                h4v hi, lo;
+                split4(p[u] * sc, hi, lo);
+                const int ks = 2 * u + (f >> 3), qf = (f >> 1) & 3;
+                char *d = buf + 2 * ks * K::STEP + (qf * K::NP + (pix ^ (qf | (ks & 1) << 2))) * 16 + (f & 1) * 8;
                 *reinterpret_cast<h4v *>(d) = hi;
                 *reinterpret_cast<h4v *>(d + K::STEP) = lo;
             }
@@ -1037,10 +1049,10 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
         };
         load_w(0);
         load_w(1);
-        // each row of taps is summed by itself, then added: a third as long a
-        // chain of roundings at the sum's full size (a 180-wide conv's error
-        // against 64 bits 2.2e-7 -> 1.3e-7 of its rms; one chain of all taps left
-        // an image 1.1e-7 off where the Winograd form had 8.5e-8 and this 7.7e-8)
+        // each tap is summed by itself, then scaled back and added: also a ninth
+        // as long a chain of roundings at the sum's full size (largest error of
+        // a 180-wide conv of unit normals against 64 bits 9.5e-7; 2.0e-6 with a
+        // row of three taps in one chain, and an image 7.6e-8 off, now 6.3e-8)
         f4v tot[RB][NT];
 #pragma unroll
         for (int rb = 0; rb < RB; ++rb)
@@ -1049,20 +1061,20 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
         const int pix0 = (2 * RB * rw + (j >> 3)) * 10 + (j & 7);
         int tap = 0;
 #pragma unroll 1
-        for (int dy = 0; dy < 3; ++dy) {
-            f4v acc[RB][NT];
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int n = 0; n < NT; ++n) acc[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
+        for (int dy = 0; dy < 3; ++dy)
 #pragma unroll 1
             for (int dx = 0; dx < 3; ++dx, ++tap) {
                 const char *ad[RB][2];
+                float un[RB];
+                f4v acc[RB][NT];
 #pragma unroll
                 for (int rb = 0; rb < RB; ++rb) {
                     const int pix = pix0 + (2 * rb + dy) * 10 + dx;
                     ad[rb][0] = buf + (q * K::NP + (pix ^ q)) * 16;
                     ad[rb][1] = buf + (q * K::NP + (pix ^ (q | 4))) * 16;
+                    un[rb] = pun[pix];
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[rb][n] = f4v{0.f, 0.f, 0.f, 0.f};
                 }
 #pragma unroll
                 for (int ks = 0; ks < KSC; ++ks) {
@@ -1082,15 +1094,15 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
                     if (ks < KSC - 2 || tap < 8) load_w(ks & 1);
                     __builtin_amdgcn_sched_barrier(0);
                 }
+#pragma unroll
+                for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) tot[rb][n][i] = fmaf(acc[rb][n][i], un[rb], tot[rb][n][i]);
             }
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb)
-#pragma unroll
-                for (int n = 0; n < NT; ++n) tot[rb][n] += acc[rb][n];
-        }
 
         // ---- epilogue: lane (j, q) holds pixel j of each row block ----
-        const float un = exp_unscale(e) * g.unscale;
         const int by = t / tx, x = (t - by * tx) * 8 + (j & 7);
         const int yt = by * K::TH;
         const __amdgpu_buffer_rsrc_t ro = buf_rsrc(g.out + (size_t)yt * g.W * g.cout, (size_t)(g.H - yt) * g.W * g.cout * 4);
@@ -1108,7 +1120,7 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
                 f4v o;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    o[i] = fmaf(tot[rb][n][i], un, b[i]) + r[i];
+                    o[i] = fmaf(tot[rb][n][i], g.unscale, b[i]) + r[i];
                     if (g.lrelu) o[i] = o[i] >= 0.f ? o[i] : o[i] * g.slope;
                 }
                 buf_store4(ro, off, __builtin_bit_cast(float4, o));
@@ -1419,7 +1431,7 @@ float split_conv_pack(const float *w, int cin, int cout, float *out) {
                     }
                     split_pack_step(rows, scs, 32 * s, cin, dst);
                 }
-    return 1.f / sc;
+    return 32768.f / sc;  // (the pixels' unscale holds the other 2^-15)
 }
 
 // Row blocks per wave: the count whose rounds over two workgroups per CU take

@@ -187,3 +187,54 @@ def test_split_conv_nonfinite(pkg, cin, cout, bad):
     assert not np.isfinite(got[near]).any()
     # (the scale may differ by the clean value's part in the maximum)
     assert np.abs(got[~near] - clean[~near]).max() < 2e-5
+
+
+def conv_f64(x, wt, b, h, w):
+    import torch
+    t = torch.from_numpy
+    y = torch.nn.functional.conv2d(t(x.astype(np.float64).reshape(h, w, -1)).permute(2, 0, 1)[None],
+                                   t(wt.astype(np.float64)), t(b.astype(np.float64)), padding=1)
+    return y[0].permute(1, 2, 0).numpy()
+
+
+# Pixels of one tile apart by up to 2^60, one of them alone among small ones: an
+# output owes nothing to pixels outside its footprint, as in fp32, so each output's
+# error is held against its own footprint's largest pixel. 2e-5 as above.
+@pytest.mark.parametrize("cin,cout,h,w", [(180, 180, 13, 11), (180, 180, 96, 100), (120, 120, 9, 20),
+                                          (60, 60, 40, 33), (180, 64, 50, 37), (120, 32, 17, 9)])
+@pytest.mark.parametrize("spread", [20, 60])
+def test_split_conv_pixels_apart(pkg, cin, cout, h, w, spread):
+    rng = np.random.default_rng(cin + cout + h + spread)
+    mag = 2.0 ** -rng.integers(0, spread, (h, w))
+    mag[h // 2 - 3:h // 2 + 4, w // 2 - 3:w // 2 + 4] = 2.0 ** -spread
+    mag[h // 2, w // 2] = 1.0
+    x = (rng.standard_normal((h, w, cin)) * mag[..., None]).astype(np.float32).reshape(h * w, cin)
+    wt = (rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5).astype(np.float32)
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, np.zeros(cout, np.float32), 0).reshape(h, w, cout)
+    want = conv_f64(x, wt, np.zeros(cout), h, w)
+    pad = np.pad(mag, 1)
+    near = np.max([pad[i:i + h, j:j + w] for i in range(3) for j in range(3)], 0)
+    err = (np.abs(got - want) / near[..., None]).max()
+    assert err < 2e-5, err
+
+
+# An infinity is that infinity times the weight's sign in every output whose
+# footprint holds it, a NaN or two opposite infinities in one tap sum a NaN.
+@pytest.mark.parametrize("cin,cout", [(180, 180), (60, 60), (180, 64)])
+@pytest.mark.parametrize("epilogue", [0, 5])
+def test_split_conv_infinities(pkg, cin, cout, epilogue):
+    h, w = 40, 33
+    rng = np.random.default_rng(9)
+    x = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = (rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5).astype(np.float32)
+    b = rng.standard_normal(cout, dtype=np.float32)
+    x[3 * w + 5, 7], x[17 * w + 12, 5], x[30 * w + 32, cin - 1], x[22 * w, 3] = np.inf, -np.inf, np.inf, np.nan
+    x[30 * w + 32, 1] = 3e38
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, b, epilogue, None, 0.2).reshape(h, w, cout)
+    with np.errstate(invalid="ignore"):
+        want = conv_f64(x, wt, b, h, w)
+    if epilogue == 5:
+        want = np.where(want < 0, 0.2 * want, want)
+    bad = ~np.isfinite(want)
+    assert np.array_equal(got[bad], want[bad].astype(np.float32), equal_nan=True)
+    assert np.abs(got[~bad] - want[~bad]).max() < 2e-5
