@@ -75,7 +75,6 @@ struct StageW {
     std::vector<BlockW> blocks;
     // the stage close: its 3x3 conv with the 1x1 patch_embed conv folded in
     float *conv_w = nullptr, *conv_b = nullptr;
-    float conv_un = 0.f;  // k_split_conv's unscale of conv_w
 };
 
 struct ProfKey {
@@ -131,8 +130,6 @@ static bool fits_in(const AllocList &l, const std::vector<BufSpec> &v) {
 struct s2s_ctx {
     s2s_arch arch{};
     int c = 0, hd = 0, hidden = 0, feat = 0, octaves = 0;
-    // the unscales of the convs that run on k_split_conv (0: the implicit GEMM)
-    float cab_un = 0.f, cbu_un = 0.f, hr_un = 0.f;
     int device = 0;
     hipStream_t stream = nullptr;
     AllocList weight_allocs;
@@ -307,10 +304,10 @@ struct s2s_ctx {
     int gemm(const char *name, const GemmArgs &g, int aload, int epi);
     int block_fwd(const BlockW &b, int hp, int wp, int shift, const float *x_in, float *x_out);
     int stage_fwd(int s, int hp, int wp, const float *x_in, float *x_out);
-    int conv_body(const char *name, const float *in, int H, int W, const float *w, float un,
+    int conv_body(const char *name, const float *in, int H, int W, const float *w,
                   const float *bias, const float *res, float *out);
     int split_conv(const char *name, const float *in, int H, int W, int ci, int co, const float *w,
-                   float un, const float *bias, const float *res, float *out, int lrelu, float slope);
+                   const float *bias, const float *res, float *out, int lrelu, float slope);
     int forward_device(int h, int w, const float *d_in, float *d_out, bool may_graph = true);
     int forward_launches(int h, int w, const float *d_in, float *d_out);
     int head(int h, int w, float *d_out);
@@ -852,20 +849,19 @@ int s2s_ctx::stage_fwd(int s, int hp, int wp, const float *x_in, float *x_out) {
     // patch_embed conv, the stage's residual) as one conv: the two
     // convolutions are folded into one at upload, and the residual is added
     // element by element, so it may write over x_in.
-    return conv_body("conv3x3_stage", src, hp, wp, st.conv_w, st.conv_un, st.conv_b, x_in, x_out);
+    return conv_body("conv3x3_stage", src, hp, wp, st.conv_w, st.conv_b, x_in, x_out);
 }
 
 // A C -> C 3x3 conv of the body (the stage close, conv_after_body), + bias +
-// residual, on k_split_conv for the widths it takes (un its weights' unscale),
-// else as the implicit-GEMM conv with the residual as its epilogue.
-int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const float *w, float un,
+// residual, on k_split_conv for the widths it takes, else as the implicit-GEMM conv with the residual as its epilogue.
+int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const float *w,
                        const float *bias, const float *res, float *out) {
     // the residual is added element by element; only a conv that reads the
     // plane it writes (a stage with no blocks) goes through `o` (free between
     // blocks)
     float *dst = in == out ? o : out;
     if (split_conv_takes(c, c)) {
-        if (split_conv(name, in, H, W, c, c, w, un, bias, res, dst, 0, 0.f)) return -1;
+        if (split_conv(name, in, H, W, c, c, w, bias, res, dst, 0, 0.f)) return -1;
     } else {
         GemmArgs g = conv_gemm(in, H, W, c, w, bias, dst, c, c);
         g.res = res;
@@ -880,8 +876,8 @@ int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const fl
 }
 
 int s2s_ctx::split_conv(const char *name, const float *in, int H, int W, int ci, int co, const float *w,
-                        float un, const float *bias, const float *res, float *out, int lrelu, float slope) {
-    const SplitConvArgs g{in, w, un, bias, res, out, H, W, ci, co, lrelu, slope};
+                        const float *bias, const float *res, float *out, int lrelu, float slope) {
+    const SplitConvArgs g{in, w, bias, res, out, H, W, ci, co, lrelu, slope};
     return run(name, split_conv_grid(H, W, ci, co), dim3(256), [&] { return launch_split_conv(g, stream); });
 }
 
@@ -985,7 +981,7 @@ int s2s_ctx::forward_launches(int h, int w, const float *d_in, float *d_out) {
             [&] { return launch_layernorm(cur, norm_w, norm_b, nullptr, o, P, c, stream); }))
         return -1;
     // (the final norm lands in the attention output's plane, free after the blocks)
-    if (conv_body("conv_after_body", o, hp, wp, cab_w, cab_un, cab_b, body, cur)) return -1;
+    if (conv_body("conv_after_body", o, hp, wp, cab_w, cab_b, body, cur)) return -1;
     return head(h, w, d_out);
 }
 
@@ -999,7 +995,7 @@ int s2s_ctx::head(int h, int w, float *d_out) {
     // conv_before_upsample + LeakyReLU(0.01) into the first feature plane
     auto before_upsample = [&]() -> int {
         if (split_conv_takes(c, feat))
-            return split_conv("conv_before_upsample", cur, hp, wp, c, feat, cbu_w, cbu_un, cbu_b, nullptr,
+            return split_conv("conv_before_upsample", cur, hp, wp, c, feat, cbu_w, cbu_b, nullptr,
                               fplanes[0], 1, 0.01f);
         g = conv_gemm(cur, hp, wp, c, cbu_w, cbu_b, fplanes[0], feat, feat);
         g.slope = 0.01f;
@@ -1136,7 +1132,7 @@ int s2s_ctx::head(int h, int w, float *d_out) {
         g.slope = 0.2f;
         if (gemm("conv_up2", g, ALOAD_SUB2, EPI_LRELU)) return -1;
         if (split_conv_takes(feat, feat)) {
-            if (split_conv("conv_hr", fplanes[2], 4 * hp, 4 * wp, feat, feat, hr_w, hr_un, hr_b, nullptr,
+            if (split_conv("conv_hr", fplanes[2], 4 * hp, 4 * wp, feat, feat, hr_w, hr_b, nullptr,
                            fplanes[3], 1, 0.2f))
                 return -1;
         } else {
@@ -1206,12 +1202,12 @@ std::vector<float> conv_relayout(const float *w, int co, int ci, const std::vect
 }
 
 // A 3x3 conv's weights [co][ci][3][3] as its kernel reads them: k_split_conv's
-// packing (*un its unscale) for the shapes it takes, else the implicit GEMM's
+// packing for the shapes it takes, else the implicit GEMM's
 // [co][tap][ci_pad4].
-std::vector<float> conv_weights(const float *w, int co, int ci, float *un) {
+std::vector<float> conv_weights(const float *w, int co, int ci) {
     if (!split_conv_takes(ci, co)) return conv_relayout(w, co, ci, nullptr);
     std::vector<float> p(split_conv_weight_floats(ci, co));
-    *un = split_conv_pack(w, ci, co, p.data());
+    split_conv_pack(w, ci, co, p.data());
     return p;
 }
 uint64_t conv_weight_floats(int co, int ci) {
@@ -1548,12 +1544,12 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
         subpixel_weights(x->data, F, F, w.data());
         return ctx->upload(w, dst);
     };
-    auto up_conv = [&](const std::string &name, int co, int ci, float **dst, float *un) -> int {
+    auto up_conv = [&](const std::string &name, int co, int ci, float **dst) -> int {
         if (ts.get(name, {co, ci, 3, 3}, &x)) return -1;
-        return ctx->upload(conv_weights(x->data, co, ci, un), dst);
+        return ctx->upload(conv_weights(x->data, co, ci), dst);
     };
     auto up_before_upsample = [&](int F) -> int {
-        return up_conv("conv_before_upsample.0.weight", F, C, &ctx->cbu_w, &ctx->cbu_un);
+        return up_conv("conv_before_upsample.0.weight", F, C, &ctx->cbu_w);
     };
 
     rc = rc || up("conv_first.bias", {C}, &ctx->cf_b);
@@ -1599,7 +1595,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
     {
         const s2s_tensor *cw;
         rc = rc || ts.get("conv_after_body.weight", {C, C, 3, 3}, &cw);
-        if (!rc) rc = ctx->upload(conv_weights(cw->data, C, C, &ctx->cab_un), &ctx->cab_w);
+        if (!rc) rc = ctx->upload(conv_weights(cw->data, C, C), &ctx->cab_w);
     }
     rc = rc || up("conv_after_body.bias", {C}, &ctx->cab_b);
 
@@ -1641,7 +1637,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
                 for (size_t k = 0; k < kk; ++k) wf[(size_t)o * kk + k] = (float)acc[k];
                 bf[o] = (float)ab;
             }
-            rc = rc || ctx->upload(conv_weights(wf.data(), C, C, &st.conv_un), &st.conv_w);
+            rc = rc || ctx->upload(conv_weights(wf.data(), C, C), &st.conv_w);
             rc = rc || ctx->upload(bf, &st.conv_b);
         }
         st.blocks.resize(A.depths[s]);
@@ -1878,7 +1874,7 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
             rc = rc || up("conv_up1.bias", {F}, &ctx->nu1_b);
             rc = rc || up_sub2("conv_up2.weight", F, &ctx->nu2_w);
             rc = rc || up("conv_up2.bias", {F}, &ctx->nu2_b);
-            rc = rc || up_conv("conv_hr.weight", F, F, &ctx->hr_w, &ctx->hr_un);
+            rc = rc || up_conv("conv_hr.weight", F, F, &ctx->hr_w);
             rc = rc || up("conv_hr.bias", {F}, &ctx->hr_b);
             rc = rc || conv_last(F);
         }

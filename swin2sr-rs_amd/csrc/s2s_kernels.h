@@ -243,12 +243,11 @@ void split_pack_step(const float *const *rows, const float *scale, int k0, int k
 
 // A 3x3 stride-1 zero-pad-1 conv of the channel-last H x W plane `in` [H*W][cin]
 // into out [H*W][cout] (k_split_conv, s2s_split.hip): + bias (or null), + res
-// [H*W][cout] (or null; may be out), then LeakyReLU(slope) if lrelu. w and
-// unscale from split_conv_pack of the [cout][cin][3][3] weights.
+// [H*W][cout] (or null; may be out), then LeakyReLU(slope) if lrelu. w from
+// split_conv_pack of the [cout][cin][3][3] weights.
 struct SplitConvArgs {
     const float *in;
     const float *w;
-    float unscale;
     const float *bias, *res;
     float *out;
     int H, W, cin, cout;
@@ -257,7 +256,7 @@ struct SplitConvArgs {
 };
 bool split_conv_takes(int cin, int cout);
 size_t split_conv_weight_floats(int cin, int cout);
-float split_conv_pack(const float *w, int cin, int cout, float *out);
+void split_conv_pack(const float *w, int cin, int cout, float *out);
 dim3 split_conv_grid(int H, int W, int cin, int cout);
 hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st);
 

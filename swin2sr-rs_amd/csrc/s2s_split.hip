@@ -948,12 +948,12 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
     constexpr int NT = TN / CS;  // this workgroup's column tiles per wave, from n0
     const int n0 = CS > 1 ? blockIdx.y * NT : 0;
     __shared__ __attribute__((aligned(16))) char buf[2 * KSC * K::STEP];
-    __shared__ float pun[K::NP];  // the pixels' unscale, less what the weights' scale adds
+    __shared__ float pun[K::NP];  // the pixels' unscale x 2^-15
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, q = lane >> 4;
     const int cw = wave % WC, rw = wave / WC;
-    const __amdgpu_buffer_rsrc_t rw_ = buf_rsrc(g.w, (size_t)WC * 9 * KSC * TN * 2 * FRAG);
+    const __amdgpu_buffer_rsrc_t rw_ = buf_rsrc(g.w, (size_t)WC * (9 * KSC * TN * 2 * FRAG + 64 * TN));
     const int wbase = cw * 9 * KSC * TN * 2 * FRAG;
     const int tx = (g.W + 7) / 8, ty = (g.H + K::TH - 1) / K::TH, nt = tx * ty;
     // tiles of this XCD: a contiguous eighth
@@ -1111,6 +1111,7 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
             const int c = 16 * (cw * TN + n0 + n) + 4 * q;
+            const f4v cs = __builtin_bit_cast(f4v, buf_load4(rw_, WC * 9 * KSC * TN * 2 * FRAG + 4 * c));
             const f4v b = __builtin_bit_cast(f4v, buf_load4(buf_rsrc(g.bias, g.bias ? (size_t)g.cout * 4 : 0), c * 4));
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
@@ -1120,7 +1121,7 @@ template <int KSC, int TN, int RB, int WC, int CS> __global__ __launch_bounds__(
                 f4v o;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    o[i] = fmaf(tot[rb][n][i], g.unscale, b[i]) + r[i];
+                    o[i] = fmaf(tot[rb][n][i], cs[i], b[i]) + r[i];
                     if (g.lrelu) o[i] = o[i] >= 0.f ? o[i] : o[i] * g.slope;
                 }
                 buf_store4(ro, off, __builtin_bit_cast(float4, o));
@@ -1406,20 +1407,18 @@ bool split_conv_takes(int cin, int cout) {
     return cin % 4 == 0 && cout % 4 == 0 && cin > 0 && cout > 0 && a <= 3 && (b == 1 || b == a);
 }
 size_t split_conv_weight_floats(int cin, int cout) {
-    return (size_t)conv_wc(cout) * 9 * conv_ks(cin) * conv_tn(cout) * 2 * (FRAG / 4);
+    // the fragments, then the columns' unscale
+    return (size_t)conv_wc(cout) * conv_tn(cout) * (9 * conv_ks(cin) * 2 * (FRAG / 4) + 16);
 }
-float split_conv_pack(const float *w, int cin, int cout, float *out) {
-    // one power of two for the whole tensor: a column 2^-15 of the largest still
-    // keeps 24 bits, and the products need no column scale
-    const float sc = split_row_scale(w, cout * cin * 9);
+void split_conv_pack(const float *w, int cin, int cout, float *out) {
     const int wc = conv_wc(cout), tn = conv_tn(cout), ks = conv_ks(cin);
     uint16_t *dst = reinterpret_cast<uint16_t *>(out);
     std::vector<float> tapw((size_t)9 * cout * cin);
     for (int o = 0; o < cout; ++o)
         for (int c = 0; c < cin; ++c)
             for (int t = 0; t < 9; ++t) tapw[((size_t)t * cout + o) * cin + c] = w[((size_t)o * cin + c) * 9 + t];
-    float scs[16];
-    std::fill(scs, scs + 16, sc);
+    std::vector<float> scale(16 * wc * tn, 1.f);
+    for (int o = 0; o < cout; ++o) scale[o] = split_row_scale(w + (size_t)o * cin * 9, cin * 9);
     for (int g = 0; g < wc; ++g)
         for (int t = 0; t < 9; ++t)
             for (int s = 0; s < ks; ++s)
@@ -1429,9 +1428,11 @@ float split_conv_pack(const float *w, int cin, int cout, float *out) {
                         const int o = 16 * (g * tn + n) + r;
                         rows[r] = o < cout ? &tapw[((size_t)t * cout + o) * cin] : nullptr;
                     }
-                    split_pack_step(rows, scs, 32 * s, cin, dst);
+                    split_pack_step(rows, &scale[16 * (g * tn + n)], 32 * s, cin, dst);
                 }
-    return 32768.f / sc;  // (the pixels' unscale holds the other 2^-15)
+    // (the pixels' unscale holds 2^-15 of it, so that a sum stays near its value)
+    float *un = reinterpret_cast<float *>(dst);
+    for (float sc : scale) *un++ = 32768.f / sc;
 }
 
 // Row blocks per wave: the count whose rounds over two workgroups per CU take

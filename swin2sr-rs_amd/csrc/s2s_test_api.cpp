@@ -409,7 +409,7 @@ int s2s_test_conv3x3_winograd(int h, int w, int c_in, int c_out, const float *x,
     const size_t P = (size_t)h * w;
     SplitConvArgs g{};
     std::vector<float> wp(split_conv_weight_floats(c_in, c_out));
-    g.unscale = split_conv_pack(wgt, c_in, c_out, wp.data());
+    split_conv_pack(wgt, c_in, c_out, wp.data());
     Dev d;
     float *dout = d.alloc<float>(P * c_out);
     g.in = d.up(x, P * c_in);

@@ -238,3 +238,17 @@ def test_split_conv_infinities(pkg, cin, cout, epilogue):
     bad = ~np.isfinite(want)
     assert np.array_equal(got[bad], want[bad].astype(np.float32), equal_nan=True)
     assert np.abs(got[~bad] - want[~bad]).max() < 2e-5
+
+
+# Output channels apart by up to 2^40: each one's error against its own weights.
+@pytest.mark.parametrize("cin,cout", [(180, 180), (120, 120), (60, 60), (180, 64), (60, 4)])
+def test_split_conv_channels_apart(pkg, cin, cout):
+    h, w = 20, 33
+    rng = np.random.default_rng(cin + cout)
+    x = rng.standard_normal((h * w, cin), dtype=np.float32)
+    mag = 2.0 ** -rng.permutation(np.linspace(0, 40, cout).astype(int))
+    wt = rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5
+    wt = (wt * mag[:, None, None, None]).astype(np.float32)
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, np.zeros(cout, np.float32), 0).reshape(h, w, cout)
+    err = (np.abs(got - conv_f64(x, wt, np.zeros(cout), h, w)) / mag).max()
+    assert err < 2e-5, err
