@@ -545,7 +545,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
 // Head columns are padded to whole tiles: 30 to 32, 10 to 16. The scales: x's
 // rows from their maximum; q and k are unit vectors (2^14); the probabilities
 // are at most 1 (2^14, in the exponent's argument); v from the bound max|x|
-// max_j sum_k |Wv[j][k]| + max|bv| over the window.
+// max_j sum_k |Wv[j][k]| + max|bv|, over the window or token by token (VSPAN).
 //
 // Items go to workgroups as window w on XCD w % 8, a window's groups one after
 // another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 80
@@ -574,6 +574,14 @@ template <int HD> struct QaCfg {
     static constexpr int TILE = 4 * KS * 2 * FRAG;   // bytes of the token tile
     static constexpr int BUF = GH * HB > TILE ? GH * HB : TILE;
 };
+// Tokens of a window share v's scale while their bounds lie within 2^VSPAN of each
+// other, as they do in real images. Further apart each has its own, and the
+// probabilities take what it lies below the largest, since a query that sees only
+// small tokens is owed their precision: with a shared scale its error is 2.1e-6 of
+// sum P |v| at 2^10 (as at 1), 2.1e-5 at 2^20 and 0.6 at 2^40, with their own at
+// most 5e-6. At 264 x 264 windows that all spread take 86 us against 84 (heads of
+// 30) and 56 against 54 (of 10).
+constexpr int VSPAN = 6;
 
 }  // namespace
 
@@ -585,6 +593,8 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
     __shared__ __attribute__((aligned(16))) char buf[K::BUF];
     __shared__ __attribute__((aligned(16))) float xun[64];  // the rows' unscale
     __shared__ __attribute__((aligned(16))) float xmx[64];  // the rows' max |x|
+    // v's scale per token, and what it lies below the largest token's (wide windows)
+    __shared__ __attribute__((aligned(16))) float vsc[64], vlow[64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 15, q = lane >> 4;
@@ -711,11 +721,16 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
             __builtin_amdgcn_sched_barrier(0);
         }
         if (wave < 4) load_x(it + istep);
-        // v's scale: the largest row maximum of the window
-        float vmx = xmx[lane];
-        vmx = xrow_max(row16_max(vmx));
-        const int ev = bound_exp(fmaf(vmx, g.v_l1, g.v_bmax));
-        const float vsc = exp_scale(ev);
+        // v's scale, from the bound of |v| of the window's largest row, or of each
+        // token's own where the rows lie further apart than 2^VSPAN (`wide`)
+        const float vb = fmaf(xmx[lane], g.v_l1, g.v_bmax);
+        const int ev = __builtin_amdgcn_readfirstlane(bound_exp(xrow_max(row16_max(vb))));
+        const bool wide = ev - __builtin_amdgcn_readfirstlane(bound_exp(-xrow_max(row16_max(-vb)))) > VSPAN;
+        if (wave == 0) {
+            const int et = wide ? max(bound_exp(vb), ev - 60) : ev;
+            vsc[lane] = exp_scale(et);
+            vlow[lane] = __builtin_bit_cast(float, (127 + et - ev) << 23);
+        }
         lds_sync();  // every wave has read the token tile
         {
             // q and k: unit vectors times 2^14. A head of 30 has both tiles
@@ -763,10 +778,11 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
 #pragma unroll
             for (int rb = 0; rb < 4; ++rb) {
                 const f4v un = *reinterpret_cast<const f4v *>(&xun[16 * rb + 4 * q]);
+                const f4v sc = *reinterpret_cast<const f4v *>(&vsc[16 * rb + 4 * q]);
                 f4v v;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
-                    v[i] = fmaf(acc[rb][2][i] * csv, un[i], biv) * vsc;
+                    v[i] = fmaf(acc[rb][2][i] * csv, un[i], biv) * sc[i];
                     v[i] = d == HD ? 1.0f : v[i];
                 }
                 h4v hi, lo;
@@ -839,34 +855,64 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
             for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) mx = fmaxf(mx, sa[kt][e]);
-            mx = half_max(mx) - 14.0f;  // (probabilities times 2^14)
+            mx = half_max(mx);
             f16acc o;
 #pragma unroll
             for (int e = 0; e < 16; ++e) o[e] = 0.f;
             const char *vb = hb + 4 * K::QB + (hh * K::VR + (r & (K::VR - 1))) * 16;
+            // o += V^T P^T, P from its value at sa[kt][e]
+            auto pv = [&](auto prob) __attribute__((always_inline)) {
 #pragma unroll
-            for (int kt = 0; kt < 2; ++kt)
+                for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const h8v vh = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB);
-                    const h8v vl = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB + K::VB / 2);
-                    h4v ph[2], pl[2];
+                    for (int s = 0; s < 2; ++s) {
+                        const h8v vh = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB);
+                        const h8v vl = *reinterpret_cast<const h8v *>(vb + (2 * kt + s) * K::VB + K::VB / 2);
+                        h4v ph[2], pl[2];
 #pragma unroll
-                    for (int a = 0; a < 2; ++a) {
-                        f4v p;
+                        for (int a = 0; a < 2; ++a) {
+                            f4v p;
 #pragma unroll
-                        for (int b = 0; b < 4; ++b) p[b] = __builtin_amdgcn_exp2f(sa[kt][8 * s + 4 * a + b] - mx);
-                        split4(p, ph[a], pl[a]);
+                            for (int b = 0; b < 4; ++b) p[b] = prob(sa[kt][8 * s + 4 * a + b]);
+                            split4(p, ph[a], pl[a]);
+                        }
+                        const h8v p8 = __builtin_shufflevector(ph[0], ph[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        const h8v l8 = __builtin_shufflevector(pl[0], pl[1], 0, 1, 2, 3, 4, 5, 6, 7);
+                        o = MFMA32H(vh, l8, o);
+                        o = MFMA32H(vl, p8, o);
+                        o = MFMA32H(vh, p8, o);
                     }
-                    const h8v p8 = __builtin_shufflevector(ph[0], ph[1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    const h8v l8 = __builtin_shufflevector(pl[0], pl[1], 0, 1, 2, 3, 4, 5, 6, 7);
-                    o = MFMA32H(vh, l8, o);
-                    o = MFMA32H(vl, p8, o);
-                    o = MFMA32H(vh, p8, o);
-                }
-            float lo, hi;
-            halves(o[SUM_E], lo, hi);
-            const float inv = exp_unscale(ev) / (SUM_HH ? hi : lo);
+            };
+            float inv = exp_unscale(ev);
+            if (!wide) {
+                mx -= 14.0f;  // (probabilities times 2^14)
+                pv([&](float v) __attribute__((always_inline)) { return __builtin_amdgcn_exp2f(v - mx); });
+                float lo, hi;
+                halves(o[SUM_E], lo, hi);
+                inv /= SUM_HH ? hi : lo;
+            } else {
+                // the small tokens' v is held larger by 1 / vlow: the probabilities
+                // times vlow, scaled anew by the query's largest such product, and
+                // the denominator summed from the probabilities themselves
+                float sum = 0.f, pm = 0.f;
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int a = 0; a < 4; ++a) {
+                        const f4v low = *reinterpret_cast<const f4v *>(&vlow[32 * kt + 8 * a + 4 * hh]);
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) {
+                            const float p = __builtin_amdgcn_exp2f(sa[kt][4 * a + b] - mx);
+                            sum += p;
+                            sa[kt][4 * a + b] = p * low[b];
+                            pm = fmaxf(pm, p * low[b]);
+                        }
+                    }
+                const int ep = bound_exp(half_max(pm));
+                const float sc = exp_scale(ep);
+                pv([&](float v) __attribute__((always_inline)) { return v * sc; });
+                inv *= exp_unscale(ep) / half_sum(sum);
+            }
             // O over this wave's own q operands, [32][HD] floats
             float *orow = reinterpret_cast<float *>(hb + qt * K::QB) + r * HD;
 #pragma unroll

@@ -87,8 +87,9 @@ def test_token_half_row_offset(pkg, monkeypatch, c, where, offset):
         assert err < bar, (err, bar)
 
 
-def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift):
-    """qkv projection and window attention in 64 bits, on [hp*wp][c] rows."""
+def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift, norms=False):
+    """qkv projection and window attention in 64 bits, on [hp*wp][c] rows; with
+    norms, of the norms of each head's v in the place of its values."""
     c = heads * hd
     X = x.astype(np.float64).reshape(hp, wp, c)
     X = np.roll(X, (-shift, -shift), (0, 1))
@@ -96,6 +97,8 @@ def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift):
     qkv = win(X) @ w.astype(np.float64).T + b
     q, k, v = (t.reshape(-1, 64, heads, hd).transpose(0, 2, 1, 3) for t in np.split(qkv, 3, -1))
     q, k = (t / np.maximum(np.linalg.norm(t, axis=-1, keepdims=True), 1e-12) for t in (q, k))
+    if norms:
+        v = np.repeat(np.linalg.norm(v, axis=-1, keepdims=True), hd, -1)
     s = q @ k.transpose(0, 1, 3, 2)
     s = s * np.exp(np.minimum(ls.astype(np.float64), np.log(100.0)))[None, :, None, None]
     s += cpb.astype(np.float64).reshape(64, 64, heads).transpose(2, 0, 1)
@@ -138,6 +141,37 @@ def test_window_attention(pkg, hd, hp, wp, shift, spread):
         hp // 8, 8, wp // 8, 8, c).transpose(0, 2, 1, 3, 4).reshape(-1, 64 * c)
     err = np.abs(win(got - want)).max(1) / np.abs(win(want)).max(1)
     assert err.max() < 5e-5, err.max()
+
+
+# Tokens of a window apart by up to 2^50: a row of the plane that the shift mask
+# parts from the rest of its windows, single tokens, and every token. An output's
+# error is held against the sum of its probabilities times the norms of v, to which
+# fp32's is in proportion, so a large token that a query hardly sees costs it
+# nothing. 5e-5 as above.
+@pytest.mark.parametrize("hd", [30, 10])
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("span", [4, 7, 20, 50])
+@pytest.mark.parametrize("where", ["rows", "token", "all"])
+def test_window_attention_tokens_apart(pkg, hd, shift, span, where):
+    heads, c, hp, wp = 6, 6 * hd, 24, 40
+    rng = np.random.default_rng(hd + shift + span)
+    x = rng.standard_normal((hp, wp, c))
+    if where == "rows":
+        x[20:] *= 2.0 ** span
+    elif where == "token":
+        x[3::8, 5::8] *= 2.0 ** span
+    else:
+        x *= 2.0 ** rng.integers(-span, 1, (hp, wp, 1))
+    x = x.reshape(hp * wp, c).astype(np.float32)
+    w = (rng.standard_normal((3 * c, c)) * 0.05).astype(np.float32)
+    b = np.zeros(3 * c, np.float32)
+    ls = np.linspace(0.0, 5.5, heads).astype(np.float32)
+    cpb = (16 / (1 + np.exp(-rng.standard_normal((4096, heads))))).astype(np.float32)
+    got = pkg.abi.test_block_attention(hp, wp, heads, hd, shift, x, w, b, ls, cpb)
+    want = attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift)
+    size = attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift, norms=True)
+    err = (np.abs(got - want) / size).max()
+    assert err < 5e-5, err
 
 
 # the tile is 8 pixels by 2 to 16 rows: planes smaller than one, of one column of
