@@ -141,13 +141,15 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 // through GEMM and task boundaries (every task walks the same stream). The row
 // scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(2 C)
 // max|ln_w| + max|ln_b|, the hidden layer's from bound(x1) max_j sum_k |W1[j][k]|
-// + max|b1| (|GELU(v)| <= |v|). A bound that a value passes by more than a factor
-// of two would be an infinite hi, so the LayerNorms sum squares of differences:
-// each wave takes its columns' mean, the squares about it, and the four (mean,
-// sum) pairs are combined. Every normalised value is then at most sqrt(C) in exact
-// arithmetic and sqrt(2 C) with any rounding of the means (the squares left out
-// are twice a product whose two squares are in). E[v^2] - mean^2 has no such
-// bound: emulated, rows of 180 with mean 2,000 times their deviation reach 870.
+// + max(b1, 0.17) (GELU(v) lies in [-0.17, max(v, 0)]). The hidden layer's is
+// shared by its units: a stage of one block is 3.0e-7 of its rms from 64 bits (fp32
+// GEMMs 6.9e-7), with one fc1 row 2^12 times the others 4.7e-7, 2^16 2.9e-6. A
+// bound that a value passes by more than a factor of two would be an infinite hi,
+// so the LayerNorms sum squares of differences: each wave takes its columns' mean
+// and the squares about it, and the four pairs are combined. A normalised value is
+// then at most sqrt(C), and sqrt(2 C) with any rounding of the means (the squares
+// left out are twice a product whose two squares are in). E[v^2] - mean^2 has no
+// such bound: emulated, rows of 180 with mean 2,000 times their deviation reach 870.
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
@@ -577,10 +579,10 @@ template <int HD> struct QaCfg {
 // Tokens of a window share v's scale while their bounds lie within 2^VSPAN of each
 // other, as they do in real images. Further apart each has its own, and the
 // probabilities take what it lies below the largest, since a query that sees only
-// small tokens is owed their precision: with a shared scale its error is 2.1e-6 of
-// sum P |v| at 2^10 (as at 1), 2.1e-5 at 2^20 and 0.6 at 2^40, with their own at
-// most 5e-6. At 264 x 264 windows that all spread take 86 us against 84 (heads of
-// 30) and 56 against 54 (of 10).
+// small tokens is owed their precision: an output is then at most 1.8e-5 of sum P |v|
+// off at any distance (in fp32 2.7e-5). With a shared scale it was that at 2^10
+// too, 2.6e-5 at 2^20 and 0.8 at 2^40. At 264 x 264 windows that all spread take 86
+// us against 84 (heads of 30) and 56 against 54 (of 10).
 constexpr int VSPAN = 6;
 
 }  // namespace
@@ -1266,7 +1268,7 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
         prm[6 * CP + c] = 1.f / s2[c];
         prm[7 * CP + c] = h.b2[c];
     }
-    float l1 = 0.f, bmax = 0.f, nw = 0.f, nb = 0.f;
+    float l1 = 0.f, bmax = 0.17f, nw = 0.f, nb = 0.f;
     for (int o = 0; o < ratio * C; ++o) {
         const float *row = h.w1 + (size_t)o * C;
         s1[o] = split_row_scale(row, C);
@@ -1276,7 +1278,7 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
         double a = 0.0;
         for (int k = 0; k < C; ++k) a += std::fabs((double)row[k]);
         l1 = std::max(l1, (float)a);
-        bmax = std::max(bmax, std::fabs(h.b1[o]));
+        bmax = std::max(bmax, h.b1[o]);
     }
     for (int c = 0; c < C; ++c) {
         nw = std::max(nw, std::fabs(h.n1w[c]));

@@ -87,6 +87,34 @@ def test_token_half_row_offset(pkg, monkeypatch, c, where, offset):
         assert err < bar, (err, bar)
 
 
+# One unit of the hidden layer with an fc1 row 2^12 times the others', or shut by a
+# bias far below 0, and no part in fc2: with the scale that the units share, the rest
+# is no further from 64 bits than the fp32 GEMMs were (6.9e-7 and 3.1e-7; the seed
+# and the sums' order move it by a tenth).
+@pytest.mark.parametrize("c", [180, 60])
+@pytest.mark.parametrize("row,bias", [(1.0, 0.0), (2.0 ** 12, 0.0), (1.0, -2.0 ** 20)])
+def test_token_half_hidden_outlier(pkg, c, row, bias):
+    M = pkg.model
+    hp, wp, p = 16, 24, "layers.0.residual_group.blocks.0.mlp."
+    arch = M.Arch(upsampler="pixelshuffle", scale=2, embed=c, heads=6, mlp_ratio=2, depths=[1])
+    wts = M.make_weights(arch, seed=5, perturb=True)
+    for k in ("fc1.weight", "fc1.bias", "fc2.weight"):
+        wts[p + k] = wts[p + k].copy()
+    wts[p + "fc1.weight"][7] *= np.float32(row)
+    wts[p + "fc1.bias"][7] += np.float32(bias)
+    wts[p + "fc2.weight"][:, 7] = 0
+    x = np.random.default_rng(c).standard_normal((c, hp, wp)).astype(np.float32)
+    want = R.rstb(x.astype(np.float64), wts, 0, 1, 8, 6)
+    be = pkg.HipBackend(arch, wts)
+    try:
+        got = be.test_rstb(0, hp, wp, np.ascontiguousarray(x.transpose(1, 2, 0).reshape(hp * wp, c)))
+    finally:
+        be.close()
+    d = got.reshape(hp, wp, c).transpose(2, 0, 1) - want
+    rel = np.linalg.norm(d) / np.linalg.norm(want)
+    assert rel < (6.9e-7 if c == 180 else 3.1e-7), rel
+
+
 def attention_f64(x, w, b, ls, cpb, hp, wp, heads, hd, shift, norms=False):
     """qkv projection and window attention in 64 bits, on [hp*wp][c] rows; with
     norms, of the norms of each head's v in the place of its values."""
