@@ -132,7 +132,7 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 // 244).
 //
 // A workgroup's 4 waves own 16 TN output columns each (C <= 64 TN), all of
-// them the task's rows: RB row blocks of 16 tokens, RB <= RBM, sized so that
+// them the task's rows: RB row blocks of 16 tokens, at most 3, sized so that
 // the two operand tiles (P0: o, then x1; P1: one C-wide chunk of the hidden
 // layer) let two workgroups run per CU. The hidden layer is made and consumed
 // C columns at a time, fc2's accumulators kept across the chunks.
@@ -1327,17 +1327,17 @@ static int split_cus() {
     return cus;
 }
 
-// Workgroups of a task size that run at once (by registers and LDS).
-static int tok_slots(int C, int rb) { return split_cus() * (tok_tn(C) > 1 ? 2 : rb < 4 ? 4 : 3); }
+// Workgroups that run at once (by registers and LDS).
+static int tok_slots(int C) { return split_cus() * (tok_tn(C) > 1 ? 2 : 4); }
 // Row blocks per task: the count whose rounds over those slots take least, a
 // round costing its row blocks plus a constant of about one (its weight stream,
 // barriers and latencies).
 static int tok_rb(int M, int C) {
-    const int nrb = M / 16;
+    const int nrb = M / 16, slots = tok_slots(C);
     int best = 1;
     long best_cost = 0;
-    for (int rb = 1; rb <= (tok_tn(C) == 1 ? 4 : 3); ++rb) {
-        const int tasks = (nrb + rb - 1) / rb, slots = tok_slots(C, rb);
+    for (int rb = 1; rb <= 3; ++rb) {
+        const int tasks = (nrb + rb - 1) / rb;
         const long cost = (long)((tasks + slots - 1) / slots) * (rb + 1);
         if (rb == 1 || cost <= best_cost) {
             best = rb;
@@ -1349,17 +1349,14 @@ static int tok_rb(int M, int C) {
 
 unsigned token_mlp_grid(int M, int C) {
     const int rb = tok_rb(M, C), tasks = (M / 16 + rb - 1) / rb;
-    return (unsigned)std::max(1, std::min(tasks, tok_slots(C, rb)));
+    return (unsigned)std::max(1, std::min(tasks, tok_slots(C)));
 }
 
 template <int TN> static void tok_launch(const TokMlpArgs &g, int rb, dim3 grid, hipStream_t st) {
     switch (rb) {
     case 1: hipLaunchKernelGGL((k_token_mlp<TN, 1>), grid, dim3(256), 0, st, g); break;
     case 2: hipLaunchKernelGGL((k_token_mlp<TN, 2>), grid, dim3(256), 0, st, g); break;
-    case 3: hipLaunchKernelGGL((k_token_mlp<TN, 3>), grid, dim3(256), 0, st, g); break;
-    default:
-        if constexpr (TN == 1) hipLaunchKernelGGL((k_token_mlp<TN, 4>), grid, dim3(256), 0, st, g);
-        break;
+    default: hipLaunchKernelGGL((k_token_mlp<TN, 3>), grid, dim3(256), 0, st, g); break;
     }
 }
 
