@@ -366,6 +366,12 @@ int s2s_test_conv3x3_winograd(int h, int w, int c_in, int c_out, const float *x,
                               const float *bias, int epilogue, const float *res, float slope,
                               float *out);
 
+/* The tile that the forward's kernels take on an h x w plane (no kernel runs):
+ * `*token` row blocks of 16 tokens per task of a block's token half (h * w a
+ * multiple of 16, c_in <= 192), `*conv` row blocks per wave of the 3x3 conv c_in ->
+ * c_out above and `*share` workgroups to a tile of it. Each may be null. */
+int s2s_test_split_tiles(int h, int w, int c_in, int c_out, int *token, int *conv, int *share);
+
 /* The real-world head's conv_up1 / conv_up2 (reference src/gpu.rs:641-669:
  * nearest-2x upsampling, conv3x3 c -> c, LeakyReLU(slope)) as the forward
  * runs them: the four 2x2 convs of the plane itself, one per output phase,

@@ -91,6 +91,8 @@ EXPORTS = {
                                    C.c_float, FP]),
     "s2s_test_conv3x3_winograd": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, FP, FP, FP,
                                             C.c_int, FP, C.c_float, FP]),
+    "s2s_test_split_tiles": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_int),
+                                       C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "s2s_test_conv3x3_shuffle2": (C.c_int, [C.c_int, C.c_int, C.c_int, C.c_int, FP, FP, FP, FP]),
     "s2s_test_rstb": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, FP, FP]),
     "s2s_test_mfma_peak": (C.c_int, [C.c_int, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double),
@@ -490,6 +492,17 @@ def test_conv3x3_winograd(x_hwc, h, w, wgt, bias, epilogue=0, res=None, slope=0.
                                         fptr(c32(bias)), epilogue, fptr(c32(res)), slope, fptr(out)),
           "s2s_test_conv3x3_winograd")
     return out
+
+
+def split_tiles(h, w, c_in, c_out):
+    """(row blocks per token task or None, row blocks per wave of the 3x3 conv,
+    workgroups to a tile of it) that an h x w plane runs with."""
+    lib = load_library()
+    v = [C.c_int(), C.c_int(), C.c_int()]
+    tok = C.byref(v[0]) if h * w % 16 == 0 else None
+    check(lib.s2s_test_split_tiles(h, w, c_in, c_out, tok, C.byref(v[1]), C.byref(v[2])),
+          "s2s_test_split_tiles")
+    return (v[0].value if tok else None, v[1].value, v[2].value)
 
 
 def test_conv3x3_shuffle2(x_hwc, h, w, wgt, bias):

@@ -234,6 +234,7 @@ size_t token_mlp_param_floats(int C, int ratio);
 void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *prm, float *ln1_bound,
                     float *fc1_l1, float *fc1_bmax);
 unsigned token_mlp_grid(int M, int C);
+int token_mlp_row_blocks(int M, int C);  // the row blocks per task that it runs
 hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st);
 // The power of two that brings the row's largest magnitude into [2^14, 2^15)
 // (1 for a zero row), and 16 weight rows' (null: zeros) k step k0 .. k0 + 31
@@ -258,6 +259,7 @@ bool split_conv_takes(int cin, int cout);
 size_t split_conv_weight_floats(int cin, int cout);
 void split_conv_pack(const float *w, int cin, int cout, float *out);
 dim3 split_conv_grid(int H, int W, int cin, int cout);
+int split_conv_row_blocks(int H, int W, int cin, int cout);  // per wave
 hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st);
 
 #define GEMM_NVARIANTS 6

@@ -1332,7 +1332,7 @@ static int tok_slots(int C) { return split_cus() * (tok_tn(C) > 1 ? 2 : 4); }
 // Row blocks per task: the count whose rounds over those slots take least, a
 // round costing its row blocks plus a constant of about one (its weight stream,
 // barriers and latencies).
-static int tok_rb(int M, int C) {
+int token_mlp_row_blocks(int M, int C) {
     const int nrb = M / 16, slots = tok_slots(C);
     int best = 1;
     long best_cost = 0;
@@ -1348,7 +1348,7 @@ static int tok_rb(int M, int C) {
 }
 
 unsigned token_mlp_grid(int M, int C) {
-    const int rb = tok_rb(M, C), tasks = (M / 16 + rb - 1) / rb;
+    const int rb = token_mlp_row_blocks(M, C), tasks = (M / 16 + rb - 1) / rb;
     return (unsigned)std::max(1, std::min(tasks, tok_slots(C)));
 }
 
@@ -1363,7 +1363,7 @@ template <int TN> static void tok_launch(const TokMlpArgs &g, int rb, dim3 grid,
 hipError_t launch_token_mlp(const TokMlpArgs &g, hipStream_t st) {
     if (g.M <= 0 || g.M % 16 || !token_mlp_takes(g.C, g.chunks)) return hipErrorInvalidValue;
     const dim3 grid(token_mlp_grid(g.M, g.C));
-    const int rb = tok_rb(g.M, g.C);
+    const int rb = token_mlp_row_blocks(g.M, g.C);
     switch (tok_tn(g.C)) {
     case 1: tok_launch<1>(g, rb, grid, st); break;
     case 2: tok_launch<2>(g, rb, grid, st); break;
@@ -1487,7 +1487,7 @@ static int conv_rb_max(int cin, int cout) {
     const int a = (cin + 63) / 64;
     return cout <= 64 ? (a == 1 ? 4 : a == 2 ? 3 : 2) : (a == 2 ? 4 : 3);
 }
-static int conv_rb(int H, int W, int cin, int cout) {
+int split_conv_row_blocks(int H, int W, int cin, int cout) {
     const int wr = 4 / conv_wc(cout), slots = 2 * split_cus();
     int best = 1;
     double best_cost = 0;
@@ -1511,10 +1511,10 @@ static long conv_tiles(int H, int W, int cout, int rb) {
 // while the one-row-block tiles alone leave half the CUs without one (180 wide:
 // 4 tiles 15.2 -> 9.4 us, 96 tiles 15.9 -> 12.6; at 180 and 224 tiles no gain).
 static int conv_split(int H, int W, int cin, int cout) {
-    return conv_rb(H, W, cin, cout) == 1 && conv_tiles(H, W, cout, 1) <= split_cus() / 2 ? conv_tn(cout) : 1;
+    return split_conv_row_blocks(H, W, cin, cout) == 1 && conv_tiles(H, W, cout, 1) <= split_cus() / 2 ? conv_tn(cout) : 1;
 }
 dim3 split_conv_grid(int H, int W, int cin, int cout) {
-    const long nt = conv_tiles(H, W, cout, conv_rb(H, W, cin, cout));
+    const long nt = conv_tiles(H, W, cout, split_conv_row_blocks(H, W, cin, cout));
     return dim3(8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, split_cus() / 4)),
                 (unsigned)conv_split(H, W, cin, cout));
 }
@@ -1536,7 +1536,7 @@ static void conv_launch(const SplitConvArgs &g, int rb, dim3 grid, hipStream_t s
 
 hipError_t launch_split_conv(const SplitConvArgs &g, hipStream_t st) {
     if (g.H <= 0 || g.W <= 0 || !split_conv_takes(g.cin, g.cout)) return hipErrorInvalidValue;
-    const int rb = conv_rb(g.H, g.W, g.cin, g.cout);
+    const int rb = split_conv_row_blocks(g.H, g.W, g.cin, g.cout);
     const dim3 grid = split_conv_grid(g.H, g.W, g.cin, g.cout);
     const int a = (g.cin + 63) / 64;
     if (g.cout <= 64) {

@@ -495,6 +495,15 @@ int s2s_test_conv3x3_nearest2(int h, int w, int c, const float *x, const float *
     return 0;
 }
 
+int s2s_test_split_tiles(int h, int w, int c_in, int c_out, int *token, int *conv, int *share) {
+    if (h <= 0 || w <= 0 || !split_conv_takes(c_in, c_out) || (token && ((long)h * w % 16 || !token_mlp_takes(c_in, 1))))
+        return fail("s2s_test_split_tiles: bad shape");
+    if (token) *token = token_mlp_row_blocks(h * w, c_in);
+    if (conv) *conv = split_conv_row_blocks(h, w, c_in, c_out);
+    if (share) *share = (int)split_conv_grid(h, w, c_in, c_out).y;
+    return 0;
+}
+
 int s2s_test_mfma_peak(int iters, int reps, double *ms, double *tflops, double *ghz) {
     if (iters <= 0 || reps <= 0 || !ms || !tflops || !ghz) return fail("s2s_test_mfma_peak: bad argument");
     int dev = 0, cus = 0;

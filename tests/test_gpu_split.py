@@ -30,8 +30,8 @@ def run_stage(pkg, orc, c, heads, ratio, depth, hp, wp, scale=1.0, seed=5):
     return np.abs(got - want).max() / np.abs(want).max()
 
 
-# (C, heads, mlp ratio, plane): one to four row blocks of 16 tokens per task,
-# with row counts that leave a partial last task, a plane of one window, widths
+# (C, heads, mlp ratio, plane): a plane of one window up to more tasks than run at
+# once, row counts that leave a partial last task, widths
 # that end in a partial k step (180 = 5 x 32 + 20) and inside a 16-column tile
 # (60, 36), the largest width (192) and other hidden widths. 1e-4 of the largest
 # value is the bar of the other stage tests.
@@ -42,6 +42,18 @@ def run_stage(pkg, orc, c, heads, ratio, depth, hp, wp, scale=1.0, seed=5):
 ])
 def test_token_half_sizes(pkg, orc, c, heads, ratio, hp, wp):
     assert run_stage(pkg, orc, c, heads, ratio, 1, hp, wp) < 1e-4
+
+
+# Each build of the token half: every count of row blocks per task (`rb`) at every
+# width class, with a partial last task and with more tasks than run at once.
+@pytest.mark.parametrize("c,heads,hp,wp,rb", [
+    (60, 6, 40, 72, 1), (60, 6, 144, 152, 2), (60, 6, 200, 200, 3), (36, 3, 264, 264, 3),
+    (120, 6, 40, 72, 1), (128, 4, 96, 96, 2), (120, 6, 128, 136, 3), (192, 6, 40, 72, 1), (180, 6, 96, 96, 2),
+    (192, 6, 136, 128, 3),
+])
+def test_token_half_row_blocks(pkg, orc, c, heads, hp, wp, rb):
+    assert pkg.abi.split_tiles(hp, wp, c, c)[0] == rb
+    assert run_stage(pkg, orc, c, heads, 2, 1, hp, wp) < 1e-4
 
 
 # magnitudes that f16 cannot hold unscaled (largest 65,504, smallest 6e-8)
@@ -232,6 +244,27 @@ def test_split_conv(pkg, cin, cout, h, w, epilogue):
     assert np.abs(got - want).max() < 2e-5
 
 
+# Each build of the conv: every count of row blocks per wave (`rb`) of every shape,
+# and the tiles shared by all of a wave's column tiles (`share`).
+@pytest.mark.parametrize("cin,cout,h,w,rb,share", [
+    (60, 60, 37, 70, 1, 2), (60, 60, 67, 129, 1, 1), (60, 60, 161, 163, 2, 1), (60, 60, 199, 211, 3, 1),
+    (60, 60, 251, 259, 3, 1), (60, 60, 230, 250, 4, 1), (120, 32, 37, 70, 1, 2), (120, 32, 99, 131, 1, 1),
+    (120, 32, 150, 133, 2, 1), (120, 32, 170, 190, 3, 1), (180, 64, 37, 70, 1, 2), (180, 64, 170, 190, 1, 1),
+    (180, 64, 161, 163, 2, 1), (120, 120, 3, 50, 1, 2), (120, 120, 37, 70, 1, 1), (120, 120, 67, 129, 2, 1),
+    (120, 120, 130, 124, 3, 1), (120, 120, 161, 163, 4, 1), (180, 180, 3, 50, 1, 3), (180, 180, 37, 70, 1, 1),
+    (180, 180, 67, 129, 2, 1), (180, 180, 130, 124, 3, 1),
+])
+def test_split_conv_row_blocks(pkg, cin, cout, h, w, rb, share):
+    assert pkg.abi.split_tiles(h, w, cin, cout)[1:] == (rb, share)
+    rng = np.random.default_rng(cin + cout + h + w)
+    x = rng.standard_normal((h * w, cin), dtype=np.float32)
+    wt = (rng.uniform(-1, 1, (cout, cin, 3, 3)) * (1 / (3 * cin)) ** 0.5).astype(np.float32)
+    b = rng.standard_normal(cout, dtype=np.float32)
+    res = rng.standard_normal((h * w, cout), dtype=np.float32)
+    got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, b, 2, res, 0.0).reshape(h, w, cout)
+    assert np.abs(got - conv_f64(x, wt, b, h, w) - res.reshape(h, w, cout)).max() < 2e-5
+
+
 # A non-finite value reaches the outputs whose footprint holds it and no other.
 @pytest.mark.parametrize("cin,cout", [(180, 180), (60, 60)])
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
@@ -314,3 +347,49 @@ def test_split_conv_channels_apart(pkg, cin, cout):
     got = pkg.abi.test_conv3x3_winograd(x, h, w, wt, np.zeros(cout, np.float32), 0).reshape(h, w, cout)
     err = (np.abs(got - conv_f64(x, wt, np.zeros(cout), h, w)) / mag).max()
     assert err < 2e-5, err
+
+
+# A non-finite token costs its window (every query of it sees the token's key) and
+# nothing outside: the rest is bit for bit what it is without.
+@pytest.mark.parametrize("hd", [30, 10])
+@pytest.mark.parametrize("shift", [0, 4])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_window_attention_nonfinite(pkg, hd, shift, bad):
+    heads, c, hp, wp = 6, 6 * hd, 24, 40
+    rng = np.random.default_rng(hd)
+    x = rng.standard_normal((hp, wp, c)).astype(np.float32)
+    w = (rng.standard_normal((3 * c, c)) * 0.05).astype(np.float32)
+    b = np.zeros(3 * c, np.float32)
+    ls = np.linspace(0.0, 5.5, heads).astype(np.float32)
+    cpb = rng.uniform(0, 16, (4096, heads)).astype(np.float32)
+    run = lambda: pkg.abi.test_block_attention(hp, wp, heads, hd, shift, x.reshape(-1, c), w, b, ls,
+                                               cpb).reshape(hp, wp, c)
+    clean = run()
+    x[shift + 9, shift + 18, 7] = bad
+    got = run()
+    hit = np.zeros((hp, wp), bool)
+    hit[shift + 8:shift + 16, shift + 16:shift + 24] = True
+    assert not np.isfinite(got[hit]).any()
+    assert np.array_equal(got[~hit], clean[~hit])
+
+
+# ... and through the token half (row by row) and the stage's closing conv (one
+# pixel further).
+@pytest.mark.parametrize("c", [180, 60])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_stage_nonfinite(pkg, c, bad):
+    M = pkg.model
+    hp, wp = 40, 48
+    arch = M.Arch(upsampler="pixelshuffle", scale=2, embed=c, heads=6, mlp_ratio=2, depths=[1])
+    x = np.random.default_rng(c).standard_normal((hp, wp, c)).astype(np.float32)
+    be = pkg.HipBackend(arch, M.make_weights(arch, seed=5, perturb=True))
+    try:
+        clean = be.test_rstb(0, hp, wp, x.reshape(-1, c)).reshape(hp, wp, c)
+        x[9, 18, 7] = bad
+        got = be.test_rstb(0, hp, wp, x.reshape(-1, c)).reshape(hp, wp, c)
+    finally:
+        be.close()
+    hit = np.zeros((hp, wp), bool)
+    hit[7:17, 15:25] = True
+    assert not np.isfinite(got[hit]).any()
+    assert np.array_equal(got[~hit], clean[~hit])
