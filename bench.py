@@ -76,9 +76,6 @@ def kernel_work(arch, h, w, hp=None, wp=None):
         # proj + LayerNorm + residual, fc1 + GELU, fc2 + LayerNorm + residual as
         # one kernel (the attention output and the block input in, the block out)
         "token_mlp": ("split", 2 * P * (C * C + 2 * Hd * C), f * P * 3 * C),
-        "proj_ln_res": ("mfma", 2 * P * C * C, f * P * 3 * C),
-        "fc1_gelu": ("mfma", 2 * P * Hd * C, f * P * (C + Hd)),
-        "fc2_ln_res": ("mfma", 2 * P * C * Hd, f * P * (Hd + 2 * C)),
         # the body's 3x3 convs (the stage close with the 1x1 folded in, and
         # conv_after_body), direct: the plane and the residual in, the plane out
         "conv3x3_stage": ("split", 2 * P * C * 9 * C, f * 3 * P * C),

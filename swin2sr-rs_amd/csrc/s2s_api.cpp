@@ -58,15 +58,12 @@ std::string hip_msg(const char *what, hipError_t e) {
 int round4(int v) { return (v + 3) / 4 * 4; }
 
 struct BlockW {
-    float *wqkv = nullptr, *bqkv = nullptr, *wproj = nullptr, *bproj = nullptr;
-    float *n1w = nullptr, *n1b = nullptr, *n2w = nullptr, *n2b = nullptr;
-    float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
+    float *wqkv = nullptr, *bqkv = nullptr;
     float *ls = nullptr, *cpbt = nullptr;
     // wqkv as k_qkv_attn reads it (qkv_attn_pack) for the head shapes it takes
     float *qkv_prm = nullptr;
     float v_l1 = 0.f, v_bmax = 0.f;
-    // the token half as k_token_mlp reads it (token_mlp_pack), for the widths
-    // it takes; wproj .. b2 above are then not uploaded
+    // the token half as k_token_mlp reads it (token_mlp_pack)
     float *tok_w = nullptr, *tok_prm = nullptr;
     float ln1_bound = 0.f, fc1_l1 = 0.f, fc1_bmax = 0.f;
 };
@@ -765,7 +762,6 @@ GemmArgs sub2_gemm(const float *in, int H, int W, int F, const float *wt, const 
 int s2s_ctx::block_fwd(const BlockW &b, int hp, int wp, int shift, const float *x_in,
                        float *x_out) {
     const int P = hp * wp;
-    GemmArgs g;
     if (qkv_attn_fused(arch.heads, hd)) {
         // 6 heads of 30 or 10: the qkv projection and the window attention as
         // one kernel (a window's q, k, v never leave the CU)
@@ -787,6 +783,7 @@ int s2s_ctx::block_fwd(const BlockW &b, int hp, int wp, int shift, const float *
     } else {
         // qkv straight into the window attention's unit layout where its
         // kernel takes the head shape, else the plane layout [P][3c]
+        GemmArgs g;
         const int epi = qkv_gemm_args(x_in, b.wqkv, b.bqkv, qkv, hp, wp, shift, arch.heads, hd, &g);
         g.b_packed = bs_packs(3 * c, c, EPI_STORE);
         if (gemm("qkv", g, ALOAD_ROWS, epi)) return -1;
@@ -797,43 +794,20 @@ int s2s_ctx::block_fwd(const BlockW &b, int hp, int wp, int shift, const float *
             return -1;
     }
 
-    if (b.tok_w) {
-        TokMlpArgs t{};
-        t.o = o;
-        t.x = x_in;
-        t.out = x_out;
-        t.w = b.tok_w;
-        t.prm = b.tok_prm;
-        t.ln1_bound = b.ln1_bound;
-        t.fc1_l1 = b.fc1_l1;
-        t.fc1_bmax = b.fc1_bmax;
-        t.inv_c = 1.0f / (float)c;
-        t.M = P;
-        t.C = c;
-        t.chunks = arch.mlp_ratio;
-        return run("token_mlp", dim3(token_mlp_grid(P, c)), dim3(256),
-                   [&] { return launch_token_mlp(t, stream); });
-    }
-
-    g = rows_gemm(o, c, b.wproj, c, b.bproj, x_out, c, P, c, c);
-    g.b_packed = bs_packs(c, c, EPI_LN_RES);
-    g.res = x_in;
-    g.ldr = c;
-    g.ln_w = b.n1w;
-    g.ln_b = b.n1b;
-    if (gemm("proj_ln_res", g, ALOAD_ROWS, EPI_LN_RES)) return -1;
-
-    g = rows_gemm(x_out, c, b.w1, c, b.b1, hid, hidden, P, hidden, c);
-    g.b_packed = bs_packs(hidden, c, EPI_GELU);
-    if (gemm("fc1_gelu", g, ALOAD_ROWS, EPI_GELU)) return -1;
-
-    g = rows_gemm(hid, hidden, b.w2, hidden, b.b2, x_out, c, P, c, hidden);
-    g.b_packed = bs_packs(c, hidden, EPI_LN_RES);
-    g.res = x_out;
-    g.ldr = c;
-    g.ln_w = b.n2w;
-    g.ln_b = b.n2b;
-    return gemm("fc2_ln_res", g, ALOAD_ROWS, EPI_LN_RES);
+    TokMlpArgs t{};
+    t.o = o;
+    t.x = x_in;
+    t.out = x_out;
+    t.w = b.tok_w;
+    t.prm = b.tok_prm;
+    t.ln1_bound = b.ln1_bound;
+    t.fc1_l1 = b.fc1_l1;
+    t.fc1_bmax = b.fc1_bmax;
+    t.inv_c = 1.0f / (float)c;
+    t.M = P;
+    t.C = c;
+    t.chunks = arch.mlp_ratio;
+    return run("token_mlp", dim3(token_mlp_grid(P, c)), dim3(256), [&] { return launch_token_mlp(t, stream); });
 }
 
 // One RSTB stage (reference src/gpu.rs:481-529): blocks, conv3x3, 1x1, + x_in.
@@ -1407,7 +1381,7 @@ int octaves_of(int scale) {
 // from s2s_create's uploads; s2s_create checks its own count against it, so
 // the two cannot drift apart.
 int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes) {
-    const uint64_t C = A.embed, C4 = round4(A.embed), H2 = (uint64_t)A.mlp_ratio * A.embed;
+    const uint64_t C = A.embed, C4 = round4(A.embed);
     const uint64_t NH = A.heads, n = (uint64_t)A.window * A.window;
     uint64_t f = 0;
     f += C;                     // conv_first's bias (the body skip)
@@ -1422,14 +1396,9 @@ int weights_device_bytes(const s2s_arch &A, const TensorSet &ts, uint64_t *bytes
         const uint64_t wqkv = qkv_attn_fused(A.heads, hd)
                                   ? qkv_attn_weight_floats(hd) + qkv_attn_param_floats(hd)
                                   : weight_floats(3 * C, C, EPI_STORE) + 3 * C;
-        // the token half: k_token_mlp's stream and parameters, or proj, norm1,
-        // norm2, fc1 and fc2 one by one
-        const uint64_t tok = token_mlp_takes(A.embed, A.mlp_ratio)
-                                 ? token_mlp_weight_floats(A.embed, A.mlp_ratio) +
-                                       token_mlp_param_floats(A.embed, A.mlp_ratio)
-                                 : weight_floats(C, C, EPI_LN_RES) + C + 4 * C +
-                                       weight_floats(H2, C, EPI_GELU) + H2 +
-                                       weight_floats(C, H2, EPI_LN_RES) + C;
+        // the token half: k_token_mlp's stream and parameters
+        const uint64_t tok = token_mlp_weight_floats(A.embed, A.mlp_ratio) +
+                             token_mlp_param_floats(A.embed, A.mlp_ratio);
         const uint64_t per_block = wqkv             // fused qkv, its bias
                                    + NH             // logit scale
                                    + tok
@@ -1671,40 +1640,23 @@ int s2s_create(const s2s_arch *arch, const s2s_tensor *tensors, size_t n_tensors
             rc = rc || ts.get(p + "attn.logit_scale", {NH, 1, 1}, &lsx);
             if (rc) break;
             rc = ctx->upload(vec_of(lsx, NH), &bw.ls);
-            if (token_mlp_takes(C, A.mlp_ratio)) {
-                TokMlpWeights tw{};
-                const struct { const char *name; std::vector<int64_t> shape; const float **dst; } parts[] = {
-                    {"attn.proj.weight", {C, C}, &tw.wproj}, {"attn.proj.bias", {C}, &tw.bproj},
-                    {"norm1.weight", {C}, &tw.n1w},          {"norm1.bias", {C}, &tw.n1b},
-                    {"norm2.weight", {C}, &tw.n2w},          {"norm2.bias", {C}, &tw.n2b},
-                    {"mlp.fc1.weight", {H2, C}, &tw.w1},     {"mlp.fc1.bias", {H2}, &tw.b1},
-                    {"mlp.fc2.weight", {C, H2}, &tw.w2},     {"mlp.fc2.bias", {C}, &tw.b2}};
-                for (const auto &e : parts) {
-                    rc = rc || ts.get(p + e.name, e.shape, &x);
-                    if (!rc) *e.dst = x->data;
-                }
-                if (rc) break;
-                std::vector<float> w(token_mlp_weight_floats(C, A.mlp_ratio));
-                std::vector<float> prm(token_mlp_param_floats(C, A.mlp_ratio));
-                token_mlp_pack(tw, C, A.mlp_ratio, w.data(), prm.data(), &bw.ln1_bound, &bw.fc1_l1,
-                               &bw.fc1_bmax);
-                rc = ctx->upload(w, &bw.tok_w) || ctx->upload(prm, &bw.tok_prm);
-            } else {
-                auto up_gemm = [&](const std::string &name, int N, int K, int epi, float **dst) -> int {
-                    if (ts.get(name, {N, K}, &x)) return -1;
-                    return ctx->upload(gemm_weights(vec_of(x, ts.numel(x)), 1, N, K, epi), dst);
-                };
-                rc = rc || up_gemm(p + "attn.proj.weight", C, C, EPI_LN_RES, &bw.wproj);
-                rc = rc || up(p + "attn.proj.bias", {C}, &bw.bproj);
-                rc = rc || up(p + "norm1.weight", {C}, &bw.n1w);
-                rc = rc || up(p + "norm1.bias", {C}, &bw.n1b);
-                rc = rc || up(p + "norm2.weight", {C}, &bw.n2w);
-                rc = rc || up(p + "norm2.bias", {C}, &bw.n2b);
-                rc = rc || up_gemm(p + "mlp.fc1.weight", H2, C, EPI_GELU, &bw.w1);
-                rc = rc || up(p + "mlp.fc1.bias", {H2}, &bw.b1);
-                rc = rc || up_gemm(p + "mlp.fc2.weight", C, H2, EPI_LN_RES, &bw.w2);
-                rc = rc || up(p + "mlp.fc2.bias", {C}, &bw.b2);
+            TokMlpWeights tw{};
+            const struct { const char *name; std::vector<int64_t> shape; const float **dst; } parts[] = {
+                {"attn.proj.weight", {C, C}, &tw.wproj}, {"attn.proj.bias", {C}, &tw.bproj},
+                {"norm1.weight", {C}, &tw.n1w},          {"norm1.bias", {C}, &tw.n1b},
+                {"norm2.weight", {C}, &tw.n2w},          {"norm2.bias", {C}, &tw.n2b},
+                {"mlp.fc1.weight", {H2, C}, &tw.w1},     {"mlp.fc1.bias", {H2}, &tw.b1},
+                {"mlp.fc2.weight", {C, H2}, &tw.w2},     {"mlp.fc2.bias", {C}, &tw.b2}};
+            for (const auto &e : parts) {
+                rc = rc || ts.get(p + e.name, e.shape, &x);
+                if (!rc) *e.dst = x->data;
             }
+            if (rc) break;
+            std::vector<float> w(token_mlp_weight_floats(C, A.mlp_ratio));
+            std::vector<float> prm(token_mlp_param_floats(C, A.mlp_ratio));
+            token_mlp_pack(tw, C, A.mlp_ratio, w.data(), prm.data(), &bw.ln1_bound, &bw.fc1_l1,
+                           &bw.fc1_bmax);
+            rc = ctx->upload(w, &bw.tok_w) || ctx->upload(prm, &bw.tok_prm);
             if (rc) break;
             // The bias table, stored [head][query][key] and scaled by log2(e)
             // for the base-2 softmax. From the converter's cpb_pre when the
