@@ -211,6 +211,9 @@ inline AttnArgs window_attn_args(const float *qkv, const float *cpbt, const floa
     return a;
 }
 
+// the current device's compute units (256 without one)
+int cu_count();
+
 // The token half of a Swin block as one kernel (k_token_mlp, s2s_split.hip):
 // out = x1 + LN2(GELU(x1 W1^T + b1) W2^T + b2), x1 = x + LN1(o Wproj^T + b),
 // over [M][C] rows (M a multiple of 16, out may be x), the hidden layer

@@ -2501,19 +2501,21 @@ hipError_t launch_mfma_peak(float *out, int blocks, int iters, hipStream_t st) {
 
 // ---- k_bsgemm dispatch ----------------------------------------------------
 
-static int cu_count() {
-    static int n = 0;
-    if (!n) {
-        int dev = 0, v = 0;
-        (void)hipGetDevice(&dev);
-        if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            v <= 0) {
-            (void)hipGetLastError();
-            v = 256;
-        }
-        n = v;
+int cu_count() {
+    static thread_local int dev_of = -1, cus = 256;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return 256;
     }
-    return n;
+    if (dev != dev_of) {
+        int n = 0;
+        const bool ok = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess;
+        if (!ok) (void)hipGetLastError();
+        cus = ok && n > 0 ? n : 256;
+        dev_of = dev;
+    }
+    return cus;
 }
 
 // K per wave and K halves of a weight shape k_bsgemm is built for (the embed

@@ -1315,20 +1315,8 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
                 }
 }
 
-static int split_cus() {
-    static thread_local int dev_of = -1, cus = 0;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 256;
-    if (dev != dev_of) {
-        int n = 0;
-        cus = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256;
-        dev_of = dev;
-    }
-    return cus;
-}
-
 // Workgroups that run at once (by registers and LDS).
-static int tok_slots(int C) { return split_cus() * (tok_tn(C) > 1 ? 2 : 4); }
+static int tok_slots(int C) { return cu_count() * (tok_tn(C) > 1 ? 2 : 4); }
 // Row blocks per task: the count whose rounds over those slots take least, a
 // round costing its row blocks plus a constant of about one (its weight stream,
 // barriers and latencies).
@@ -1424,7 +1412,7 @@ void qkv_attn_pack(const float *wqkv, const float *bqkv, int hd, float *w, float
 unsigned qkv_attention_grid(int hp, int wp, int hd) {
     const int nw = (hp / 8) * (wp / 8), ng = hd == 30 ? 3 : 1;
     const int per_xcd = ((nw + 7) / 8) * ng;
-    const int slots = std::max(1, split_cus() * 2 / 8);
+    const int slots = std::max(1, cu_count() * 2 / 8);
     return 8u * (unsigned)std::min(per_xcd, slots);
 }
 
@@ -1488,7 +1476,7 @@ static int conv_rb_max(int cin, int cout) {
     return cout <= 64 ? (a == 1 ? 4 : a == 2 ? 3 : 2) : (a == 2 ? 4 : 3);
 }
 int split_conv_row_blocks(int H, int W, int cin, int cout) {
-    const int wr = 4 / conv_wc(cout), slots = 2 * split_cus();
+    const int wr = 4 / conv_wc(cout), slots = 2 * cu_count();
     int best = 1;
     double best_cost = 0;
     for (int rb = 1; rb <= conv_rb_max(cin, cout); ++rb) {
@@ -1511,11 +1499,11 @@ static long conv_tiles(int H, int W, int cout, int rb) {
 // while the one-row-block tiles alone leave half the CUs without one (180 wide:
 // 4 tiles 15.2 -> 9.4 us, 96 tiles 15.9 -> 12.6; at 180 and 224 tiles no gain).
 static int conv_split(int H, int W, int cin, int cout) {
-    return split_conv_row_blocks(H, W, cin, cout) == 1 && conv_tiles(H, W, cout, 1) <= split_cus() / 2 ? conv_tn(cout) : 1;
+    return split_conv_row_blocks(H, W, cin, cout) == 1 && conv_tiles(H, W, cout, 1) <= cu_count() / 2 ? conv_tn(cout) : 1;
 }
 dim3 split_conv_grid(int H, int W, int cin, int cout) {
     const long nt = conv_tiles(H, W, cout, split_conv_row_blocks(H, W, cin, cout));
-    return dim3(8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, split_cus() / 4)),
+    return dim3(8u * (unsigned)std::min<long>((nt + 7) / 8, std::max(1, cu_count() / 4)),
                 (unsigned)conv_split(H, W, cin, cout));
 }
 
