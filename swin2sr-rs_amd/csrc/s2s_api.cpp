@@ -240,24 +240,24 @@ struct s2s_ctx {
     int upload(const std::vector<float> &host, float **dev);
     int alloc(AllocList &list, size_t floats, float **dev, const char *what, bool wide = false,
               bool planned = false);
-    // qkv buffer floats: the plane layout or the attention unit layout, and at
-    // least 36 planes of 4x4-pixel tiles x C (the plan's size is part of what
-    // callers budget with); in the x4 head the Winograd 5x5 conv's V and M
-    // (stride F), at most the whole plane's tiles
+    // qkv buffer floats: the plane layout or the attention unit layout (read and
+    // written for the head shapes k_qkv_attn does not take), and at least 36
+    // planes of 4x4-pixel tiles x C (see body_specs); in the x4 head the
+    // Winograd 5x5 conv's V and M (stride F), at most the whole plane's tiles
     size_t qkv_floats(int hp, int wp) const {
         const size_t plane = (size_t)hp * wp * 3 * c;
         const size_t q = qkv_unit_layout(arch.heads, hd, c)
                              ? std::max(plane, attn_unit_floats(hp, wp, arch.heads, hd))
                              : plane;
-        const size_t qb = wino_body(c) ? std::max(q, WINO_POS * wino_tiles(hp, wp) * c) : q;
+        const size_t qb = released_body(c) ? std::max(q, WINO_POS * plan_tiles(hp, wp) * c) : q;
         return up2_wino ? std::max(qb, WINO_POS * wino5_tiles(hp, wp) * feat) : qb;
     }
     // MLP hidden buffer floats (at least 36 planes of tiles x F with a
-    // conv_before_upsample head, as above)
+    // conv_before_upsample head; see body_specs)
     size_t hid_floats(int hp, int wp) const {
         const size_t h = (size_t)hp * wp * hidden;
-        const bool head = arch.upsampler != S2S_PIXELSHUFFLE_DIRECT && wino_head(c, feat);
-        return head ? std::max(h, WINO_POS * wino_tiles(hp, wp) * feat) : h;
+        const bool head = arch.upsampler != S2S_PIXELSHUFFLE_DIRECT && released_head(c, feat);
+        return head ? std::max(h, WINO_POS * plan_tiles(hp, wp) * feat) : h;
     }
     // The buffers of a padded plane's body, and of an image's head (with the
     // host path's device copies of the input and output when `io`); `bind`
@@ -518,9 +518,12 @@ int s2s_ctx::alloc(AllocList &list, size_t floats, float **dev, const char *what
 }
 
 // Body buffers for a padded plane: the activation, the in-stage working copy,
-// conv_first's output (the body skip), qkv (also the Winograd convs'
-// transform-domain products), the attention output (also the final norm's
-// output) and the MLP hidden layer.
+// conv_first's output (the body skip), qkv (also the x4 head's 5x5 products), the
+// attention output (also the final norm's output) and the MLP hidden layer, which
+// no kernel reads: k_token_mlp keeps it on the CU. The list is a contract, not
+// what the kernels need. s2s_plan_bytes, a caller's allocation limit, the sizes
+// that fit the allocation-free entry's workspace and those refused past 2 GiB all
+// follow from it, and the tile sizes that callers derive from them.
 void s2s_ctx::body_specs(int hp, int wp, bool bind, std::vector<BufSpec> &v) {
     const size_t P = (size_t)hp * wp;
     auto d = [&](float **p) { return bind ? p : nullptr; };

@@ -278,9 +278,8 @@ const char *gemm_kernel_name(const GemmArgs &g, int aload, int epi);
 void gemm_geometry(const GemmArgs &g, int aload, int epi, dim3 *grid, dim3 *block);
 hipError_t launch_attention(const AttnArgs &g, hipStream_t st, unsigned *grid_out);
 constexpr int WINO_POS = 36;
-// 4x4-pixel tiles of a plane (the plan's qkv and MLP buffers hold at least 36 of
-// their planes)
-inline size_t wino_tiles(int H, int W) { return (size_t)((H + 3) / 4) * ((W + 3) / 4); }
+// 4x4-pixel tiles of a plane, which the plan's minimum sizes are counted in
+inline size_t plan_tiles(int H, int W) { return (size_t)((H + 3) / 4) * ((W + 3) / 4); }
 // Winograd F(2x2,5x5) for the x4 head's composed 5x5 conv (F = 64 -> 48, the
 // pixel_shuffle(4) finish): the same six points and B^T; the 2x2 output
 // tiles covering Ho x Wo pixels of an H x W plane, the patch origin 2t - 2.
@@ -301,8 +300,8 @@ hipError_t launch_wino5_finish(const float *m, int ldm, const float *bias, float
 unsigned wino5_finish_grid(int Ho, int Wo);
 // The released body widths, and their conv_before_upsample: what
 // s2s_test_conv3x3_winograd takes and the plan's minimum sizes are stated for.
-inline bool wino_body(int c) { return c == 60 || c == 120 || c == 180; }
-inline bool wino_head(int c, int f) { return wino_body(c) && f % 4 == 0 && f <= 64; }
+inline bool released_body(int c) { return c == 60 || c == 120 || c == 180; }
+inline bool released_head(int c, int f) { return released_body(c) && f % 4 == 0 && f <= 64; }
 unsigned attention_grid(const AttnArgs &g);
 hipError_t launch_pad_input(const float *in, float *out, int h, int w, int hp, int wp,
                             hipStream_t st);

@@ -186,7 +186,7 @@ extern "C" int s2s_selftest(const s2s_arch *arch, const s2s_tensor *tensors, siz
         const int shapes[4][3] = {{2, 4, 60}, {34, 41, 120}, {17, 70, 180}, {8, 10, arch->embed}};
         for (auto &sh : shapes) {
             const int h = sh[0], w = sh[1], c = sh[2];
-            if (!wino_body(c)) continue;
+            if (!released_body(c)) continue;
             std::vector<float> x = seq((size_t)h * w * c, 0.3f), wgt = seq((size_t)c * c * 9, 1.1f),
                                b = seq(c, 2.2f), res = seq((size_t)h * w * c, 0.9f), got((size_t)h * w * c);
             for (float &v : wgt) v /= std::sqrt(9.0f * c);
@@ -203,7 +203,7 @@ extern "C" int s2s_selftest(const s2s_arch *arch, const s2s_tensor *tensors, siz
     // conv_before_upsample as the forward runs it (C -> F, then LeakyReLU) at the
     // checkpoint's width and a head of 64 features, on a plane ending in
     // partial tiles
-    if (wino_head(arch->embed, 64)) {
+    if (released_head(arch->embed, 64)) {
         const int h = 11, w = 13, c = arch->embed, f = 64;
         std::vector<float> x = seq((size_t)h * w * c, 0.4f), wgt = seq((size_t)f * c * 9, 1.3f),
                            b = seq(f, 2.5f), got((size_t)h * w * f);

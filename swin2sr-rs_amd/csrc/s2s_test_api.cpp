@@ -402,8 +402,8 @@ int s2s_test_conv3x3_winograd(int h, int w, int c_in, int c_out, const float *x,
     if (epilogue != 0 && epilogue != 2 && epilogue != 5) return fail("epilogue must be 0, 2 or 5");
     if (epilogue == 2 && !res) return fail("residual epilogue needs res");
     if (h <= 0 || w <= 0) return fail("the conv needs a non-empty plane");
-    const bool body = c_out == c_in && wino_body(c_in);
-    if (!body && !wino_head(c_in, c_out))
+    const bool body = c_out == c_in && released_body(c_in);
+    if (!body && !released_head(c_in, c_out))
         return fail("the conv is the body's C -> C conv, C in {60, 120, 180}, or "
                     "conv_before_upsample's C -> F, F <= 64 and a multiple of 4");
     const size_t P = (size_t)h * w;

@@ -91,8 +91,9 @@ def _fused_octaves(arch: M.Arch) -> int:
     return 2 if arch.octaves >= 2 and arch.feat == 64 else 1
 
 
-def _wino_before_upsample(arch: M.Arch) -> bool:
-    """The MLP buffer is planned for at least 36 planes of tiles x feat."""
+def _released_head(arch: M.Arch) -> bool:
+    """A released width with a conv_before_upsample head: the MLP buffer is
+    planned for at least 36 planes of 4x4-pixel tiles x feat."""
     return (arch.upsampler in ("pixelshuffle", "pixelshuffle_aux", "nearest+conv")
             and arch.embed in (60, 120, 180) and arch.feat % 4 == 0 and arch.feat <= 64)
 
@@ -118,7 +119,7 @@ def _plan_terms(arch: M.Arch, h: int, w: int):
         # the x4 head's Winograd 5x5 conv: 36 planes of 2x2-pixel tiles x F
         qkv = max(qkv, 36 * ((hp + 1) // 2) * ((wp + 1) // 2) * f)
     hid = P * arch.mlp_ratio * c
-    if _wino_before_upsample(arch):
+    if _released_head(arch):
         # at least 36 planes of F per tile
         hid = max(hid, 36 * ((hp + 3) // 4) * ((wp + 3) // 4) * f)
     terms = [P * c] * 3 + [qkv, P * c, hid]
@@ -154,7 +155,7 @@ def per_pixel_floats(arch: M.Arch) -> int:
         t = (arch.window + 1) // 2
         qkv = max(qkv, -(-36 * t * t * f // (arch.window * arch.window)))
     hid = arch.mlp_ratio * c
-    if _wino_before_upsample(arch):
+    if _released_head(arch):
         t = (arch.window + 3) // 4
         hid = max(hid, -(-36 * t * t * f // (arch.window * arch.window)))
     body = 3 * c + qkv + c + hid

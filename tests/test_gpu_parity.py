@@ -254,11 +254,11 @@ def test_block_attention_fused(pkg, orc, shift, hp, wp):
                                    (72, 72, 60)])
 @pytest.mark.parametrize("epi", [0, 2, 5])
 def test_conv3x3_winograd(pkg, orc, h, w, c, epi):
-    """The body's C -> C convs (the stage close, conv_after_body) run as
-    Winograd F(4x4,3x3) at the released widths: against the oracle's direct
-    conv, at the same bar as the direct kernel, up to the headline plane
-    (264 x 264 x 180, the borders' zero padding included); a 2x2 plane is
-    all border, and 5x7 and 33x39 end in partial 4x4 tiles."""
+    """The body's C -> C convs (the stage close, conv_after_body) as the forward
+    runs them at the released widths: against the oracle's direct conv, at the
+    same bar as the fp32 kernel, up to the headline plane (264 x 264 x 180, the
+    borders' zero padding included); a 2x2 plane is all border, and 5x7 and
+    33x39 end in partial tiles."""
     cin = cout = c
     r = rng(h * w + cin + cout + epi + 7)
     x = r.standard_normal((cin, h, w), dtype=np.float32)
@@ -282,10 +282,8 @@ def test_conv3x3_winograd(pkg, orc, h, w, c, epi):
                                          (72, 80, 120, 32), (264, 264, 180, 64), (40, 48, 180, 4)])
 @pytest.mark.parametrize("epi", [0, 5])
 def test_conv3x3_winograd_narrow(pkg, orc, h, w, cin, cout, epi):
-    """conv_before_upsample's C -> F conv (F <= 64) as the head runs it:
-    Winograd F(4x4,3x3) with the transform-domain GEMM on the weight-stationary
-    kernel's narrow (64-column) build and its products in a buffer of their
-    own, then LeakyReLU(0.01); against the oracle's direct conv."""
+    """conv_before_upsample's C -> F conv (F <= 64) as the head runs it, then
+    LeakyReLU(0.01); against the oracle's direct conv."""
     r = rng(h * w + cin * cout + epi)
     x = r.standard_normal((cin, h, w), dtype=np.float32)
     wt = (r.standard_normal((cout, cin, 3, 3), dtype=np.float32) / np.sqrt(9 * cin)).astype(np.float32)

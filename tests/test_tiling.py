@@ -65,8 +65,8 @@ def test_per_pixel_floats_stays_within_the_crates_device_model(pkg):
 def test_plan_floats_counts_the_unit_layout_and_the_composed_octaves(pkg):
     """The terms the old figure missed: the qkv buffer's real size (the
     attention's unit layout, (heads+1)/2 x (6 hd + 2) floats a pixel = 546 at
-    hd = 30; the body's Winograd convs' 36 transform planes of 4x4-pixel
-    tiles, 9 C / 4 = 405 floats a pixel; the x4 head's Winograd 5x5 conv's 36
+    hd = 30; at least 36 planes of 4x4-pixel tiles of C, 9 C / 4 = 405 floats
+    a pixel; the x4 head's Winograd 5x5 conv's 36
     planes of 2x2-pixel tiles of F = 64, 576 a pixel: whichever is largest)
     and the head planes the composed octaves never allocate."""
     M, T = pkg.model, pkg.tiling
