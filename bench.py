@@ -655,7 +655,8 @@ def bench_mfma_peak(args, pkg):
     nothing else), `steps` launches timed with events, at two loop lengths
     (the longer one's rate is the ceiling; the pair shows the launch is
     amortised). The implied shader clock is the rate over 64 FLOPs per cycle
-    per SIMD. One JSON line."""
+    per SIMD. Then the same of the f16 MFMA that the split contractions run on, on
+    zeros and on random operands. One JSON line."""
     res = {}
     for iters in (5000, 40000):
         ms, tf, ghz = pkg.abi.mfma_peak(iters, max(args.steps, 1))
@@ -664,12 +665,21 @@ def bench_mfma_peak(args, pkg):
                            "implied_clock_GHz": round(ghz, 3)}
         log(f"bench: mfma peak probe, {4 * iters} MFMAs per wave: {ms:.3f} ms, {tf:.2f} TFLOP/s "
             f"({100 * tf * 1e12 / MFMA_FP32_PEAK:.1f}% of 157.3), implied clock {ghz:.3f} GHz")
+    f16 = {}
+    for zeros in (True, False):
+        for iters in (20000, 160000):
+            ms, tf = pkg.abi.mfma_peak_f16(iters, max(args.steps, 1), zeros)
+            key = f"{'zeros' if zeros else 'random'} {iters}"
+            f16[key] = {"ms_per_launch": round(ms, 4), "TFLOPs": round(tf, 1),
+                        "frac_of_spec": round(tf * 1e12 / MFMA_F16_PEAK, 4)}
+            log(f"bench: f16 mfma peak probe, {key} rounds of 4: {ms:.3f} ms, {tf:.1f} TFLOP/s "
+                f"({100 * tf * 1e12 / MFMA_F16_PEAK:.1f}% of 2516.6)")
     print(json.dumps({"metric": "fp32 MFMA TFLOP/s under pure MFMA load @1 GPU", "unit": "TFLOP/s",
                       "n_gpus": 1, "steps": args.steps, "higher_is_better": True, "dtype": "f32",
                       "data": "register operands",
                       "config": {"workload": "k_mfma_peak: one 512-thread workgroup per CU, 4 independent "
                                              "v_mfma_f32_16x16x4f32 per loop iteration per wave"},
-                      "loops": res}), flush=True)
+                      "loops": res, "f16_loops": f16}), flush=True)
 
 
 WORKLOADS = ["classical-x4", "rstb", "lightweight-x2", "classical-x2", "realworld-x4",

@@ -404,6 +404,10 @@ int s2s_test_rstb(s2s_ctx *ctx, int stage, int hp, int wp, const float *x, float
  * that rate implies at 64 fp32 matrix FLOPs per cycle per SIMD. */
 int s2s_test_mfma_peak(int iters, int reps, double *ms, double *tflops, double *ghz);
 
+/* The same of v_mfma_f32_16x16x32_f16 (16,384 FLOPs), which the split
+ * contractions run on, with zeros or random operands. */
+int s2s_test_mfma_peak_f16(int iters, int reps, int zeros, double *ms, double *tflops);
+
 #if defined(__GNUC__) || defined(__clang__)
 #pragma GCC visibility pop
 #endif

@@ -97,6 +97,8 @@ EXPORTS = {
     "s2s_test_rstb": (C.c_int, [C.c_void_p, C.c_int, C.c_int, C.c_int, FP, FP]),
     "s2s_test_mfma_peak": (C.c_int, [C.c_int, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_double),
                                      C.POINTER(C.c_double)]),
+    "s2s_test_mfma_peak_f16": (C.c_int, [C.c_int, C.c_int, C.c_int, C.POINTER(C.c_double),
+                                         C.POINTER(C.c_double)]),
     "s2s_test_conv3x3_nearest2": (C.c_int, [C.c_int, C.c_int, C.c_int, FP, FP, FP, C.c_float, FP]),
 }
 
@@ -361,6 +363,14 @@ def mfma_peak(iters: int = 20000, reps: int = 5) -> Tuple[float, float, float]:
     check(load_library().s2s_test_mfma_peak(iters, reps, C.byref(ms), C.byref(tf), C.byref(ghz)),
           "s2s_test_mfma_peak")
     return ms.value, tf.value, ghz.value
+
+
+def mfma_peak_f16(iters: int = 20000, reps: int = 5, zeros: bool = False) -> Tuple[float, float]:
+    """(ms per launch, TFLOP/s) of the f16 matrix peak probe."""
+    ms, tf = C.c_double(), C.c_double()
+    check(load_library().s2s_test_mfma_peak_f16(iters, reps, 1 if zeros else 0, C.byref(ms), C.byref(tf)),
+          "s2s_test_mfma_peak_f16")
+    return ms.value, tf.value
 
 
 def test_qkv_windows(hp, wp, heads, head_dim, shift, x, wqkv, bqkv):

@@ -364,6 +364,7 @@ hipError_t launch_window_map(int hp, int wp, int shift, int32_t *yx, uint8_t *re
 // issuing 4 * iters independent v_mfma_f32_16x16x4f32; one float per thread
 // to `out` (blocks * 512 floats).
 hipError_t launch_mfma_peak(float *out, int blocks, int iters, hipStream_t st);
+hipError_t launch_mfma_peak_f16(float *out, int blocks, int iters, int zeros, hipStream_t st);
 
 // The ABI's thread-local error slot (defined in s2s_api.cpp): records `msg`
 // for s2s_last_error() and returns -1. Internal to the library.

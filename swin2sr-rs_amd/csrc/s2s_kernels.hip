@@ -2493,6 +2493,33 @@ __global__ __launch_bounds__(512) void k_mfma_peak(float *out, int iters, float 
     out[(size_t)blockIdx.x * 512 + threadIdx.x] = a0[0] + a1[1] + a2[2] + a3[3];
 }
 
+// The same of v_mfma_f32_16x16x32_f16, 16,384 FLOPs each, on operands drawn from
+// [-1, 1) or zeros: what toggles in the multipliers sets the clock.
+__global__ __launch_bounds__(512) void k_mfma_peak_f16(float *out, int iters, int zeros) {
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    unsigned s = blockIdx.x * 512 + threadIdx.x;
+    h8 p[4];
+    for (int k = 0; k < 4; ++k)
+        for (int i = 0; i < 8; ++i) {
+            s = s * 1664525u + 1013904223u;
+            p[k][i] = (_Float16)(zeros ? 0.f : (float)(int)s * 0x1p-31f);
+        }
+    f4v a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0, a2 = a0, a3 = a0;
+    for (int i = 0; i < iters; ++i) {
+        a0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[0], p[1], a0, 0, 0, 0);
+        a1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[2], p[3], a1, 0, 0, 0);
+        a2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[0], p[3], a2, 0, 0, 0);
+        a3 = __builtin_amdgcn_mfma_f32_16x16x32_f16(p[2], p[1], a3, 0, 0, 0);
+    }
+    out[(size_t)blockIdx.x * 512 + threadIdx.x] = a0[0] + a1[1] + a2[2] + a3[3];
+}
+
+hipError_t launch_mfma_peak_f16(float *out, int blocks, int iters, int zeros, hipStream_t st) {
+    if (blocks <= 0 || iters <= 0) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_mfma_peak_f16, dim3((unsigned)blocks), dim3(512), 0, st, out, iters, zeros);
+    return hipGetLastError();
+}
+
 hipError_t launch_mfma_peak(float *out, int blocks, int iters, hipStream_t st) {
     if (blocks <= 0 || iters <= 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_mfma_peak, dim3((unsigned)blocks), dim3(512), 0, st, out, iters, 1.0f);

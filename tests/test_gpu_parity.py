@@ -610,3 +610,10 @@ def test_mfma_peak_probe(pkg):
     ms, tf, ghz = pkg.abi.mfma_peak(2000, 3)
     assert ms > 0 and 0 < tf <= 157.3 * 1.03, (ms, tf)
     assert abs(ghz - tf * 1e12 / (256 * 4 * 64) / 1e9) < 0.05 * ghz, (tf, ghz)
+
+
+def test_mfma_peak_f16_probe(pkg):
+    """The same for the f16 probe: at most the 2,516.6 TFLOP/s spec figure."""
+    for zeros in (True, False):
+        ms, tf = pkg.abi.mfma_peak_f16(2000, 3, zeros)
+        assert ms > 0 and 0 < tf <= 2516.6 * 1.03, (ms, tf)
