@@ -4,19 +4,21 @@
 // f16(x) and lo = f16(x - hi): 22 bits of it, and a product a b as the three
 // products hi hi + hi lo + lo hi, each exact in the MFMA's fp32 accumulation
 // (the lo lo term is 2^-22 of it and below). v_mfma_f32_16x16x32_f16 takes 32 k
-// where the fp32 v_mfma_f32_16x16x4f32 takes 4 in twice the time, so three of
-// them are 4.4 times the fp32 rate (measured 2,043 / 3 against 154.7 TFLOP/s
-// under pure MFMA load). The error is no larger than the fp32 MFMA's, whose
-// accumulator rounds once per 4 k: on K = 192 dot products of unit normals,
-// rms 1.63e-7 of the result's rms against 2.47e-7, at K = 384 2.24e-7 against
-// 3.56e-7.
+// where the fp32 v_mfma_f32_16x16x4f32 takes 4 in twice the time; under pure MFMA
+// load three of them make 3.8 times the fp32 rate on random operands (1,789 / 3
+// against 155 TFLOP/s) and 4.9 times on zeros, the chip's clock making the
+// difference. The error is no larger than the fp32 MFMA's, whose accumulator
+// rounds once per 4 k: on K = 192 dot products of unit normals, rms 1.63e-7 of the
+// result's rms against 2.47e-7, at K = 384 2.24e-7 against 3.56e-7.
 //
 // The scales keep f16's exponent range out of the way. A weight row is scaled
 // at upload so that its largest element lies in [2^14, 2^15); an activation row
-// by 2^(14 - floor(log2 B)), B its largest magnitude or a bound of it. A bound
-// that is loose by 2^10 costs nothing: an element 2^-10 of the row's bound
-// still has both parts normal, and what f16 drops is 2^-39 of B. The products
-// are scaled back in fp32, exactly (powers of two), before the bias.
+// (a token's, a pixel's) by 2^(14 - floor(log2 B)), B its largest magnitude or a
+// bound of it. What f16 drops is 2^-39 of B, so an element down to 2^-14 of it
+// keeps its 22 bits, and below that a sum still keeps its largest terms'. Where
+// values that owe each other nothing would share a scale (the pixels of a conv's
+// tile, the tokens of a window) each has its own. The products are scaled back in
+// fp32, exactly (powers of two), before the bias.
 //
 // A operand tiles live in LDS in MFMA fragment order: per (row block of 16,
 // k step of 32, part) 1 KiB, lane l = 16 q + r holding row r, k = 8 q .. 8 q + 7,
@@ -153,7 +155,7 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
-// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 106 us where the
+// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 104-110 us where the
 // three GEMMs took 228 (22.6 GFLOP as three f16 products each: 41 us of MFMA at
 // the rate real data reaches, the rest VALU, which does not overlap MFMA on a
 // SIMD, operand reads and barriers); 2,880 tokens 15 us against 3 launches of
@@ -166,7 +168,10 @@ template <int TN, int RB> struct TokCfg {
     static constexpr int KS = 2 * TN;                 // k steps per GEMM
     // weight ring, k steps (a divisor of KS); with three row blocks of 180 the
     // registers go to the operand prefetch instead of a third step (126 -> 119
-    // us at 69,696 tokens), with fewer the ring is what hides L2's latency
+    // us at 69,696 tokens), with fewer the ring is what hides L2's latency. 120
+    // wide, 69,696 and 2,880 tokens: 56.4 and 10.5 us, with a ring of two steps
+    // 57.6 and 11.0, without the prefetch 57.8 and 10.6; 60 wide 24.9 and 7.0,
+    // with a ring of one step 25.5 and 7.3, without the prefetch 24.9 and 7.1
     static constexpr int WD = TN == 3 ? (RB == 3 ? 2 : 3) : (TN == 2 ? 4 : 2);
     static constexpr bool PRE = TN < 3 || RB == 3;  // operands read a k step ahead
 };
@@ -551,7 +556,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
 //
 // Items go to workgroups as window w on XCD w % 8, a window's groups one after
 // another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 80
-// us (the fp32 MFMA form with the weights in registers took 146); 2,880 tokens
+// us (77-83; the fp32 MFMA form with the weights in registers took 146); 2,880 tokens
 // 13.4 (19.9). 6 heads of 10: 5,184 tokens 13.7 us and 526,592 286, where the
 // qkv GEMM and the attention as two kernels took 20.6 and 355. With three
 // workgroups per CU (168 registers) the form of 30 spills 76 registers.
@@ -970,9 +975,9 @@ template <int HD> __global__ __launch_bounds__(64 * QaCfg<HD>::NW, 2) void k_qkv
 // 8 by q and the parity of the k step, for the writes' banks (frag_slot).
 //
 // Tiles go to workgroups in plane order within each XCD, so that halos are shared
-// in its L2. MI355X: 264 x 264 x 180 in 133 us, where F(4x4,3x3) Winograd (a
+// in its L2. MI355X: 264 x 264 x 180 in 127-137 us, where F(4x4,3x3) Winograd (a
 // quarter of the multiply-adds, in fp32, and 560 MB of transform planes) took 176;
-// 40 x 72 x 180 20.8 (31.7); 544 x 968 x 60 160 (338); 64 -> 64 at 1952 x 2592 1.26
+// 40 x 72 x 180 20.1 (31.7); 544 x 968 x 60 162 (338); 64 -> 64 at 1952 x 2592 1.29
 // ms where the fp32 implicit GEMM took 3.1. 81 us of the first are MFMA issue at
 // the clock the kernel runs at. One workgroup per CU with six row blocks per wave
 // and operands read ahead: 138 us.
