@@ -141,17 +141,19 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 //
 // Weights stream through a register ring of WD k steps, refilled as consumed,
 // through GEMM and task boundaries (every task walks the same stream). The row
-// scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(2 C)
-// max|ln_w| + max|ln_b|, the hidden layer's from bound(x1) max_j sum_k |W1[j][k]|
-// + max(b1, 0.17) (GELU(v) lies in [-0.17, max(v, 0)]). The hidden layer's is
-// shared by its units: a stage of one block is 3.0e-7 of its rms from 64 bits (fp32
-// GEMMs 6.9e-7), with one fc1 row 2^12 times the others 4.7e-7, 2^16 2.9e-6. A
-// bound that a value passes by more than a factor of two would be an infinite hi,
-// so the LayerNorms sum squares of differences: each wave takes its columns' mean
-// and the squares about it, and the four pairs are combined. A normalised value is
-// then at most sqrt(C), and sqrt(2 C) with any rounding of the means (the squares
-// left out are twice a product whose two squares are in). E[v^2] - mean^2 has no
-// such bound: emulated, rows of 180 with mean 2,000 times their deviation reach 870.
+// scales: o's from the row's maximum, x1's from the bound max|x| + sqrt(C)
+// max|ln_w| + max|ln_b| (a normalised value is at most sqrt(C)), the hidden
+// layer's from bound(x1) max_j sum_k |W1[j][k]| + max(b1, 0.17) (GELU(v) lies in
+// [-0.17, max(v, 0)]). The hidden layer's is shared by its units: a stage of one
+// block is 3.0e-7 of its rms from 64 bits (fp32 GEMMs 6.9e-7), with one fc1 row 2^12
+// times the others 4.7e-7, 2^16 2.9e-6.
+//
+// A bound that a value passes by more than a factor of two would be an infinite
+// hi, so the variance E[v^2] - mean^2 must not cancel: Wproj, W2 and their biases
+// are uploaded less their mean over the output columns (in 64 bits, rounded once),
+// which takes each row's mean off v, and a LayerNorm is the same without it. As
+// given, rows of 180 whose mean is 2,000 times their deviation normalise to 870
+// (emulated) and come out as NaN, and an fp32 GEMM loses the mean's digits of v.
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
@@ -234,7 +236,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
     constexpr int KS = K::KS, CP = K::CP;
     __shared__ __attribute__((aligned(16))) char P0[RB * KS * 2 * FRAG];
     __shared__ __attribute__((aligned(16))) char P1[RB * KS * 2 * FRAG];
-    // per row: 4 waves' means and sums of squares of LN2; LN1's, the 4 waves' max
+    // per row: 4 waves' (sum, sum of squares) of LN2; LN1's, the 4 waves' max
     // |x| and o's row unscale lie in P1, which is free until the first chunk
     __shared__ __attribute__((aligned(16))) float red2[RB * 16][8];
     __shared__ __attribute__((aligned(16))) float lnp[4 * CP];  // LN1, LN2 weights and biases
@@ -250,15 +252,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
     const __amdgpu_buffer_rsrc_t rw = buf_rsrc(g.w, (size_t)4 * steps * TN * 2 * FRAG);
     const int wbase = wave * steps * TN * 2 * FRAG;
     const __amdgpu_buffer_rsrc_t rp = buf_rsrc(g.prm, (size_t)(8 + 2 * g.chunks) * CP * 4);
-    // the waves' columns: this wave's 1 / count, and each one's share of the row
-    auto cols_of = [&](int w) __attribute__((always_inline)) { return min(max(C - 16 * TN * w, 0), 16 * TN); };
-    auto uniform = [](float v) __attribute__((always_inline)) {
-        return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
-    };
     const float inv_c = g.inv_c;
-    const float inv_n = uniform(1.0f / (float)max(cols_of(wave), 1));
-    const float share[4] = {uniform((float)cols_of(0) * inv_c), uniform((float)cols_of(1) * inv_c),
-                            uniform((float)cols_of(2) * inv_c), uniform((float)cols_of(3) * inv_c)};
 
     for (int i = tid; i < CP; i += 256)
         reinterpret_cast<float4 *>(lnp)[i] = buf_load4(rp, 16 * i);
@@ -369,53 +363,35 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
             for (int t = 0; t < TN; ++t) acc[rb][t] = f4v{0.f, 0.f, 0.f, 0.f};
         tok_gemm<TN, RB, false>(acc, P0, st, rw, wbase, lane, steps);
 
-        // v = acc scaled back + bias, less the wave's mean of the row (acc; the
-        // padding stays 0), the mean and the sum of squares to LDS; after the
-        // barrier the rows' 1/std, and what is left of the mean times it
+        // v = acc scaled back + bias, its row sums (and max |x1|'s part) to
+        // LDS; after the barrier the rows' mean and 1/std
         float mean[RB], rstd[RB];
         auto norm_stats = [&](float(*red)[8], const float (&un)[RB]) __attribute__((always_inline)) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                float s = 0.f;
+                float s1 = 0.f, s2 = 0.f;
 #pragma unroll
                 for (int t = 0; t < TN; ++t)
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const float v = fmaf(acc[rb][t][i] * cs[t][i], un[rb], b[t][i]);
                         acc[rb][t][i] = v;
-                        s += v;
+                        s1 += v;
+                        s2 = fmaf(v, v, s2);
                     }
-                mean[rb] = xrow_sum(s) * inv_n;
-            }
-#pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
-                float s = 0.f;
-#pragma unroll
-                for (int t = 0; t < TN; ++t) {
-                    const float m = off[t] != BUF_OOB ? mean[rb] : 0.f;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float d = acc[rb][t][i] - m;
-                        acc[rb][t][i] = d;
-                        s = fmaf(d, d, s);
-                    }
-                }
-                s = xrow_sum(s);
-                if (lane < 32) red[rb * 16 + j][4 * q + wave] = q ? s : mean[rb];
+                const float s = xrow_sum2(s1, s2);
+                if (lane < 32) red[rb * 16 + j][2 * wave + q] = s;
             }
         };
         auto norm_finish = [&](const float(*red)[8]) __attribute__((always_inline)) {
 #pragma unroll
             for (int rb = 0; rb < RB; ++rb) {
-                const f4v u = *reinterpret_cast<const f4v *>(&red[rb * 16 + j][0]);
-                const f4v v = *reinterpret_cast<const f4v *>(&red[rb * 16 + j][4]);
-                float m = 0.f, var = ((v[0] + v[1]) + (v[2] + v[3])) * inv_c;
-#pragma unroll
-                for (int w = 0; w < 4; ++w) m = fmaf(u[w], share[w], m);
-#pragma unroll
-                for (int w = 0; w < 4; ++w) var = fmaf((u[w] - m) * share[w], u[w] - m, var);
+                const float4 u = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][0]);
+                const float4 v = *reinterpret_cast<const float4 *>(&red[rb * 16 + j][4]);
+                const float m = ((u.x + u.z) + (v.x + v.z)) * inv_c;
+                const float var = fmaxf(((u.y + u.w) + (v.y + v.w)) * inv_c - m * m, 0.f);
                 rstd[rb] = __builtin_amdgcn_rsqf(var + 1e-5f);
-                mean[rb] = (m - mean[rb]) * rstd[rb];
+                mean[rb] = m * rstd[rb];
             }
         };
         auto load_ln = [&](int a, f4v(&lw)[TN], f4v(&lb)[TN]) __attribute__((always_inline)) {
@@ -1255,23 +1231,36 @@ size_t token_mlp_weight_floats(int C, int ratio) {
 }
 size_t token_mlp_param_floats(int C, int ratio) { return (size_t)(8 + 2 * ratio) * 64 * tok_tn(C); }
 
+// [C][K] weights less each k's mean over the C columns.
+static std::vector<float> centred(const float *w, int C, int K) {
+    std::vector<double> mean(K, 0.0);
+    for (int c = 0; c < C; ++c)
+        for (int k = 0; k < K; ++k) mean[k] += w[(size_t)c * K + k];
+    std::vector<float> out((size_t)C * K);
+    for (int c = 0; c < C; ++c)
+        for (int k = 0; k < K; ++k) out[(size_t)c * K + k] = (float)(w[(size_t)c * K + k] - mean[k] / C);
+    return out;
+}
+
 void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *prm, float *ln1_bound,
                     float *fc1_l1, float *fc1_bmax) {
     const int tn = tok_tn(C), CP = 64 * tn, ks = 2 * tn;
     uint16_t *dst = reinterpret_cast<uint16_t *>(w);
     std::fill(prm, prm + token_mlp_param_floats(C, ratio), 0.f);
     std::vector<float> sp(C), s2(C), s1((size_t)ratio * C);
+    const std::vector<float> wproj = centred(h.wproj, C, C), w2 = centred(h.w2, C, ratio * C);
+    const std::vector<float> bproj = centred(h.bproj, C, 1), b2 = centred(h.b2, C, 1);
     for (int c = 0; c < C; ++c) {
-        sp[c] = split_row_scale(h.wproj + (size_t)c * C, C);
-        s2[c] = split_row_scale(h.w2 + (size_t)c * ratio * C, ratio * C);
+        sp[c] = split_row_scale(&wproj[(size_t)c * C], C);
+        s2[c] = split_row_scale(&w2[(size_t)c * ratio * C], ratio * C);
         prm[c] = h.n1w[c];
         prm[CP + c] = h.n1b[c];
         prm[2 * CP + c] = h.n2w[c];
         prm[3 * CP + c] = h.n2b[c];
         prm[4 * CP + c] = 1.f / sp[c];
-        prm[5 * CP + c] = h.bproj[c];
+        prm[5 * CP + c] = bproj[c];
         prm[6 * CP + c] = 1.f / s2[c];
-        prm[7 * CP + c] = h.b2[c];
+        prm[7 * CP + c] = b2[c];
     }
     float l1 = 0.f, bmax = 0.17f, nw = 0.f, nb = 0.f;
     for (int o = 0; o < ratio * C; ++o) {
@@ -1289,7 +1278,7 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
         nw = std::max(nw, std::fabs(h.n1w[c]));
         nb = std::max(nb, std::fabs(h.n1b[c]));
     }
-    *ln1_bound = sqrtf(2.0f * (float)C) * nw + nb;
+    *ln1_bound = sqrtf((float)C) * nw + nb;
     *fc1_l1 = l1;
     *fc1_bmax = bmax;
     // the stream of each wave: proj, then per chunk fc1 and fc2
@@ -1306,13 +1295,13 @@ void token_mlp_pack(const TokMlpWeights &h, int C, int ratio, float *w, float *p
                         sc[r] = 0.f;
                         if (c >= C) continue;
                         if (gm == 0) {
-                            rows[r] = h.wproj + (size_t)c * C;
+                            rows[r] = &wproj[(size_t)c * C];
                             sc[r] = sp[c];
                         } else if (gm % 2 == 1) {
                             rows[r] = h.w1 + ((size_t)ch * C + c) * C;
                             sc[r] = s1[(size_t)ch * C + c];
                         } else {
-                            rows[r] = h.w2 + (size_t)c * ratio * C + (size_t)ch * C;
+                            rows[r] = &w2[(size_t)c * ratio * C + (size_t)ch * C];
                             sc[r] = s2[c];
                         }
                     }
