@@ -700,7 +700,7 @@ def main():
                          "single-RSTB micro-bench; lightweight-x2, classical-x2, realworld-x4: "
                          "configs 0, 2, 3 whole-image; compressed-x4-tiled: config 4; "
                          "copy-ceiling: the runtime's device copy at several sizes; "
-                         "mfma-peak: the fp32 matrix rate under pure MFMA load")
+                         "mfma-peak: the fp32 and f16 matrix rates under pure MFMA load")
     ap.add_argument("--lanes", type=int, default=1, choices=[0, 1],
                     help="also time two images per step through the two-lane batched entry "
                          "(reported as two_lane_serving; value stays the one-image rate); with "

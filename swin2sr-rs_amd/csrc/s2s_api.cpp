@@ -830,7 +830,8 @@ int s2s_ctx::stage_fwd(int s, int hp, int wp, const float *x_in, float *x_out) {
 }
 
 // A C -> C 3x3 conv of the body (the stage close, conv_after_body), + bias +
-// residual, on k_split_conv for the widths it takes, else as the implicit-GEMM conv with the residual as its epilogue.
+// residual, on k_split_conv for the widths it takes, else as the implicit-GEMM
+// conv with the residual as its epilogue.
 int s2s_ctx::conv_body(const char *name, const float *in, int H, int W, const float *w,
                        const float *bias, const float *res, float *out) {
     // the residual is added element by element; only a conv that reads the
@@ -1179,8 +1180,7 @@ std::vector<float> conv_relayout(const float *w, int co, int ci, const std::vect
 }
 
 // A 3x3 conv's weights [co][ci][3][3] as its kernel reads them: k_split_conv's
-// packing for the shapes it takes, else the implicit GEMM's
-// [co][tap][ci_pad4].
+// packing for the shapes it takes, else the implicit GEMM's [co][tap][ci_pad4].
 std::vector<float> conv_weights(const float *w, int co, int ci) {
     if (!split_conv_takes(ci, co)) return conv_relayout(w, co, ci, nullptr);
     std::vector<float> p(split_conv_weight_floats(ci, co));

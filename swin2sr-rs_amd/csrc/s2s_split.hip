@@ -157,7 +157,7 @@ __device__ __forceinline__ int frag_col(int T, int j, int q) {
 //
 // Every task of a launch has RB row blocks (the launcher's choice), workgroup b
 // taking tasks b, b + gridDim.x, ...; the next task's rows are loaded while this
-// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 104-110 us where the
+// one's last epilogue runs. MI355X: 69,696 tokens x 180 in 104-106 us where the
 // three GEMMs took 228 (22.6 GFLOP as three f16 products each: 41 us of MFMA at
 // the rate real data reaches, the rest VALU, which does not overlap MFMA on a
 // SIMD, operand reads and barriers); 2,880 tokens 15 us against 3 launches of
@@ -171,9 +171,9 @@ template <int TN, int RB> struct TokCfg {
     // weight ring, k steps (a divisor of KS); with three row blocks of 180 the
     // registers go to the operand prefetch instead of a third step (126 -> 119
     // us at 69,696 tokens), with fewer the ring is what hides L2's latency. 120
-    // wide, 69,696 and 2,880 tokens: 56.4 and 10.5 us, with a ring of two steps
-    // 57.6 and 11.0, without the prefetch 57.8 and 10.6; 60 wide 24.9 and 7.0,
-    // with a ring of one step 25.5 and 7.3, without the prefetch 24.9 and 7.1
+    // wide, 69,696 and 2,880 tokens: 59.3 and 7.8 us, with a ring of two steps
+    // 60.0 and 8.4, without the prefetch 61.0 and 8.0; 60 wide 23.8 and 4.2,
+    // with a ring of one step 24.6 and 4.6, without the prefetch 23.9 and 4.2
     static constexpr int WD = TN == 3 ? (RB == 3 ? 2 : 3) : (TN == 2 ? 4 : 2);
     static constexpr bool PRE = TN < 3 || RB == 3;  // operands read a k step ahead
 };
@@ -533,7 +533,7 @@ template <int TN, int RB> __global__ __launch_bounds__(256, 2) void k_token_mlp(
 // Items go to workgroups as window w on XCD w % 8, a window's groups one after
 // another, so they read its rows through one L2. MI355X, 69,696 tokens x 180: 80
 // us (77-83; the fp32 MFMA form with the weights in registers took 146); 2,880 tokens
-// 13.4 (19.9). 6 heads of 10: 5,184 tokens 13.7 us and 526,592 286, where the
+// 13.4 (19.9). 6 heads of 10: 5,184 tokens 13.7 us and 526,592 296, where the
 // qkv GEMM and the attention as two kernels took 20.6 and 355. With three
 // workgroups per CU (168 registers) the form of 30 spills 76 registers.
 // ---------------------------------------------------------------------------
